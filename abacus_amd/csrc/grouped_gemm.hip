@@ -103,25 +103,6 @@ typedef float f32x16_t __attribute__((ext_vector_type(16)));
 // complete).  Output: lane l holds column (l % kRows) and, in register q,
 // row out_row(l, q).
 template <typename T, int SHAPE> struct MfmaOp;
-template <> struct MfmaOp<uint16_t, 16> {
-  static constexpr int kRows = 16, kKB = 32, kAcc = 4;
-  using Acc = f32x4_t;
-  __device__ static inline void run(Acc& acc, const Vec16& a, const Vec16& b) {
-    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a),
-                                                  __builtin_bit_cast(bf16x8_t, b), acc, 0, 0, 0);
-  }
-  __device__ static inline int out_row(int lane, int q) { return 4 * (lane >> 4) + q; }
-};
-template <> struct MfmaOp<float, 16> {
-  static constexpr int kRows = 16, kKB = 16, kAcc = 4;
-  using Acc = f32x4_t;
-  __device__ static inline void run(Acc& acc, const Vec16& a, const Vec16& b) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(bits_f32(a.w[j]), bits_f32(b.w[j]), acc, 0, 0, 0);
-  }
-  __device__ static inline int out_row(int lane, int q) { return 4 * (lane >> 4) + q; }
-};
 template <> struct MfmaOp<uint16_t, 32> {
   static constexpr int kRows = 32, kKB = 16, kAcc = 16;
   using Acc = f32x16_t;
@@ -893,7 +874,9 @@ __device__ inline TileId tile_of_logical(int L, int MTp, int NTp) {
 // row tiles of row-grouped kinds): block b of the kind's G blocks (G a
 // multiple of 8, so b % 8 is still the XCD the block runs on when a launch
 // runs several kinds back to back).  lds: the work-group's LDS_BYTES.
-template <typename T, int KIND, int BMT = BM>
+// RK: the fixed reduction length is not a whole number of k-tiles (row-grouped
+// kinds); the last k-tile's chunks beyond it then read the zero page.
+template <typename T, int KIND, int BMT = BM, bool RK = false>
 __device__ __attribute__((always_inline)) inline void gemm_tile(const GemmArgs& g, int b, int G, char* lds,
                                                                 const RowIndex* ri) {
   using KT = KindTraits<KIND>;
@@ -992,8 +975,8 @@ __device__ __attribute__((always_inline)) inline void gemm_tile(const GemmArgs& 
     dma_k0 = (kt - half * ktiles_half) * BKT;
   };
   auto dma = [&](int n) __attribute__((always_inline)) {
-    if (n < DMA_A) sa.template issue_one<KT::WGRAD>(n, dma_stage, wave_u, dma_k0, k_len);
-    else sb.template issue_one<KT::WGRAD>(n - DMA_A, dma_stage + A_BYTES, wave_u, dma_k0, k_len);
+    if (n < DMA_A) sa.template issue_one<KT::WGRAD || RK>(n, dma_stage, wave_u, dma_k0, k_len);
+    else sb.template issue_one<KT::WGRAD || RK>(n - DMA_A, dma_stage + A_BYTES, wave_u, dma_k0, k_len);
   };
 
   // rows of this wave's part of the tile that hold data (wave-uniform)
@@ -1663,7 +1646,7 @@ __global__ __launch_bounds__(NT, 1) void gemm_tiles_kernel(GemmArgs g) {
 // (gemm_wgrad_tiles).  Blocks are dispatched in index order, so the long
 // tiles go first and the weight gradient's blocks start on the CUs that the
 // long tiles' last partial round leaves idle.
-template <typename T, int KR, int KW>
+template <typename T, int KR, int KW, bool RK>
 __global__ __launch_bounds__(NT, 1) void gemm_rows_kernel(GemmArgs g1, GemmArgs g2, GemmArgs g3, int n1, int n2) {
   static_assert(KW < 0 || sizeof(T) == 2, "weight gradients in a row launch: bf16 only");
   __shared__ __attribute__((aligned(1024))) char lds[LDS_ALLOC];
@@ -1673,8 +1656,8 @@ __global__ __launch_bounds__(NT, 1) void gemm_rows_kernel(GemmArgs g1, GemmArgs 
   const int b = blockIdx.x;
   if (b < n1 + n2) {
     const RowIndex ri = build_row_index<NT>(g1, offs_s, cum_s[0], cum_s[1]);
-    if (b < n1) gemm_tile<T, KR, BM>(g1, b, n1, lds, &ri);
-    else gemm_tile<T, KR, THIN>(g2, b - n1, n2, lds, &ri);
+    if (b < n1) gemm_tile<T, KR, BM, RK>(g1, b, n1, lds, &ri);
+    else gemm_tile<T, KR, THIN, RK>(g2, b - n1, n2, lds, &ri);
   } else {
     if constexpr (KW >= 0) {
       __shared__ int next_s;
@@ -1738,15 +1721,9 @@ __global__ __launch_bounds__(256) void split_reduce_kernel(GemmArgs g) {
 
 }  // namespace pipe
 
-// Tile configuration per (dtype, kind).
+// Tile configuration of the generic kernel per (dtype, kind): fp32 only (every
+// bf16 shape runs on the pipelined kernel).
 template <typename T, int KIND> struct Cfg;
-#ifndef ABACUS_BF16_CFG
-#define ABACUS_BF16_CFG 256, 256, 64, 2, 2, 32, 1
-#endif
-template <int KIND> struct Cfg<uint16_t, KIND> {
-  static constexpr int v[7] = {ABACUS_BF16_CFG};
-  static constexpr int BM = v[0], BN = v[1], BK = v[2], WM = v[3], WN = v[4], SHAPE = v[5], MINB = v[6];
-};
 #ifndef ABACUS_F32_CFG
 #define ABACUS_F32_CFG 128, 128, 32, 2, 2, 32, 2
 #endif
@@ -1843,8 +1820,13 @@ int launch_rows(const GemmArgs& g1, int R, const GemmArgs* gw, int64_t n1, bool 
     hipLaunchKernelGGL(pipe::ctr_zero_kernel, dim3(1), dim3(64), 0, s, gc.tile_ctr);
     ABACUS_CHECK_LAUNCH(name);
   }
-  hipLaunchKernelGGL((pipe::gemm_rows_kernel<T, KR, KW>), dim3((unsigned)(n1 + n2 + n3)), dim3(pipe::NT), 0, s, ga,
-                     gt, gc, (int)n1, (int)n2);
+  const dim3 grid((unsigned)(n1 + n2 + n3));
+  if (g1.Kdim % pipe::kBKT<T> == 0)
+    hipLaunchKernelGGL((pipe::gemm_rows_kernel<T, KR, KW, false>), grid, dim3(pipe::NT), 0, s, ga, gt, gc, (int)n1,
+                       (int)n2);
+  else
+    hipLaunchKernelGGL((pipe::gemm_rows_kernel<T, KR, KW, true>), grid, dim3(pipe::NT), 0, s, ga, gt, gc, (int)n1,
+                       (int)n2);
   ABACUS_CHECK_LAUNCH(name);
   return 0;
 }
@@ -1960,10 +1942,12 @@ int launch_pipe_pair(const GemmArgs& a, int Ra, const GemmArgs& b, int Rb, hipSt
 }
 
 // The pipelined DMA kernel whenever every dimension it tiles is a whole
-// number of 16-byte chunks and the fixed reduction length is a whole number
-// of k-tiles (always true for the workloads; the generic kernel covers the
-// rest).  The routed-row count of a row-grouped kind is free: its tiles clamp
-// their row addresses to the expert's last row.  bf16: every kind.  fp32:
+// number of 16-byte chunks.  A fixed reduction that is not a whole number of
+// k-tiles takes the kernel's ragged form (its last k-tile reads zeros past the
+// end), compiled apart because the test costs three VALU instructions per DMA;
+// the routed-row count of a row-grouped kind is free: its tiles clamp
+// their row addresses to the expert's last row.  bf16: every kind and shape.
+// fp32:
 // the gate/up forward and data gradient, the down projection's forward and
 // the weight gradients (one block per tile, when their tile groups fill
 // evenly), once there is at least one round of 256 x 256 tiles over the CUs
@@ -1974,7 +1958,7 @@ template <int KIND>
 bool pipe_ok(int dtype, const GemmArgs& g, int R) {
   using KT = KindTraits<KIND>;
   if (g.Ndim % 8 != 0 || (KT::WGRAD && g.Mdim % 8 != 0)) return false;
-  if (dtype == kBF16) return KT::WGRAD || g.Kdim % pipe::BK == 0;
+  if (dtype == kBF16) return true;
   constexpr int BNH = KT::DUAL_B ? pipe::BN / 2 : pipe::BN;
   if (dtype == kF32 && KT::WGRAD) {
     // one round of per-expert tiles, in GM x GN groups that all hold the
@@ -1985,7 +1969,7 @@ bool pipe_ok(int dtype, const GemmArgs& g, int R) {
     if (mt > pipe::GM && mt % pipe::GM != 0) return false;
     return (int64_t)g.E * mt * ((g.Ndim + BNH - 1) / BNH) >= cu_count();
   }
-  if (dtype != kF32 || KIND == kDownDgrad || g.Kdim % pipe::kBKT<float> != 0) return false;
+  if (dtype != kF32 || KIND == kDownDgrad) return false;
   return (int64_t)((R + pipe::BM - 1) / pipe::BM) * ((g.Ndim + BNH - 1) / BNH) >= cu_count();
 }
 
@@ -2014,7 +1998,6 @@ int dispatch_gemm(int dtype, const GemmArgs& g, int R, hipStream_t s, const char
     if (dtype == kBF16) return launch_pipe<uint16_t, KIND>(g, R, s, name);
     if constexpr (!KindTraits<KIND>::WGRAD && KIND != kDownDgrad) return launch_pipe<float, KIND>(g, R, s, name);
   }
-  if (dtype == kBF16) return launch_gemm<uint16_t, KIND>(g, R, s, name);
   return launch_gemm<float, KIND>(g, R, s, name);
 }
 
