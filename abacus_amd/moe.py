@@ -134,6 +134,19 @@ class _RouterFunction(torch.autograd.Function):
         return dx, dw, None, None, None, None
 
 
+def _whole_vectors(n: int, x: torch.Tensor) -> int:
+    """n rounded up to whole 16-byte vectors of x's type."""
+    vec = 16 // x.element_size()
+    return -(-n // vec) * vec
+
+
+def _decode_ws_bytes(x_TD: torch.Tensor, R: int, M: int, E: int) -> int:
+    """Workspace of abacus_experts_decode_fwd for R routed rows, -1 where it does not take the shape."""
+    if not x_TD.is_cuda:
+        return -1
+    return query("abacus_experts_decode_ws_bytes", R, x_TD.shape[1], M, E, _lib.dtype_code(x_TD.dtype))
+
+
 class _MoEFunction(torch.autograd.Function):
     """MoE.forward (moe.py:60-86) fused: router -> dispatch -> grouped SwiGLU -> combine."""
 
@@ -158,17 +171,28 @@ class _MoEFunction(torch.autograd.Function):
             float(bias_speed) if update else 0.0, dt, ptr(counts), ptr(offsets), ptr(pos), ptr(perm), ptr(xp),
             ptr(base), s,
         )
-        gate = torch.empty(R, M, dtype=x_TD.dtype, device=dev) if need_grad else None
-        up = torch.empty(R, M, dtype=x_TD.dtype, device=dev) if need_grad else None
-        h = torch.empty(R, M, dtype=x_TD.dtype, device=dev)
-        call(
-            "abacus_moe_gateup_fwd", ptr(xp), ptr(w_gate), ptr(w_up), ptr(offsets), R, D, M, E, dt,
-            ptr(gate), ptr(up), ptr(h), s,
-        )
         y = torch.empty(R, D, dtype=x_TD.dtype, device=dev)
-        ws_bytes = _lib.query("abacus_moe_down_fwd_ws_bytes", R, M, D, E, dt, device=dev)
-        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes > 0 else None
-        call("abacus_moe_down_fwd", ptr(h), ptr(w_down), ptr(offsets), R, M, D, E, dt, ptr(y), ptr(ws), ws_bytes, s)
+        decode_ws = -1 if need_grad else _decode_ws_bytes(x_TD, R, M, E)
+        if decode_ws >= 0:  # a small batch without gradients: the weight-streaming kernels
+            gate = up = None
+            ld_h = _whole_vectors(M, x_TD)
+            h = torch.empty(R, ld_h, dtype=x_TD.dtype, device=dev)
+            ws = torch.empty(decode_ws, dtype=torch.uint8, device=dev) if decode_ws > 0 else None
+            call(
+                "abacus_experts_decode_fwd", ptr(xp), ptr(w_gate), ptr(w_up), ptr(w_down), ptr(offsets), R, D, M, E, dt,
+                ld_h, ptr(h), ptr(y), ptr(ws), decode_ws, s,
+            )
+        else:
+            gate = torch.empty(R, M, dtype=x_TD.dtype, device=dev) if need_grad else None
+            up = torch.empty(R, M, dtype=x_TD.dtype, device=dev) if need_grad else None
+            h = torch.empty(R, M, dtype=x_TD.dtype, device=dev)
+            call(
+                "abacus_moe_gateup_fwd", ptr(xp), ptr(w_gate), ptr(w_up), ptr(offsets), R, D, M, E, dt,
+                ptr(gate), ptr(up), ptr(h), s,
+            )
+            ws_bytes = _lib.query("abacus_moe_down_fwd_ws_bytes", R, M, D, E, dt, device=dev)
+            ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes > 0 else None
+            call("abacus_moe_down_fwd", ptr(h), ptr(w_down), ptr(offsets), R, M, D, E, dt, ptr(y), ptr(ws), ws_bytes, s)
         out = torch.empty(T, D, dtype=x_TD.dtype, device=dev)
         call("abacus_moe_combine_fwd", ptr(y), ptr(weights), ptr(idx32), ptr(pos), T, D, K, dt, ptr(out), s)
         if need_grad:
@@ -409,9 +433,11 @@ class MoE(torch.nn.Module):
         speed = router.bias_update_speed if router.training else None
         operands = (x_TD, router.w_DE, _contig(self.w_gate_EDM), _contig(self.w_up_EDM), _contig(self.w_down_EMD))
         D, M = self.dim, self.w_gate_EDM.shape[2]
-        vec = 16 // x_TD.element_size()  # the GPU kernels move rows in 16-byte vectors
-        Dp, Mp = -(-D // vec) * vec, -(-M // vec) * vec
+        Dp, Mp = _whole_vectors(D, x_TD), _whole_vectors(M, x_TD)  # the GPU kernels move rows in 16-byte vectors
+        need_grad = torch.is_grad_enabled() and any(t.requires_grad for t in operands)
         padded = x_TD.is_cuda and (Dp != D or Mp != M)
+        if padded and not need_grad:  # (a small forward batch streams weight rows of any length)
+            padded = _decode_ws_bytes(x_TD, x_TD.shape[0] * self.top_k, M, self.n_experts) < 0
         if padded:
             # D and M zero-padded to whole vectors: zero columns of x and rows of w_DE add exact
             # zeros to the logits; a zero hidden unit has silu(0) * 0 = 0 and meets a zero row of
@@ -419,7 +445,6 @@ class MoE(torch.nn.Module):
             x_p, w_DE, w_gate, w_up, w_down = operands
             operands = (F.pad(x_p, (0, Dp - D)), F.pad(w_DE, (0, 0, 0, Dp - D)), F.pad(w_gate, (0, Mp - M, 0, Dp - D)),
                         F.pad(w_up, (0, Mp - M, 0, Dp - D)), F.pad(w_down, (0, Dp - D, 0, Mp - M)))
-        need_grad = torch.is_grad_enabled() and any(t.requires_grad for t in operands)
         out_TD = _MoEFunction.apply(
             *operands, router.expert_bias_E, self.top_k, router.route_scale, speed, need_grad, record,
         )

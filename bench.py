@@ -38,6 +38,7 @@ METRIC = "MoE-layer fwd+bwd tokens/sec on 1 MI355X; grouped-GEMM MFMA util %, di
 GEMM_FLOPS = {  # multiples of R*D*M per entry point
     "abacus_moe_gateup_fwd": 4,
     "abacus_moe_down_fwd": 2,
+    "abacus_experts_decode_fwd": 6,      # all three products (small batches)
     "abacus_moe_down_bwd_dgrad": 2,
     "abacus_moe_down_bwd_wgrad": 2,
     "abacus_moe_down_bwd": 4,            # dgrad + wgrad in one launch
@@ -101,6 +102,7 @@ def weight_stream_bytes(wl, e_touched):
     return {
         "abacus_moe_gateup_fwd": s * (2 * e_touched * D * M + R * D + R * M),
         "abacus_moe_down_fwd": s * (e_touched * M * D + R * M + R * D),
+        "abacus_experts_decode_fwd": s * (3 * e_touched * D * M + 2 * R * M + 2 * R * D),
     }
 
 

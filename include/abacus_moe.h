@@ -128,6 +128,19 @@ int abacus_moe_gateup_fwd(const void* x_perm_RD, const void* w_gate_EDM, const v
 int abacus_moe_down_fwd(const void* h_RM, const void* w_down_EMD, const int32_t* offsets_E1, int64_t R, int64_t M,
                         int64_t D, int64_t E, int dtype, void* y_RD, void* ws, int64_t ws_bytes, void* stream);
 
+/* Replaces moe.py:78-80 for a small batch without gradients (GPU only): gate,
+ * up, silu(gate) * up and the down projection by kernels that stream each
+ * touched expert's weights once.  Takes R <= 16 E (bf16) or 64 E (fp32), D a multiple of the 16-byte
+ * vector, D and M at least 16 vectors; M may be any such size (the weight rows
+ * of M elements need no alignment).  h: (R, ld_h) scratch, ld_h = M rounded up
+ * to whole vectors.  ws: abacus_experts_decode_ws_bytes bytes (-1: the shape is
+ * not taken; 0: none needed), the slices of the down projection's reduction. */
+int64_t abacus_experts_decode_ws_bytes(int64_t R, int64_t D, int64_t M, int64_t E, int dtype);
+int abacus_experts_decode_fwd(const void* x_perm_RD, const void* w_gate_EDM, const void* w_up_EDM,
+                              const void* w_down_EMD, const int32_t* offsets_E1, int64_t R, int64_t D, int64_t M,
+                              int64_t E, int dtype, int64_t ld_h, void* h, void* y_RD, void* ws, int64_t ws_bytes,
+                              void* stream);
+
 /* Replaces moe.py:81-85: out[t] = sum over the token's experts (ascending)
  * of y[pos(t,k)] * weights_TK[t,k]. */
 int abacus_moe_combine_fwd(const void* y_RD, const void* weights_TK, const int32_t* idx_TK, const int32_t* pos_TK,
