@@ -5,8 +5,13 @@
 // scores never leave the chip: each block owns 128 query rows of one (batch,
 // head) and walks the 64-key tiles up to its last query, keeping a running
 // row max and row sum (online softmax, fp32) and rescaling its fp32 output
-// accumulators as the max grows.  bf16, head_dim 64; q, k, v and o in the
-// projections' (B, L, H, K) layout, so no permuted copies are made.
+// accumulators as the max grows.  bf16, head_dim 64 or 128 and any length; q, k,
+// v and o in the projections' (B, L, H, K) layout, so no permuted copies are made.
+//
+// Lengths off the blocks: rows past the end are loaded from the last row (a
+// block's query rows, a tile's DMA rows) and never stored.  As keys they lie
+// after every real query, so the causal mask covers them; as queries of the
+// dk/dv walk they get lse2 = +inf, so their probabilities are 0.
 //
 // Layouts in registers (v_mfma_f32_32x32x16_bf16, D = A B with lane l giving
 // A[l % 32][8 (l / 32) .. +7] and B[8 (l / 32) .. +7][l % 32], and holding
@@ -25,11 +30,10 @@
 namespace abacus {
 namespace {
 
-constexpr int kHeadDim = 64;
 constexpr int kQRows = 128;   // query rows per block (4 waves x 32)
 constexpr int kKeys = 64;     // keys per tile
 constexpr int kAttnThreads = 256;
-constexpr int kTileBytes = kKeys * kHeadDim * 2;  // one K or V tile: 8 KB
+template <int HD> constexpr int kTileBytes = kKeys * HD * 2;  // one K or V tile: 8 KB (16 KB at head dim 128)
 constexpr int kStages = 2;  // LDS ring depth (2 measured faster than 3: 32 KB per block, more blocks per CU)
 static_assert(kStages == 2 || kStages == 3, "the ring's waits cover one or two tiles ahead");
 
@@ -42,34 +46,42 @@ __device__ inline void mfma32(attn_f32x16& acc, const Vec16& a, const Vec16& b) 
                                                 acc, 0, 0, 0);
 }
 
-// A K or V tile in LDS: 64 rows (keys) of 8 16-byte chunks (dims), the chunk
-// index XOR-swizzled by row: with m = row / 2, swz = (m % 2) * 4 + (m / 2) % 4.
-// Rows 2 apart land 128 bytes apart in the bank space, so a K fragment read
-// (16 consecutive rows, one chunk) needs the 8 even rows of a block of 16 on 8
-// different chunks (swz is a permutation of 0..7 over them), and a V^T read
-// (rows r..r+3, r a multiple of 4, chunks c..c+3 of 8) needs rows r and r+2
-// on complementary halves of the chunks (swz(r+2) = swz(r) ^ 4).  Both are
-// then free of bank conflicts.
-__device__ inline int tile_swz(int row) { return (((row >> 1) & 1) << 2) | ((row >> 2) & 3); }
-__device__ inline int tile_off(int row, int chunk) { return (row * 8 + (chunk ^ tile_swz(row))) * 16; }
+// A K or V tile in LDS: 64 rows (keys) of HD / 8 16-byte chunks (dims), the chunk
+// index XOR-swizzled by row.  Head dim 64: with m = row / 2, swz = (m % 2) * 4 +
+// (m / 2) % 4.  Rows 2 apart land 128 bytes apart in the bank space, so a K
+// fragment read (16 consecutive rows, one chunk) needs the 8 even rows of a block
+// of 16 on 8 different chunks (swz is a permutation of 0..7 over them), and a V^T
+// read (rows r..r+3, r a multiple of 4, chunks c..c+3 of 8) needs rows r and r+2
+// on complementary halves of the chunks (swz(r+2) = swz(r) ^ 4).  Head dim 128: a
+// row is a whole turn of the banks, so 16 consecutive rows need 16 different
+// chunks and rows r..r+3 four different groups of 4: swz = (row % 4) * 4 +
+// (row / 4) % 4.  Either way both reads are free of bank conflicts.
+template <int HD> __device__ inline int tile_swz(int row) {
+  return HD == 64 ? (((row >> 1) & 1) << 2) | ((row >> 2) & 3) : ((row & 3) << 2) | ((row >> 2) & 3);
+}
+template <int HD> __device__ inline int tile_off(int row, int chunk) {
+  return (row * (HD / 8) + (chunk ^ tile_swz<HD>(row))) * 16;
+}
 
 // K fragment (A of S^T): key `row0 + l % 32`, dims 16 c + 8 (l / 32) .. +7.
+template <int HD>
 __device__ inline Vec16 frag_k(const char* tile, int row0, int c, int lane) {
-  return *reinterpret_cast<const Vec16*>(tile + tile_off(row0 + (lane & 31), 2 * c + (lane >> 5)));
+  return *reinterpret_cast<const Vec16*>(tile + tile_off<HD>(row0 + (lane & 31), 2 * c + (lane >> 5)));
 }
 
 // V^T fragment (A of O^T): dim `d0 + l % 32`, keys 16 c + 8 (l / 32) .. +7,
 // from the row-major (key, dim) tile through the LDS transpose read (lane j of
 // each 16-lane group receives element j % 4 of the reads of lanes 4i + j / 4).
+template <int HD>
 __device__ inline Vec16 frag_vt(const char* tile, int d0, int c, int lane) {
   const int grp = lane >> 4, s = lane & 15;
   const int d = d0 + 16 * (grp & 1) + 4 * (s & 3);
   const int key = 16 * c + 8 * (grp >> 1) + (s >> 2);
   const int b = (d & 7) * 2;
   const attn_v4i16 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-      (__attribute__((address_space(3))) attn_v4i16*)(tile + tile_off(key, d >> 3) + b));
+      (__attribute__((address_space(3))) attn_v4i16*)(tile + tile_off<HD>(key, d >> 3) + b));
   const attn_v4i16 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-      (__attribute__((address_space(3))) attn_v4i16*)(tile + tile_off(key + 4, d >> 3) + b));
+      (__attribute__((address_space(3))) attn_v4i16*)(tile + tile_off<HD>(key + 4, d >> 3) + b));
   const uint2 a = __builtin_bit_cast(uint2, lo), b2 = __builtin_bit_cast(uint2, hi);
   Vec16 v;
   v.w[0] = a.x;
@@ -122,24 +134,34 @@ __device__ inline Vec16 row_chunk_operand(const attn_f32x16& s, int c2) {
   return pf;
 }
 
-// DMA of one 64-row x 128-byte tile (K, V, Q or dO rows of a (batch, head))
-// into a swizzled LDS tile: two instructions per thread; instruction i of wave
-// w writes LDS positions p = (4 i + w) * 64 + lane, which hold (row p / 8,
-// chunk (p % 8) ^ swz(row)) of the tile.
+// DMA of one 64-row tile (K, V, Q or dO rows of a (batch, head)) into a swizzled
+// LDS tile: HD / 32 instructions per thread; instruction i of wave w writes LDS
+// positions p = (4 i + w) * 64 + lane, which hold (row p / (HD / 8), chunk
+// (p % (HD / 8)) ^ swz(row)) of the tile.  `last` is the tile's last row that
+// exists; the rows after it repeat it.
+template <int HD>
 struct TileDma {
-  int64_t off[2];
+  static constexpr int N = HD / 32, CH = HD / 8;
+  uint32_t off[N];  // elements: a tile's rows span 64 * H * HD of them
   int wave_u;
-  __device__ inline void init(int64_t row_stride, int wave, int lane) {
+  __device__ static inline uint32_t offset(uint32_t row_stride, int i, int last) {
+    const int p = i * 256 + (int)threadIdx.x, row = p / CH;
+    return (uint32_t)min(row, last) * row_stride + ((p % CH) ^ tile_swz<HD>(row)) * 8;
+  }
+  __device__ inline void init(int64_t row_stride, int wave) {
     wave_u = __builtin_amdgcn_readfirstlane(wave);
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int p = (i * 4 + wave) * 64 + lane, row = p >> 3;
-      off[i] = (int64_t)row * row_stride + ((p & 7) ^ tile_swz(row)) * 8;
-    }
+    for (int i = 0; i < N; ++i) off[i] = offset((uint32_t)row_stride, i, kKeys - 1);
   }
-  __device__ inline void issue(const uint16_t* rows0, char* tile) const {
+  __device__ inline void issue(const uint16_t* rows0, char* tile, int64_t row_stride, int last) const {
+    if (last >= kKeys - 1) {
 #pragma unroll
-    for (int i = 0; i < 2; ++i) dma16(rows0 + off[i], tile + (i * 4 + wave_u) * 1024);
+      for (int i = 0; i < N; ++i) dma16(rows0 + off[i], tile + (i * 4 + wave_u) * 1024);
+    } else {
+#pragma unroll
+      for (int i = 0; i < N; ++i)
+        dma16(rows0 + offset((uint32_t)row_stride, i, last), tile + (i * 4 + wave_u) * 1024);
+    }
   }
 };
 
@@ -149,39 +171,41 @@ struct TileDma {
 // alone when nq is odd), so every work-group carries the same work; with one
 // block per work-group the launch ran 1.3x longer than its average share
 // (92.7 against 72.1 us for the forward at B4 L2048 H16).
-typedef char AttnRing[kStages][2][kTileBytes];
+template <int HD> using AttnRing = char[kStages][2][kTileBytes<HD>];
 
 // o = softmax(mask(q k^T * scale)) v for one (batch, head) and query block qb
 // (128 queries); lse2 = row max + log2(row sum) of the base-2 scaled scores.
+template <int HD>
 __device__ __attribute__((always_inline)) inline void attn_fwd_block(const uint16_t* __restrict__ q,
                                                                     const uint16_t* __restrict__ k,
                                                                     const uint16_t* __restrict__ v, int L, int H,
                                                                     float scale_log2, uint16_t* __restrict__ o,
                                                                     float* __restrict__ lse2, int qb,
-                                                                    AttnRing& lds) {  // [stage][K, V]
+                                                                    AttnRing<HD>& lds) {  // [stage][K, V]
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, h = lane >> 5;
   const int head = blockIdx.y, batch = blockIdx.z;
-  const int64_t row_stride = (int64_t)H * kHeadDim;  // elements between consecutive tokens
-  const int64_t base = ((int64_t)batch * L * H + head) * kHeadDim;
+  const int64_t row_stride = (int64_t)H * HD;  // elements between consecutive tokens
+  const int64_t base = ((int64_t)batch * L * H + head) * HD;
   const int q0 = qb * kQRows + wave * 32;  // this wave's first query
-  const int my_q = q0 + (lane & 31);
+  const int my_q = q0 + (lane & 31), ld_q = min(my_q, L - 1);
 
   // Q^T fragments (B of S^T): query my_q, dims 16 c + 8 h .. +7
-  Vec16 qf[4];
+  Vec16 qf[HD / 16];
 #pragma unroll
-  for (int c = 0; c < 4; ++c) qf[c] = ld16(q + base + (int64_t)my_q * row_stride + 16 * c + 8 * h);
+  for (int c = 0; c < HD / 16; ++c) qf[c] = ld16(q + base + (int64_t)ld_q * row_stride + 16 * c + 8 * h);
 
-  TileDma dma;
-  dma.init(row_stride, wave, lane);
+  TileDma<HD> dma;
+  dma.init(row_stride, wave);
   auto dma_tile = [&](int j, int stage) __attribute__((always_inline)) {
     const int64_t t0 = base + (int64_t)j * kKeys * row_stride;
-    dma.issue(k + t0, lds[stage][0]);
-    dma.issue(v + t0, lds[stage][1]);
+    const int last = L - 1 - j * kKeys;
+    dma.issue(k + t0, lds[stage][0], row_stride, last);
+    dma.issue(v + t0, lds[stage][1], row_stride, last);
   };
 
-  attn_f32x16 oacc[2];
+  attn_f32x16 oacc[HD / 32];
 #pragma unroll
-  for (int t = 0; t < 2; ++t)
+  for (int t = 0; t < HD / 32; ++t)
 #pragma unroll
     for (int r = 0; r < 16; ++r) oacc[t][r] = 0.f;
   float m_run = -__builtin_inff(), l_run = 0.f;
@@ -196,7 +220,7 @@ __device__ __attribute__((always_inline)) inline void attn_fwd_block(const uint1
     for (int kh = 0; kh < 2; ++kh) {
       s[kh] = zero;
 #pragma unroll
-      for (int c = 0; c < 4; ++c) mfma32(s[kh], frag_k(kt, 32 * kh, c, lane), qf[c]);
+      for (int c = 0; c < HD / 16; ++c) mfma32(s[kh], frag_k<HD>(kt, 32 * kh, c, lane), qf[c]);
     }
     // on the wave's diagonal tiles, mask keys after the query
     if constexpr (decltype(diag)::value) {
@@ -224,7 +248,7 @@ __device__ __attribute__((always_inline)) inline void attn_fwd_block(const uint1
       const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
       l_run *= alpha;
 #pragma unroll
-      for (int t = 0; t < 2; ++t)
+      for (int t = 0; t < HD / 32; ++t)
 #pragma unroll
         for (int r = 0; r < 16; ++r) oacc[t][r] *= alpha;
       m_run = m_new;
@@ -244,7 +268,7 @@ __device__ __attribute__((always_inline)) inline void attn_fwd_block(const uint1
     for (int c = 0; c < 4; ++c) {
       const Vec16 pf = row_chunk_operand(s[c >> 1], c & 1);
 #pragma unroll
-      for (int t = 0; t < 2; ++t) mfma32(oacc[t], frag_vt(vt, 32 * t, c, lane), pf);
+      for (int t = 0; t < HD / 32; ++t) mfma32(oacc[t], frag_vt<HD>(vt, 32 * t, c, lane), pf);
     }
   };
 
@@ -253,9 +277,10 @@ __device__ __attribute__((always_inline)) inline void attn_fwd_block(const uint1
   // after which no wave still reads tile j-1's stage), tile j + kStages-1 is
   // sent into that stage.
   constexpr int kAhead = kStages - 1;
-  const int ntiles = (qb * kQRows + kQRows) / kKeys;  // keys 0 .. the block's last query (>= 2)
+  const int ntiles = min(qb * kQRows + kQRows - 1, L - 1) / kKeys + 1;  // keys 0 .. the block's last query
 #pragma unroll
-  for (int t = 0; t < kAhead; ++t) dma_tile(t, t);
+  for (int t = 0; t < kAhead; ++t)
+    if (t < ntiles) dma_tile(t, t);
   for (int j = 0; j < ntiles; ++j) {
     const int buf = j % kStages;
     // tiles j+1 .. j+kAhead-1 (4 instructions each) may still be in flight
@@ -270,11 +295,12 @@ __device__ __attribute__((always_inline)) inline void attn_fwd_block(const uint1
       tile_step(lds[buf][0], lds[buf][1], key0, std::false_type{});
     }
   }
+  if (my_q >= L) return;
   // o = O / l, rounded once to bf16; lse2 for the backward
   const float inv = 1.0f / l_run;
   uint16_t* orow = o + base + (int64_t)my_q * row_stride;
 #pragma unroll
-  for (int t = 0; t < 2; ++t)
+  for (int t = 0; t < HD / 32; ++t)
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
       uint2 w;
@@ -285,17 +311,18 @@ __device__ __attribute__((always_inline)) inline void attn_fwd_block(const uint1
   if (h == 0) lse2[((int64_t)batch * H + head) * L + my_q] = m_run + __builtin_amdgcn_logf(l_run);
 }
 
-__global__ __launch_bounds__(kAttnThreads) void attn_fwd_kernel(const uint16_t* __restrict__ q,
+template <int HD>
+__global__ __launch_bounds__(kAttnThreads, HD == 64 ? 3 : 2) void attn_fwd_kernel(const uint16_t* __restrict__ q,
                                                                 const uint16_t* __restrict__ k,
                                                                 const uint16_t* __restrict__ v, int L, int H,
                                                                 float scale_log2, uint16_t* __restrict__ o,
                                                                 float* __restrict__ lse2) {
-  __shared__ __attribute__((aligned(1024))) AttnRing lds;
-  const int nq = L / kQRows, p = blockIdx.x;
-  attn_fwd_block(q, k, v, L, H, scale_log2, o, lse2, nq - 1 - p, lds);
+  __shared__ __attribute__((aligned(1024))) AttnRing<HD> lds;
+  const int nq = (L + kQRows - 1) / kQRows, p = blockIdx.x;
+  attn_fwd_block<HD>(q, k, v, L, H, scale_log2, o, lse2, nq - 1 - p, lds);
   if (p != nq - 1 - p) {
     __syncthreads();  // every wave is done with the ring
-    attn_fwd_block(q, k, v, L, H, scale_log2, o, lse2, p, lds);
+    attn_fwd_block<HD>(q, k, v, L, H, scale_log2, o, lse2, p, lds);
   }
 }
 
@@ -305,21 +332,22 @@ __global__ __launch_bounds__(kAttnThreads) void attn_fwd_kernel(const uint16_t* 
 // dk = scale dz^T q, dv = P^T dO.  P is rebuilt from the forward's lse2.
 
 // D[b, h, i] = sum over the head dim of dO * o (fp32 from the bf16 values):
-// 8 lanes per (b, l, h) row, 32 rows per block.
+// HD / 8 lanes per (b, l, h) row.
+template <int HD>
 __global__ __launch_bounds__(256) void attn_bwd_dot_kernel(const uint16_t* __restrict__ o,
                                                            const uint16_t* __restrict__ dout, int64_t rows, int L,
                                                            int H, float* __restrict__ dvec) {
-  const int64_t r = (int64_t)blockIdx.x * 32 + (threadIdx.x >> 3);
-  const int li = threadIdx.x & 7;
+  constexpr int LPR = HD / 8;
+  const int64_t r = (int64_t)blockIdx.x * (256 / LPR) + threadIdx.x / LPR;
+  const int li = threadIdx.x % LPR;
   float acc = 0.f;
   if (r < rows) {
-    const Vec16 a = ld16(o + r * kHeadDim + li * 8), b = ld16(dout + r * kHeadDim + li * 8);
+    const Vec16 a = ld16(o + r * HD + li * 8), b = ld16(dout + r * HD + li * 8);
 #pragma unroll
     for (int w = 0; w < 4; ++w) acc += lo_bf16(a.w[w]) * lo_bf16(b.w[w]) + hi_bf16(a.w[w]) * hi_bf16(b.w[w]);
   }
-  acc += __shfl_xor(acc, 1, 64);
-  acc += __shfl_xor(acc, 2, 64);
-  acc += __shfl_xor(acc, 4, 64);
+#pragma unroll
+  for (int o = 1; o < LPR; o <<= 1) acc += __shfl_xor(acc, o, 64);
   if (li == 0 && r < rows) {
     const int64_t b = r / ((int64_t)L * H), l = (r / H) % L, hh = r % H;
     dvec[(b * H + hh) * L + l] = acc;
@@ -330,35 +358,37 @@ __global__ __launch_bounds__(256) void attn_bwd_dot_kernel(const uint16_t* __res
 // block's last query: the forward's tile walk, with the scores' layout
 // (lane l: its query's scores against keys 8g + 4h + 0..3 of each half)
 // shared by S^T = K Q^T and dP^T = V dO^T, and dq^T += K^T dz^T.
+template <int HD>
 __device__ __attribute__((always_inline)) inline void attn_bwd_dq_block(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
     const uint16_t* __restrict__ dout, const float* __restrict__ lse2, const float* __restrict__ dvec, int L, int H,
-    float scale_log2, float scale, uint16_t* __restrict__ dq, int qb, AttnRing& lds) {  // [stage][K, V]
+    float scale_log2, float scale, uint16_t* __restrict__ dq, int qb, AttnRing<HD>& lds) {  // [stage][K, V]
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, h = lane >> 5;
   const int head = blockIdx.y, batch = blockIdx.z;
-  const int64_t row_stride = (int64_t)H * kHeadDim;
-  const int64_t base = ((int64_t)batch * L * H + head) * kHeadDim;
+  const int64_t row_stride = (int64_t)H * HD;
+  const int64_t base = ((int64_t)batch * L * H + head) * HD;
   const int q0 = qb * kQRows + wave * 32;
-  const int my_q = q0 + (lane & 31);
-  const int64_t stat = ((int64_t)batch * H + head) * L + my_q;
+  const int my_q = q0 + (lane & 31), ld_q = min(my_q, L - 1);
+  const int64_t stat = ((int64_t)batch * H + head) * L + ld_q;
   const float my_lse = lse2[stat], my_d = dvec[stat];
 
-  Vec16 qf[4], df[4];  // B operands: q and dO of my_q, dims 16 c + 8 h .. +7
+  Vec16 qf[HD / 16], df[HD / 16];  // B operands: q and dO of my_q, dims 16 c + 8 h .. +7
 #pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    qf[c] = ld16(q + base + (int64_t)my_q * row_stride + 16 * c + 8 * h);
-    df[c] = ld16(dout + base + (int64_t)my_q * row_stride + 16 * c + 8 * h);
+  for (int c = 0; c < HD / 16; ++c) {
+    qf[c] = ld16(q + base + (int64_t)ld_q * row_stride + 16 * c + 8 * h);
+    df[c] = ld16(dout + base + (int64_t)ld_q * row_stride + 16 * c + 8 * h);
   }
-  TileDma dma;
-  dma.init(row_stride, wave, lane);
+  TileDma<HD> dma;
+  dma.init(row_stride, wave);
   auto dma_tile = [&](int j, int stage) __attribute__((always_inline)) {
     const int64_t t0 = base + (int64_t)j * kKeys * row_stride;
-    dma.issue(k + t0, lds[stage][0]);
-    dma.issue(v + t0, lds[stage][1]);
+    const int last = L - 1 - j * kKeys;
+    dma.issue(k + t0, lds[stage][0], row_stride, last);
+    dma.issue(v + t0, lds[stage][1], row_stride, last);
   };
-  attn_f32x16 dqacc[2];
+  attn_f32x16 dqacc[HD / 32];
 #pragma unroll
-  for (int t = 0; t < 2; ++t)
+  for (int t = 0; t < HD / 32; ++t)
 #pragma unroll
     for (int r = 0; r < 16; ++r) dqacc[t][r] = 0.f;
 
@@ -370,9 +400,9 @@ __device__ __attribute__((always_inline)) inline void attn_bwd_dq_block(
       sc[kh] = zero;
       dp[kh] = zero;
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        mfma32(sc[kh], frag_k(kt, 32 * kh, c, lane), qf[c]);
-        mfma32(dp[kh], frag_k(vt, 32 * kh, c, lane), df[c]);
+      for (int c = 0; c < HD / 16; ++c) {
+        mfma32(sc[kh], frag_k<HD>(kt, 32 * kh, c, lane), qf[c]);
+        mfma32(dp[kh], frag_k<HD>(vt, 32 * kh, c, lane), df[c]);
       }
     }
     // dz = P (dP - D), P = 0 for keys after the query
@@ -390,14 +420,15 @@ __device__ __attribute__((always_inline)) inline void attn_bwd_dq_block(
     for (int c = 0; c < 4; ++c) {
       const Vec16 zf = row_chunk_operand(sc[c >> 1], c & 1);
 #pragma unroll
-      for (int t = 0; t < 2; ++t) mfma32(dqacc[t], frag_vt(kt, 32 * t, c, lane), zf);
+      for (int t = 0; t < HD / 32; ++t) mfma32(dqacc[t], frag_vt<HD>(kt, 32 * t, c, lane), zf);
     }
   };
 
   constexpr int kAhead = kStages - 1;
-  const int ntiles = (qb * kQRows + kQRows) / kKeys;
+  const int ntiles = min(qb * kQRows + kQRows - 1, L - 1) / kKeys + 1;
 #pragma unroll
-  for (int t = 0; t < kAhead; ++t) dma_tile(t, t);
+  for (int t = 0; t < kAhead; ++t)
+    if (t < ntiles) dma_tile(t, t);
   for (int j = 0; j < ntiles; ++j) {
     const int buf = j % kStages;
     if (kAhead >= 2 && j + 1 < ntiles) wait_vmcnt<(kAhead >= 2 ? 4 : 0)>();
@@ -411,9 +442,10 @@ __device__ __attribute__((always_inline)) inline void attn_bwd_dq_block(
       tile_step(lds[buf][0], lds[buf][1], key0, std::false_type{});
     }
   }
+  if (my_q >= L) return;
   uint16_t* row = dq + base + (int64_t)my_q * row_stride;
 #pragma unroll
-  for (int t = 0; t < 2; ++t)
+  for (int t = 0; t < HD / 32; ++t)
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
       uint2 w;
@@ -423,16 +455,17 @@ __device__ __attribute__((always_inline)) inline void attn_bwd_dq_block(
     }
 }
 
-__global__ __launch_bounds__(kAttnThreads) void attn_bwd_dq_kernel(
+template <int HD>
+__global__ __launch_bounds__(kAttnThreads, HD == 64 ? 2 : 1) void attn_bwd_dq_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
     const uint16_t* __restrict__ dout, const float* __restrict__ lse2, const float* __restrict__ dvec, int L, int H,
     float scale_log2, float scale, uint16_t* __restrict__ dq) {
-  __shared__ __attribute__((aligned(1024))) AttnRing lds;
-  const int nq = L / kQRows, p = blockIdx.x;
-  attn_bwd_dq_block(q, k, v, dout, lse2, dvec, L, H, scale_log2, scale, dq, nq - 1 - p, lds);
+  __shared__ __attribute__((aligned(1024))) AttnRing<HD> lds;
+  const int nq = (L + kQRows - 1) / kQRows, p = blockIdx.x;
+  attn_bwd_dq_block<HD>(q, k, v, dout, lse2, dvec, L, H, scale_log2, scale, dq, nq - 1 - p, lds);
   if (p != nq - 1 - p) {
     __syncthreads();
-    attn_bwd_dq_block(q, k, v, dout, lse2, dvec, L, H, scale_log2, scale, dq, p, lds);
+    attn_bwd_dq_block<HD>(q, k, v, dout, lse2, dvec, L, H, scale_log2, scale, dq, p, lds);
   }
 }
 
@@ -445,45 +478,47 @@ __global__ __launch_bounds__(kAttnThreads) void attn_bwd_dq_kernel(
 // lane exchange.  The query tile's lse2 and D values come through LDS.
 typedef float AttnStats[kStages][2][kKeys];
 
+template <int HD>
 __device__ __attribute__((always_inline)) inline void attn_bwd_dkdv_block(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
     const uint16_t* __restrict__ dout, const float* __restrict__ lse2, const float* __restrict__ dvec, int L, int H,
     float scale_log2, float scale, uint16_t* __restrict__ dk, uint16_t* __restrict__ dv, int kb,
-    AttnRing& lds, AttnStats& stats) {  // [stage][Q, dO], [stage][lse2, D]
+    AttnRing<HD>& lds, AttnStats& stats) {  // [stage][Q, dO], [stage][lse2, D]
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, h = lane >> 5;
   const int head = blockIdx.y, batch = blockIdx.z;
-  const int64_t row_stride = (int64_t)H * kHeadDim;
-  const int64_t base = ((int64_t)batch * L * H + head) * kHeadDim;
+  const int64_t row_stride = (int64_t)H * HD;
+  const int64_t base = ((int64_t)batch * L * H + head) * HD;
   const int64_t stat0 = ((int64_t)batch * H + head) * L;
   const int k0 = kb * kQRows + wave * 32;  // this wave's first key
-  const int my_k = k0 + (lane & 31);
+  const int my_k = k0 + (lane & 31), ld_k = min(my_k, L - 1);
 
-  Vec16 kf[4], vf[4];  // B operands: k and v of my_k, dims 16 c + 8 h .. +7
+  Vec16 kf[HD / 16], vf[HD / 16];  // B operands: k and v of my_k, dims 16 c + 8 h .. +7
 #pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    kf[c] = ld16(k + base + (int64_t)my_k * row_stride + 16 * c + 8 * h);
-    vf[c] = ld16(v + base + (int64_t)my_k * row_stride + 16 * c + 8 * h);
+  for (int c = 0; c < HD / 16; ++c) {
+    kf[c] = ld16(k + base + (int64_t)ld_k * row_stride + 16 * c + 8 * h);
+    vf[c] = ld16(v + base + (int64_t)ld_k * row_stride + 16 * c + 8 * h);
   }
-  TileDma dma;
-  dma.init(row_stride, wave, lane);
+  TileDma<HD> dma;
+  dma.init(row_stride, wave);
   const int qt0 = kb * kQRows / kKeys;  // the first query tile that sees these keys
   auto fetch_tile = [&](int j, int stage) __attribute__((always_inline)) {
     const int qs = (qt0 + j) * kKeys;
     const int64_t t0 = base + (int64_t)qs * row_stride;
-    dma.issue(q + t0, lds[stage][0]);
-    dma.issue(dout + t0, lds[stage][1]);
+    dma.issue(q + t0, lds[stage][0], row_stride, L - 1 - qs);
+    dma.issue(dout + t0, lds[stage][1], row_stride, L - 1 - qs);
   };
-  // the tile's 64 lse2 and 64 D values: 32 threads, one float4 each
-  auto load_stats = [&](int j, float4& out) __attribute__((always_inline)) {
-    const int qs = (qt0 + j) * kKeys;
-    if (tid < 32) out = *reinterpret_cast<const float4*>((tid < 16 ? lse2 : dvec) + stat0 + qs + 4 * (tid & 15));
+  // the tile's 64 lse2 and 64 D values, one per thread of the first two waves
+  // (queries past the end: lse2 = +inf, so that P = 0)
+  auto load_stats = [&](int j, float& out) __attribute__((always_inline)) {
+    const int qs = (qt0 + j) * kKeys + (tid & 63);
+    if (tid < 128) out = qs < L ? (tid < 64 ? lse2 : dvec)[stat0 + qs] : (tid < 64 ? __builtin_inff() : 0.f);
   };
-  auto store_stats = [&](int stage, const float4& val) __attribute__((always_inline)) {
-    if (tid < 32) *reinterpret_cast<float4*>(&stats[stage][tid >> 4][4 * (tid & 15)]) = val;
+  auto store_stats = [&](int stage, float val) __attribute__((always_inline)) {
+    if (tid < 128) stats[stage][tid >> 6][tid & 63] = val;
   };
-  attn_f32x16 dkacc[2], dvacc[2];
+  attn_f32x16 dkacc[HD / 32], dvacc[HD / 32];
 #pragma unroll
-  for (int t = 0; t < 2; ++t)
+  for (int t = 0; t < HD / 32; ++t)
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       dkacc[t][r] = 0.f;
@@ -497,9 +532,9 @@ __device__ __attribute__((always_inline)) inline void attn_bwd_dkdv_block(
     for (int qh = 0; qh < 2; ++qh) {
       attn_f32x16 sc = zero, dp = zero;
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        mfma32(sc, frag_k(qt, 32 * qh, c, lane), kf[c]);
-        mfma32(dp, frag_k(dt, 32 * qh, c, lane), vf[c]);
+      for (int c = 0; c < HD / 16; ++c) {
+        mfma32(sc, frag_k<HD>(qt, 32 * qh, c, lane), kf[c]);
+        mfma32(dp, frag_k<HD>(dt, 32 * qh, c, lane), vf[c]);
       }
       attn_f32x16 pz;  // P, then sc becomes dz
 #pragma unroll
@@ -525,9 +560,9 @@ __device__ __attribute__((always_inline)) inline void attn_bwd_dkdv_block(
         const Vec16 pf = row_chunk_operand(pz, c2);
         const Vec16 zf = row_chunk_operand(sc, c2);
 #pragma unroll
-        for (int t = 0; t < 2; ++t) {
-          mfma32(dvacc[t], frag_vt(dt, 32 * t, c, lane), pf);
-          mfma32(dkacc[t], frag_vt(qt, 32 * t, c, lane), zf);
+        for (int t = 0; t < HD / 32; ++t) {
+          mfma32(dvacc[t], frag_vt<HD>(dt, 32 * t, c, lane), pf);
+          mfma32(dkacc[t], frag_vt<HD>(qt, 32 * t, c, lane), zf);
         }
       }
     }
@@ -535,9 +570,9 @@ __device__ __attribute__((always_inline)) inline void attn_bwd_dkdv_block(
 
   constexpr int kAhead = kStages - 1;
   static_assert(kAhead == 1, "the stats are staged one tile ahead");
-  const int ntiles = L / kKeys - qt0;
+  const int ntiles = (L + kKeys - 1) / kKeys - qt0;
   {
-    float4 st0 = make_float4(0.f, 0.f, 0.f, 0.f);
+    float st0 = 0.f;
     fetch_tile(0, 0);
     load_stats(0, st0);
     store_stats(0, st0);
@@ -546,7 +581,7 @@ __device__ __attribute__((always_inline)) inline void attn_bwd_dkdv_block(
     const int buf = j % kStages;
     wait_vmcnt<0>();
     __syncthreads();
-    float4 st = make_float4(0.f, 0.f, 0.f, 0.f);
+    float st = 0.f;
     const bool more = j + 1 < ntiles;
     if (more) {
       fetch_tile(j + 1, (j + 1) % kStages);
@@ -560,10 +595,11 @@ __device__ __attribute__((always_inline)) inline void attn_bwd_dkdv_block(
     }
     if (more) store_stats((j + 1) % kStages, st);
   }
+  if (my_k >= L) return;
   uint16_t* krow = dk + base + (int64_t)my_k * row_stride;
   uint16_t* vrow = dv + base + (int64_t)my_k * row_stride;
 #pragma unroll
-  for (int t = 0; t < 2; ++t)
+  for (int t = 0; t < HD / 32; ++t)
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
       uint2 w;
@@ -576,18 +612,58 @@ __device__ __attribute__((always_inline)) inline void attn_bwd_dkdv_block(
     }
 }
 
-__global__ __launch_bounds__(kAttnThreads) void attn_bwd_dkdv_kernel(
+template <int HD>
+__global__ __launch_bounds__(kAttnThreads, HD == 64 ? 2 : 1) void attn_bwd_dkdv_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
     const uint16_t* __restrict__ dout, const float* __restrict__ lse2, const float* __restrict__ dvec, int L, int H,
     float scale_log2, float scale, uint16_t* __restrict__ dk, uint16_t* __restrict__ dv) {
-  __shared__ __attribute__((aligned(1024))) AttnRing lds;
+  __shared__ __attribute__((aligned(1024))) AttnRing<HD> lds;
   __shared__ __attribute__((aligned(16))) AttnStats stats;
-  const int nk = L / kQRows, p = blockIdx.x;
-  attn_bwd_dkdv_block(q, k, v, dout, lse2, dvec, L, H, scale_log2, scale, dk, dv, p, lds, stats);
+  const int nk = (L + kQRows - 1) / kQRows, p = blockIdx.x;
+  attn_bwd_dkdv_block<HD>(q, k, v, dout, lse2, dvec, L, H, scale_log2, scale, dk, dv, p, lds, stats);
   if (p != nk - 1 - p) {
     __syncthreads();
-    attn_bwd_dkdv_block(q, k, v, dout, lse2, dvec, L, H, scale_log2, scale, dk, dv, nk - 1 - p, lds, stats);
+    attn_bwd_dkdv_block<HD>(q, k, v, dout, lse2, dvec, L, H, scale_log2, scale, dk, dv, nk - 1 - p, lds, stats);
   }
+}
+
+int check_attention(int64_t B, int64_t L, int64_t H, int64_t K, int dtype) {
+  ABACUS_CHECK_ARG(dtype == kBF16, "attention: bf16 only (dtype code %d)", dtype);
+  ABACUS_CHECK_ARG(K == 64 || K == 128, "attention: head_dim %lld (these kernels take 64 and 128)", (long long)K);
+  ABACUS_CHECK_ARG(B >= 1 && H >= 1 && L >= 1 && L <= (1 << 24), "attention: seq_len %lld out of range", (long long)L);
+  ABACUS_CHECK_ARG(B * H * L * K < (1ll << 40) && H * K < (1 << 24) && B <= 65535 && H <= 65535, "attention: shape too large");
+  return 0;
+}
+
+template <int HD>
+int launch_fwd(const uint16_t* q, const uint16_t* k, const uint16_t* v, int64_t B, int64_t L, int64_t H, float scale,
+               uint16_t* o, float* lse, hipStream_t s) {
+  const int64_t nq = (L + kQRows - 1) / kQRows;
+  const float scale_log2 = scale * 1.4426950408889634f;  // scores to base 2
+  hipLaunchKernelGGL(attn_fwd_kernel<HD>, dim3((unsigned)((nq + 1) / 2), (unsigned)H, (unsigned)B), dim3(kAttnThreads),
+                     0, s, q, k, v, (int)L, (int)H, scale_log2, o, lse);
+  ABACUS_CHECK_LAUNCH("attention_fwd");
+  return 0;
+}
+
+template <int HD>
+int launch_bwd(const uint16_t* q, const uint16_t* k, const uint16_t* v, const uint16_t* o, const uint16_t* dout,
+               const float* lse, int64_t B, int64_t L, int64_t H, float scale, uint16_t* dq, uint16_t* dk, uint16_t* dv,
+               float* ws, hipStream_t s) {
+  const int64_t rows = B * L * H, nq = (L + kQRows - 1) / kQRows;
+  const float scale_log2 = scale * 1.4426950408889634f;
+  constexpr int kDotRows = 256 / (HD / 8);
+  hipLaunchKernelGGL(attn_bwd_dot_kernel<HD>, dim3((unsigned)((rows + kDotRows - 1) / kDotRows)), dim3(256), 0, s, o,
+                     dout, rows, (int)L, (int)H, ws);
+  ABACUS_CHECK_LAUNCH("attention_bwd (dot)");
+  const dim3 grid((unsigned)((nq + 1) / 2), (unsigned)H, (unsigned)B);  // block pairs
+  hipLaunchKernelGGL(attn_bwd_dkdv_kernel<HD>, grid, dim3(kAttnThreads), 0, s, q, k, v, dout, lse, ws, (int)L, (int)H,
+                     scale_log2, scale, dk, dv);
+  ABACUS_CHECK_LAUNCH("attention_bwd (dk, dv)");
+  hipLaunchKernelGGL(attn_bwd_dq_kernel<HD>, grid, dim3(kAttnThreads), 0, s, q, k, v, dout, lse, ws, (int)L, (int)H,
+                     scale_log2, scale, dq);
+  ABACUS_CHECK_LAUNCH("attention_bwd (dq)");
+  return 0;
 }
 
 }  // namespace
@@ -595,37 +671,35 @@ __global__ __launch_bounds__(kAttnThreads) void attn_bwd_dkdv_kernel(
 
 using namespace abacus;
 
+extern "C" int abacus_attention_any_fwd(const void* q_BLHK, const void* k_BLHK, const void* v_BLHK, int64_t B,
+                                        int64_t L, int64_t H, int64_t K, float scale, int dtype, void* o_BLHK,
+                                        float* lse_BHL, void* stream) {
+  if (check_attention(B, L, H, K, dtype)) return 1;
+  ABACUS_CHECK_ARG(q_BLHK && k_BLHK && v_BLHK && o_BLHK && lse_BHL, "attention: null pointer");
+  ABACUS_CHECK_ARG(((uintptr_t)q_BLHK | (uintptr_t)k_BLHK | (uintptr_t)v_BLHK | (uintptr_t)o_BLHK) % 16 == 0,
+                   "attention: q, k, v, o must be 16-byte aligned");
+  return (K == 64 ? launch_fwd<64> : launch_fwd<128>)((const uint16_t*)q_BLHK, (const uint16_t*)k_BLHK,
+                                                      (const uint16_t*)v_BLHK, B, L, H, scale, (uint16_t*)o_BLHK,
+                                                      lse_BHL, (hipStream_t)stream);
+}
+
 extern "C" int abacus_attention_fwd(const void* q_BLHK, const void* k_BLHK, const void* v_BLHK, int64_t B, int64_t L,
                                     int64_t H, int64_t K, float scale, int dtype, void* o_BLHK, float* lse_BHL,
                                     void* stream) {
   ABACUS_CHECK_ARG(dtype == kBF16, "attention: bf16 only (dtype code %d)", dtype);
-  ABACUS_CHECK_ARG(K == kHeadDim, "attention: head_dim %lld (this kernel takes %d)", (long long)K, kHeadDim);
-  ABACUS_CHECK_ARG(B >= 1 && H >= 1 && L >= kQRows && L % kQRows == 0 && L <= (1 << 24),
-                   "attention: seq_len %lld must be a positive multiple of %d", (long long)L, kQRows);
-  ABACUS_CHECK_ARG(B * H * L * K < (1ll << 40) && B <= 65535 && H <= 65535, "attention: shape too large");
-  ABACUS_CHECK_ARG(q_BLHK && k_BLHK && v_BLHK && o_BLHK && lse_BHL, "attention: null pointer");
-  ABACUS_CHECK_ARG(((uintptr_t)q_BLHK | (uintptr_t)k_BLHK | (uintptr_t)v_BLHK | (uintptr_t)o_BLHK) % 16 == 0,
-                   "attention: q, k, v, o must be 16-byte aligned");
-  const float scale_log2 = scale * 1.4426950408889634f;  // scores to base 2
-  hipLaunchKernelGGL(attn_fwd_kernel, dim3((unsigned)((L / kQRows + 1) / 2), (unsigned)H, (unsigned)B),
-                     dim3(kAttnThreads), 0,
-                     (hipStream_t)stream, (const uint16_t*)q_BLHK, (const uint16_t*)k_BLHK, (const uint16_t*)v_BLHK,
-                     (int)L, (int)H, scale_log2, (uint16_t*)o_BLHK, lse_BHL);
-  ABACUS_CHECK_LAUNCH("attention_fwd");
-  return 0;
+  ABACUS_CHECK_ARG(K == 64, "attention: head_dim %lld (this entry point takes 64)", (long long)K);
+  ABACUS_CHECK_ARG(L >= kQRows && L % kQRows == 0, "attention: seq_len %lld must be a positive multiple of %d",
+                   (long long)L, kQRows);
+  return abacus_attention_any_fwd(q_BLHK, k_BLHK, v_BLHK, B, L, H, K, scale, dtype, o_BLHK, lse_BHL, stream);
 }
 
 extern "C" int64_t abacus_attention_bwd_ws_bytes(int64_t B, int64_t L, int64_t H) { return B * H * L * 4; }
 
-extern "C" int abacus_attention_bwd(const void* q_BLHK, const void* k_BLHK, const void* v_BLHK, const void* o_BLHK,
-                                    const void* dout_BLHK, const float* lse_BHL, int64_t B, int64_t L, int64_t H,
-                                    int64_t K, float scale, int dtype, void* dq_BLHK, void* dk_BLHK, void* dv_BLHK,
-                                    float* ws, int64_t ws_bytes, void* stream) {
-  ABACUS_CHECK_ARG(dtype == kBF16, "attention: bf16 only (dtype code %d)", dtype);
-  ABACUS_CHECK_ARG(K == kHeadDim, "attention: head_dim %lld (this kernel takes %d)", (long long)K, kHeadDim);
-  ABACUS_CHECK_ARG(B >= 1 && H >= 1 && L >= kQRows && L % kQRows == 0 && L <= (1 << 24),
-                   "attention: seq_len %lld must be a positive multiple of %d", (long long)L, kQRows);
-  ABACUS_CHECK_ARG(B * H * L * K < (1ll << 40) && B <= 65535 && H <= 65535, "attention: shape too large");
+extern "C" int abacus_attention_any_bwd(const void* q_BLHK, const void* k_BLHK, const void* v_BLHK, const void* o_BLHK,
+                                        const void* dout_BLHK, const float* lse_BHL, int64_t B, int64_t L, int64_t H,
+                                        int64_t K, float scale, int dtype, void* dq_BLHK, void* dk_BLHK, void* dv_BLHK,
+                                        float* ws, int64_t ws_bytes, void* stream) {
+  if (check_attention(B, L, H, K, dtype)) return 1;
   ABACUS_CHECK_ARG(q_BLHK && k_BLHK && v_BLHK && o_BLHK && dout_BLHK && lse_BHL && dq_BLHK && dk_BLHK && dv_BLHK && ws,
                    "attention: null pointer");
   ABACUS_CHECK_ARG(((uintptr_t)q_BLHK | (uintptr_t)k_BLHK | (uintptr_t)v_BLHK | (uintptr_t)o_BLHK |
@@ -634,20 +708,20 @@ extern "C" int abacus_attention_bwd(const void* q_BLHK, const void* k_BLHK, cons
                    "attention: tensors must be 16-byte aligned");
   ABACUS_CHECK_ARG(ws_bytes >= B * H * L * 4, "attention_bwd: workspace of %lld bytes, need %lld",
                    (long long)ws_bytes, (long long)(B * H * L * 4));
-  const hipStream_t s = (hipStream_t)stream;
-  const int64_t rows = B * L * H;
-  const float scale_log2 = scale * 1.4426950408889634f;
-  hipLaunchKernelGGL(attn_bwd_dot_kernel, dim3((unsigned)((rows + 31) / 32)), dim3(256), 0, s,
-                     (const uint16_t*)o_BLHK, (const uint16_t*)dout_BLHK, rows, (int)L, (int)H, ws);
-  ABACUS_CHECK_LAUNCH("attention_bwd (dot)");
-  const dim3 grid((unsigned)((L / kQRows + 1) / 2), (unsigned)H, (unsigned)B);  // block pairs
-  hipLaunchKernelGGL(attn_bwd_dkdv_kernel, grid, dim3(kAttnThreads), 0, s, (const uint16_t*)q_BLHK,
-                     (const uint16_t*)k_BLHK, (const uint16_t*)v_BLHK, (const uint16_t*)dout_BLHK, lse_BHL, ws,
-                     (int)L, (int)H, scale_log2, scale, (uint16_t*)dk_BLHK, (uint16_t*)dv_BLHK);
-  ABACUS_CHECK_LAUNCH("attention_bwd (dk, dv)");
-  hipLaunchKernelGGL(attn_bwd_dq_kernel, grid, dim3(kAttnThreads), 0, s, (const uint16_t*)q_BLHK,
-                     (const uint16_t*)k_BLHK, (const uint16_t*)v_BLHK, (const uint16_t*)dout_BLHK, lse_BHL, ws,
-                     (int)L, (int)H, scale_log2, scale, (uint16_t*)dq_BLHK);
-  ABACUS_CHECK_LAUNCH("attention_bwd (dq)");
-  return 0;
+  return (K == 64 ? launch_bwd<64> : launch_bwd<128>)(
+      (const uint16_t*)q_BLHK, (const uint16_t*)k_BLHK, (const uint16_t*)v_BLHK, (const uint16_t*)o_BLHK,
+      (const uint16_t*)dout_BLHK, lse_BHL, B, L, H, scale, (uint16_t*)dq_BLHK, (uint16_t*)dk_BLHK, (uint16_t*)dv_BLHK,
+      ws, (hipStream_t)stream);
+}
+
+extern "C" int abacus_attention_bwd(const void* q_BLHK, const void* k_BLHK, const void* v_BLHK, const void* o_BLHK,
+                                    const void* dout_BLHK, const float* lse_BHL, int64_t B, int64_t L, int64_t H,
+                                    int64_t K, float scale, int dtype, void* dq_BLHK, void* dk_BLHK, void* dv_BLHK,
+                                    float* ws, int64_t ws_bytes, void* stream) {
+  ABACUS_CHECK_ARG(dtype == kBF16, "attention: bf16 only (dtype code %d)", dtype);
+  ABACUS_CHECK_ARG(K == 64, "attention: head_dim %lld (this entry point takes 64)", (long long)K);
+  ABACUS_CHECK_ARG(L >= kQRows && L % kQRows == 0, "attention: seq_len %lld must be a positive multiple of %d",
+                   (long long)L, kQRows);
+  return abacus_attention_any_bwd(q_BLHK, k_BLHK, v_BLHK, o_BLHK, dout_BLHK, lse_BHL, B, L, H, K, scale, dtype, dq_BLHK,
+                                  dk_BLHK, dv_BLHK, ws, ws_bytes, stream);
 }

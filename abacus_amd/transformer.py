@@ -15,7 +15,7 @@ reference's:
 
 The MoE layer inside each block is abacus_amd.moe.MoE (the HIP path).  On
 the GPU, RMSNorm, the q/k norms fused with the rotary embedding, and causal
-attention in bf16 with head dim 64 (L a multiple of 128) also run on this
+attention in bf16 with head dim 64 or 128 also run on this
 library's HIP kernels; the (L, L) scores never reach HBM and stay fp32 where
 the reference rounds them to the activation dtype.  Other attention inputs go
 to torch's fused causal kernels (flash / memory-efficient), and on the CPU,
@@ -291,9 +291,16 @@ def _fused_causal_attention(q, k, v):
 
 
 def _flash_ok(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> bool:
-    """abacus_attention_fwd takes contiguous bf16 (B, L, H, 64) q, k, v on the GPU, L a multiple of 128."""
-    return (q.is_cuda and q.dim() == 4 and q.dtype == torch.bfloat16 and q.shape[-1] == 64 and q.shape[1] % 128 == 0
+    """The HIP flash kernels take contiguous bf16 (B, L, H, 64 or 128) q, k, v on the GPU, any L >= 1."""
+    return (q.is_cuda and q.dim() == 4 and q.dtype == torch.bfloat16 and q.shape[-1] in (64, 128) and q.numel() > 0
+            and q.shape[0] <= 65535 and q.shape[2] <= 65535 and q.shape[2] * q.shape[3] < 1 << 24
             and all(t.dtype == q.dtype and t.shape == q.shape and t.is_contiguous() for t in (q, k, v)))
+
+
+def _flash_entry(q: torch.Tensor, direction: str) -> str:
+    """abacus_attention_* for whole 128-token blocks of 64-wide heads, abacus_attention_any_* for the rest."""
+    whole = q.shape[1] % 128 == 0 and q.shape[3] == 64
+    return f"abacus_attention_{direction}" if whole else f"abacus_attention_any_{direction}"
 
 
 class _FlashAttentionFunction(torch.autograd.Function):
@@ -309,7 +316,7 @@ class _FlashAttentionFunction(torch.autograd.Function):
         B, L, H, K = q_BLHK.shape
         o = torch.empty_like(q_BLHK)
         lse = torch.empty(B, H, L, dtype=torch.float32, device=q_BLHK.device)
-        _lib.call("abacus_attention_fwd", _lib.ptr(q_BLHK), _lib.ptr(k_BLHK), _lib.ptr(v_BLHK), B, L, H, K,
+        _lib.call(_flash_entry(q_BLHK, "fwd"), _lib.ptr(q_BLHK), _lib.ptr(k_BLHK), _lib.ptr(v_BLHK), B, L, H, K,
                   1.0 / math.sqrt(K), _lib.BF16, _lib.ptr(o), _lib.ptr(lse), _lib.stream_of(q_BLHK.device))
         ctx.save_for_backward(q_BLHK, k_BLHK, v_BLHK, o, lse)
         return o
@@ -322,7 +329,7 @@ class _FlashAttentionFunction(torch.autograd.Function):
         dq, dk, dv = (torch.empty_like(q) for _ in range(3))
         nbytes = _lib.query("abacus_attention_bwd_ws_bytes", B, L, H)
         ws = torch.empty(nbytes // 4, dtype=torch.float32, device=q.device)
-        _lib.call("abacus_attention_bwd", _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(o), _lib.ptr(d_o),
+        _lib.call(_flash_entry(q, "bwd"), _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(o), _lib.ptr(d_o),
                   _lib.ptr(lse), B, L, H, K, 1.0 / math.sqrt(K), _lib.BF16, _lib.ptr(dq), _lib.ptr(dk), _lib.ptr(dv),
                   _lib.ptr(ws), nbytes, _lib.stream_of(q.device))
         return dq, dk, dv

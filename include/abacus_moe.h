@@ -293,7 +293,11 @@ int abacus_rmsnorm_rope_bwd(const void* dy, const void* x, const void* gamma, co
 int abacus_attention_fwd(const void* q_BLHK, const void* k_BLHK, const void* v_BLHK, int64_t B, int64_t L, int64_t H,
                          int64_t K, float scale, int dtype, void* o_BLHK, float* lse_BHL, void* stream);
 
-/* Bytes of fp32 workspace abacus_attention_bwd needs (one value per query). */
+/* The same for any L >= 1 and K = 64 or 128. */
+int abacus_attention_any_fwd(const void* q_BLHK, const void* k_BLHK, const void* v_BLHK, int64_t B, int64_t L,
+                             int64_t H, int64_t K, float scale, int dtype, void* o_BLHK, float* lse_BHL, void* stream);
+
+/* Bytes of fp32 workspace the attention backward needs (one value per query). */
 int64_t abacus_attention_bwd_ws_bytes(int64_t B, int64_t L, int64_t H);
 
 /* Causal attention backward: the gradients of abacus_attention_fwd's o with
@@ -307,6 +311,12 @@ int abacus_attention_bwd(const void* q_BLHK, const void* k_BLHK, const void* v_B
                          const void* dout_BLHK, const float* lse_BHL, int64_t B, int64_t L, int64_t H, int64_t K,
                          float scale, int dtype, void* dq_BLHK, void* dk_BLHK, void* dv_BLHK, float* ws,
                          int64_t ws_bytes, void* stream);
+
+/* The same for any L >= 1 and K = 64 or 128 (abacus_attention_any_fwd's o and lse_BHL). */
+int abacus_attention_any_bwd(const void* q_BLHK, const void* k_BLHK, const void* v_BLHK, const void* o_BLHK,
+                             const void* dout_BLHK, const float* lse_BHL, int64_t B, int64_t L, int64_t H, int64_t K,
+                             float scale, int dtype, void* dq_BLHK, void* dk_BLHK, void* dv_BLHK, float* ws,
+                             int64_t ws_bytes, void* stream);
 
 /* Cross-entropy of the decoder's logits (kernels/liger.py:12-47, called at
  * trainer.py:81-85), forward: for the N rows of logits_NV ((N, V), `dtype`)
