@@ -62,6 +62,10 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "abacus_moe_router_wgrad_noalloc": (_I, [_P, _P, _P, _I64, _I64, _I64, _I64, _I, _P, _P]),
     "abacus_experts_decode_ws_bytes": (_I64, [_I64, _I64, _I64, _I64, _I]),
     "abacus_experts_decode_fwd": (_I, [_P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _I, _I64, _P, _P, _P, _I64, _P]),
+    "abacus_experts_pad_columns": (_I, [_P, _I64, _I64, _I64, _P, _P]),
+    "abacus_experts_down_fwd": (_I, [_P, _P, _P, _I64, _I64, _I64, _I64, _I64, _P, _P, _I64, _P]),
+    "abacus_experts_down_bwd": (_I, [_P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _P, _P, _P, _P, _P]),
+    "abacus_experts_gateup_bwd": (_I, [_P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _P, _P, _P, _P, _P]),
     "abacus_router_gating_bwd": (_I, [_P, _P, _P, _I64, _I64, _D, _I, _P, _P]),
     "abacus_router_update_bias": (_I, [_P, _I64, _I64, _D, _I, _P, _P]),
     "abacus_rmsnorm_fwd": (_I, [_P, _P, _I64, _I64, _F, _I, _P, _P, _P]),

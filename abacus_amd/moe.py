@@ -140,6 +140,19 @@ def _whole_vectors(n: int, x: torch.Tensor) -> int:
     return -(-n // vec) * vec
 
 
+def _hidden_pitch(M: int, x: torch.Tensor) -> int:
+    """Row pitch of the hidden activations: M, in bf16 on the GPU rounded up to whole vectors."""
+    return _whole_vectors(M, x) if x.is_cuda and x.dtype == torch.bfloat16 else M
+
+
+def _pad_columns(w_EDM: torch.Tensor, M: int, ld: int) -> torch.Tensor:
+    """A copy of bf16 w with rows of ld elements, zero past M."""
+    E, D, _ = w_EDM.shape
+    out = torch.empty(E, D, ld, dtype=w_EDM.dtype, device=w_EDM.device)
+    call("abacus_experts_pad_columns", ptr(w_EDM), E * D, M, ld, ptr(out), _lib.stream_of(w_EDM.device))
+    return out
+
+
 def _decode_ws_bytes(x_TD: torch.Tensor, R: int, M: int, E: int) -> int:
     """Workspace of abacus_experts_decode_fwd for R routed rows, -1 where it does not take the shape."""
     if not x_TD.is_cuda:
@@ -183,16 +196,24 @@ class _MoEFunction(torch.autograd.Function):
                 ld_h, ptr(h), ptr(y), ptr(ws), decode_ws, s,
             )
         else:
-            gate = torch.empty(R, M, dtype=x_TD.dtype, device=dev) if need_grad else None
-            up = torch.empty(R, M, dtype=x_TD.dtype, device=dev) if need_grad else None
-            h = torch.empty(R, M, dtype=x_TD.dtype, device=dev)
+            ld = _hidden_pitch(M, x_TD)
+            if ld != M:  # bf16 rows of gate and up weights start at any alignment: aligned copies, zero past M
+                w_gate, w_up = (_pad_columns(w, M, ld) for w in (w_gate, w_up))
+            gate = torch.empty(R, ld, dtype=x_TD.dtype, device=dev) if need_grad else None
+            up = torch.empty(R, ld, dtype=x_TD.dtype, device=dev) if need_grad else None
+            h = torch.empty(R, ld, dtype=x_TD.dtype, device=dev)
             call(
-                "abacus_moe_gateup_fwd", ptr(xp), ptr(w_gate), ptr(w_up), ptr(offsets), R, D, M, E, dt,
+                "abacus_moe_gateup_fwd", ptr(xp), ptr(w_gate), ptr(w_up), ptr(offsets), R, D, ld, E, dt,
                 ptr(gate), ptr(up), ptr(h), s,
             )
-            ws_bytes = _lib.query("abacus_moe_down_fwd_ws_bytes", R, M, D, E, dt, device=dev)
+            ws_bytes = _lib.query("abacus_moe_down_fwd_ws_bytes", R, ld, D, E, dt, device=dev)
             ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes > 0 else None
-            call("abacus_moe_down_fwd", ptr(h), ptr(w_down), ptr(offsets), R, M, D, E, dt, ptr(y), ptr(ws), ws_bytes, s)
+            if ld != M:
+                call("abacus_experts_down_fwd", ptr(h), ptr(w_down), ptr(offsets), R, M, ld, D, E, ptr(y), ptr(ws),
+                     ws_bytes, s)
+            else:
+                call("abacus_moe_down_fwd", ptr(h), ptr(w_down), ptr(offsets), R, M, D, E, dt, ptr(y), ptr(ws),
+                     ws_bytes, s)
         out = torch.empty(T, D, dtype=x_TD.dtype, device=dev)
         call("abacus_moe_combine_fwd", ptr(y), ptr(weights), ptr(idx32), ptr(pos), T, D, K, dt, ptr(out), s)
         if need_grad:
@@ -208,7 +229,7 @@ class _MoEFunction(torch.autograd.Function):
         (x_TD, w_DE, w_gate, w_up, w_down, xp, gate, up, h, y, weights, score, idx32, pos,
          offsets, wt) = ctx.saved_tensors
         T, D = x_TD.shape
-        E, _, M = w_gate.shape
+        E, M, _ = w_down.shape
         K = idx32.shape[1]
         R = T * K
         dev, dt = x_TD.device, _lib.dtype_code(x_TD.dtype, x_TD.device)
@@ -223,8 +244,24 @@ class _MoEFunction(torch.autograd.Function):
         )
         # Each data gradient and the weight gradient beside it go in one launch
         # when both are wanted (abacus_moe_down_bwd / abacus_moe_gateup_bwd).
-        dgate = torch.empty(R, M, dtype=x_TD.dtype, device=dev)
-        dup = torch.empty(R, M, dtype=x_TD.dtype, device=dev)
+        ld = gate.shape[1]
+        dgate = torch.empty(R, ld, dtype=x_TD.dtype, device=dev)
+        dup = torch.empty(R, ld, dtype=x_TD.dtype, device=dev)
+        if ld != M:  # w_gate and w_up are the forward's padded copies
+            dw_down = torch.empty_like(w_down)
+            dw_gate, dw_up = (torch.empty(E, D, M, dtype=x_TD.dtype, device=dev) for _ in range(2))
+            dxp = torch.empty(R, D, dtype=x_TD.dtype, device=dev)
+            call(
+                "abacus_experts_down_bwd", ptr(dy), ptr(w_down), ptr(gate), ptr(up), ptr(h), ptr(offsets), R, M, ld, D, E,
+                ptr(dgate), ptr(dup), ptr(dw_down), ptr(_lib.tile_ctr(dev)), s,
+            )
+            call(
+                "abacus_experts_gateup_bwd", ptr(dgate), ptr(dup), ptr(w_gate), ptr(w_up), ptr(xp), ptr(offsets), R, D, M,
+                ld, E, ptr(dxp), ptr(dw_gate), ptr(dw_up), ptr(_lib.tile_ctr(dev)), s,
+            )
+            dx, dw_DE = _router_dgrad_wgrad(needs[0], needs[1], x_TD, w_DE, dlogit, idx32, pos, dxp, wt)
+            return (dx, dw_DE, dw_gate if needs[2] else None, dw_up if needs[3] else None,
+                    dw_down if needs[4] else None, None, None, None, None, None, None)
         dw_down = None
         if needs[4]:
             dw_down = torch.empty_like(w_down)
@@ -435,7 +472,7 @@ class MoE(torch.nn.Module):
         D, M = self.dim, self.w_gate_EDM.shape[2]
         Dp, Mp = _whole_vectors(D, x_TD), _whole_vectors(M, x_TD)  # the GPU kernels move rows in 16-byte vectors
         need_grad = torch.is_grad_enabled() and any(t.requires_grad for t in operands)
-        padded = x_TD.is_cuda and (Dp != D or Mp != M)
+        padded = x_TD.is_cuda and (Dp != D or _hidden_pitch(M, x_TD) != Mp)
         if padded and not need_grad:  # (a small forward batch streams weight rows of any length)
             padded = _decode_ws_bytes(x_TD, x_TD.shape[0] * self.top_k, M, self.n_experts) < 0
         if padded:

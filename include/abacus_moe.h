@@ -141,6 +141,24 @@ int abacus_experts_decode_fwd(const void* x_perm_RD, const void* w_gate_EDM, con
                               int64_t E, int dtype, int64_t ld_h, void* h, void* y_RD, void* ws, int64_t ws_bytes,
                               void* stream);
 
+/* The expert products in bf16 for a hidden size M that is not whole 16-byte
+ * vectors (GPU only).  The hidden activations (gate, up, h, dgate, dup) have rows
+ * of ld = M rounded up to 8 elements, zero past M; pad_columns copies w_gate and
+ * w_up (E*D rows of M) into rows of ld, which abacus_moe_gateup_fwd takes as a
+ * hidden size of ld; w_down, and every weight gradient, keep rows and columns of
+ * M.  Otherwise as abacus_moe_down_fwd (workspace of abacus_moe_down_fwd_ws_bytes
+ * for ld), abacus_moe_down_bwd and abacus_moe_gateup_bwd. */
+int abacus_experts_pad_columns(const void* src, int64_t rows, int64_t M, int64_t ld, void* dst, void* stream);
+int abacus_experts_down_fwd(const void* h, const void* w_down_EMD, const int32_t* offsets_E1, int64_t R, int64_t M,
+                            int64_t ld, int64_t D, int64_t E, void* y_RD, void* ws, int64_t ws_bytes, void* stream);
+int abacus_experts_down_bwd(const void* dy_RD, const void* w_down_EMD, const void* gate, const void* up, const void* h,
+                            const int32_t* offsets_E1, int64_t R, int64_t M, int64_t ld, int64_t D, int64_t E,
+                            void* dgate, void* dup, void* dw_down_EMD, int32_t* tile_ctr, void* stream);
+int abacus_experts_gateup_bwd(const void* dgate, const void* dup, const void* w_gate_pad, const void* w_up_pad,
+                              const void* x_perm_RD, const int32_t* offsets_E1, int64_t R, int64_t D, int64_t M,
+                              int64_t ld, int64_t E, void* dx_perm_RD, void* dw_gate_EDM, void* dw_up_EDM,
+                              int32_t* tile_ctr, void* stream);
+
 /* Replaces moe.py:81-85: out[t] = sum over the token's experts (ascending)
  * of y[pos(t,k)] * weights_TK[t,k]. */
 int abacus_moe_combine_fwd(const void* y_RD, const void* weights_TK, const int32_t* idx_TK, const int32_t* pos_TK,
