@@ -65,7 +65,9 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "abacus_experts_pad_columns": (_I, [_P, _I64, _I64, _I64, _P, _P]),
     "abacus_experts_down_fwd": (_I, [_P, _P, _P, _I64, _I64, _I64, _I64, _I64, _P, _P, _I64, _P]),
     "abacus_experts_down_bwd": (_I, [_P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _P, _P, _P, _P, _P]),
-    "abacus_experts_gateup_bwd": (_I, [_P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _P, _P, _P, _P, _P]),
+    "abacus_experts_gateup_bwd_ws_bytes": (_I64, [_I64, _I64, _I64, _I64, _I]),
+    "abacus_experts_gateup_bwd": (_I, [_P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _I, _P, _P, _P, _P, _P, _I64,
+                                       _P]),
     "abacus_router_gating_bwd": (_I, [_P, _P, _P, _I64, _I64, _D, _I, _P, _P]),
     "abacus_router_update_bias": (_I, [_P, _I64, _I64, _D, _I, _P, _P]),
     "abacus_rmsnorm_fwd": (_I, [_P, _P, _I64, _I64, _F, _I, _P, _P, _P]),

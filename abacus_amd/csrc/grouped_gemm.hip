@@ -22,6 +22,7 @@
 // v_mfma_f32_16x16x4_f32; accumulation is always fp32.
 #include <algorithm>
 #include <atomic>
+#include <cmath>
 #include <type_traits>
 
 #include "common.h"
@@ -91,6 +92,12 @@ struct GemmArgs {
   // split_parts <= 1: every tile runs whole.
   int split_from, split_parts, split_cus;
   float* split_ws;
+  // Sliced launch (pipelined kernel, row-grouped kinds without a fused
+  // epilogue): every tile runs as ksplit slices of the reduction, each writing
+  // its rows of an fp32 (ksplit, R, Ndim) workspace, which rows_reduce_kernel
+  // adds in slice order.  <= 1: none.
+  int ksplit;
+  float* ksplit_ws;
   // Pipelined kernel, row-grouped kinds: nonzero when expert remainders of at
   // most THIN rows go to thin tiles (else every row tile is a full one).
   int thin;
@@ -815,19 +822,31 @@ __device__ inline bool find_row_tile(const GemmArgs& g, int mt, int& e, int& row
   return false;
 }
 
-__device__ inline void row_tile(int r, int mt_real, int NTp, int& mt, int& nt) {
-  const int full = (mt_real / GM) * GM * NTp;  // tiles in whole groups of GM rows
+// Real tile r of mt_real row tiles x NT column tiles -> its row and column tile:
+// groups of GM rows x GN columns, column group by column group, the last rows'
+// and the last columns' groups short.  Every number is a real tile: a block
+// without one, between others, costs more than its launch, because the dispatcher
+// gives the shader engines their blocks in a fixed turn, whatever they still run.
+// With NT padded to whole column groups, N = 320 (two tiles of four real) left
+// half of each XCD idle (us, padded -> now): bf16 E 64 D 320 M 11456, 2135 tokens
+// top-2, sliced down forward 240 -> 151; E 128 D 2048 M 768, 8192 tokens top-8,
+// gate/up forward (6 of 8) 669 -> 551, down backward (3 of 4) 663 -> 608.
+__device__ inline void row_tile(int r, int mt_real, int NT, int& mt, int& nt) {
+  const int full = (mt_real / GM) * GM * NT;  // tiles in whole groups of GM rows
+  int rows = GM, m0 = 0;
   if (r < full) {
-    const int gi = r / (GM * GN), w = r % (GM * GN);
-    const int ngn = NTp / GN;
-    mt = (gi / ngn) * GM + w / GN;
-    nt = (gi % ngn) * GN + w % GN;
+    m0 = r / (GM * NT) * GM;
+    r %= GM * NT;
   } else {
-    const int rows = mt_real % GM;  // the short last group (nonzero when r >= full)
-    const int r2 = r - full;
-    mt = (mt_real / GM) * GM + (r2 % (rows * GN)) / GN;
-    nt = (r2 / (rows * GN)) * GN + r2 % GN;
+    rows = mt_real % GM;  // the short last group (nonzero when r >= full)
+    m0 = mt_real / GM * GM;
+    r -= full;
   }
+  const int c0 = r / (rows * GN) * GN;  // this column group's first tile
+  const int cols = min(GN, NT - c0);
+  r -= c0 * rows;
+  mt = m0 + r / cols;
+  nt = c0 + r % cols;
 }
 
 // Slices per tile of a split tail of `tail` tiles: enough to cover the CUs,
@@ -837,8 +856,18 @@ __device__ inline int split_slices(const GemmArgs& g, int tail) {
 }
 
 // Block b -> (real tile r, slice; -1 = whole).  False: the block has no tile.
-__device__ inline bool block_to_row_tile(const GemmArgs& g, int b, int total, int& r, int& part) {
+// A sliced launch (g.ksplit) numbers its slices innermost: kslice.
+__device__ inline bool block_to_row_tile(const GemmArgs& g, int b, int total, int& r, int& part, int& kslice) {
   part = -1;
+  kslice = 0;
+  if (g.ksplit > 1) {
+    const int units = total * g.ksplit, per = (units + 7) / 8, j = b >> 3;
+    const int u = (b & 7) * per + j;
+    if (j >= per || u >= units) return false;
+    r = u / g.ksplit;
+    kslice = u - r * g.ksplit;
+    return true;
+  }
   if (g.split_parts > 1) {
     const int whole = total / g.split_cus * g.split_cus;
     if (b < g.split_from) {
@@ -906,12 +935,13 @@ __device__ __attribute__((always_inline)) inline void gemm_tile(const GemmArgs& 
   // ---------------- tile -> (expert, rows, columns) ----------------
   int e = -1, row0 = 0, row_end = 0, k_len = 0, n0 = 0;
   int part = -1, slot = 0;  // slice of a split tail tile, its workspace slot
+  int kslice = 0;           // slice of a sliced launch
   TileId tl;
   if (!KT::WGRAD) {
     const int mt_real = ri->total[BMT == BM ? 0 : 1];
     const int total = mt_real * g.tiles_n;
     int r;
-    if (!block_to_row_tile(g, b, total, r, part)) return;
+    if (!block_to_row_tile(g, b, total, r, part, kslice)) return;
     row_tile(r, mt_real, g.tiles_n, tl.mt, tl.nt);
     if (part >= 0) slot = r - total / g.split_cus * g.split_cus;
   } else {
@@ -952,6 +982,10 @@ __device__ __attribute__((always_inline)) inline void gemm_tile(const GemmArgs& 
     const int S = split_slices(g, ri->total[BMT == BM ? 0 : 1] * g.tiles_n % g.split_cus);
     const int per = (ktiles_all + S - 1) / S;
     kbase = part * per;
+    ktiles = max(0, min(per, ktiles_all - kbase));
+  } else if (!KT::WGRAD && g.ksplit > 1) {
+    const int per = (ktiles_all + g.ksplit - 1) / g.ksplit;
+    kbase = kslice * per;
     ktiles = max(0, min(per, ktiles_all - kbase));
   }
   const int a_lim = KT::WGRAD ? g.Mdim : row_end;
@@ -1126,6 +1160,27 @@ __device__ __attribute__((always_inline)) inline void gemm_tile(const GemmArgs& 
           *reinterpret_cast<float4*>(ws + (wm * WTM + i * 32 + rl) * BN + b_col(j) + 8 * gq + ch) =
               make_float4(acc[i][j][4 * gq], acc[i][j][4 * gq + 1], acc[i][j][4 * gq + 2], acc[i][j][4 * gq + 3]);
     return;
+  }
+  if constexpr (KIND == kDownFwd || KIND == kGateUpDgrad) {
+    if (g.ksplit > 1) {  // a slice of the whole launch: its fp32 rows, for rows_reduce_kernel
+      float* ws = g.ksplit_ws + (int64_t)kslice * g.Mdim * g.Ndim;
+      const int rl = lane & 31, ch = 4 * (lane >> 5);
+#pragma unroll
+      for (int i = 0; i < FM; ++i) {
+        const int row = row0 + wm * WTM + i * 32 + rl;
+        if (row >= row_end) continue;
+#pragma unroll
+        for (int j = 0; j < FN; ++j)
+#pragma unroll
+          for (int gq = 0; gq < 4; ++gq) {
+            const int col = n0 + b_col(j) + 8 * gq + ch;
+            if (col < g.Ndim)
+              *reinterpret_cast<float4*>(ws + (int64_t)row * g.Ndim + col) =
+                  make_float4(acc[i][j][4 * gq], acc[i][j][4 * gq + 1], acc[i][j][4 * gq + 2], acc[i][j][4 * gq + 3]);
+          }
+      }
+      return;
+    }
   }
   if constexpr (sizeof(T) == 4) {
     // fp32: the C tile (256 KB for 256 x 256) does not fit in LDS, so it goes
@@ -1693,6 +1748,31 @@ __global__ __launch_bounds__(NT, 1) void gemm_rows_kernel(GemmArgs g1, GemmArgs 
   }
 }
 
+// The output of a sliced launch: its slices added in slice order, four elements
+// per thread, rounded once to T.
+template <typename T>
+__global__ __launch_bounds__(256) void rows_reduce_kernel(const float* __restrict__ ws, int64_t n, int slices,
+                                                          T* __restrict__ out) {
+  const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
+  if (i >= n) return;
+  float4 t = *reinterpret_cast<const float4*>(ws + i);
+  for (int s = 1; s < slices; ++s) {
+    const float4 u = *reinterpret_cast<const float4*>(ws + s * n + i);
+    t.x += u.x;
+    t.y += u.y;
+    t.z += u.z;
+    t.w += u.w;
+  }
+  if constexpr (sizeof(T) == 4) {
+    *reinterpret_cast<float4*>(out + i) = t;
+  } else {
+    uint2 w;
+    w.x = pack_bf16x2(t.x, t.y);
+    w.y = pack_bf16x2(t.z, t.w);
+    *reinterpret_cast<uint2*>(out + i) = w;
+  }
+}
+
 // Adds the slices of each split tail tile in slice order and writes the tile
 // (kinds whose epilogue is a plain store of the product, rounded to T).  Block
 // (i, j) serves rows kSplitReduceRows j .. +kSplitReduceRows-1 of tail tile i:
@@ -1779,9 +1859,9 @@ int launch_gemm(const GemmArgs& g, int R, hipStream_t s, const char* name) {
   return 0;
 }
 
-// Sizes the padded logical tile space of a pipelined launch: MTp row tiles x
-// NTp column tiles (x E for wgrad), whole GM x GN groups.  Returns the number
-// of blocks (0: nothing to do).
+// Sizes the logical tile space of a pipelined launch: MTp row tiles x NT column
+// tiles (x E and whole GM x GN groups for wgrad).  Returns the number of blocks
+// (0: nothing to do).
 // Row-grouped kinds bound their full row tiles by sum_e ceil(S_e / BM) <=
 // ceil(R / BM) + E; with thin tiles (g.thin) every full tile covers more than
 // THIN rows, so there are at most R / (THIN + 1).
@@ -1793,9 +1873,9 @@ int64_t pipe_grid(GemmArgs& g, int R) {
                            : (g.thin ? R / (pipe::THIN + 1) : (R + pipe::BM - 1) / pipe::BM + g.E);
   const int nt = (g.Ndim + BNH - 1) / BNH;
   g.tiles_m = pipe::round_up(mt, pipe::GM);
-  g.tiles_n = pipe::round_up(nt, pipe::GN);
+  g.tiles_n = KT::WGRAD ? pipe::round_up(nt, pipe::GN) : nt;
   if (mt == 0 || nt == 0) return 0;
-  return (int64_t)(KT::WGRAD ? g.E : 1) * g.tiles_m * g.tiles_n;
+  return (int64_t)(KT::WGRAD ? g.E : 1) * g.tiles_m * g.tiles_n;  // (GM is 8: blocks b % 8 stay XCDs)
 }
 
 inline int cu_count();
@@ -1816,7 +1896,7 @@ template <typename T, int KIND>
 int64_t pipe_grid_thin(GemmArgs& g, int R) {
   static_assert(!KindTraits<KIND>::WGRAD, "row-grouped kinds");
   constexpr int BNH = KindTraits<KIND>::DUAL_B ? pipe::kThinN<T> / 2 : pipe::kThinN<T>;
-  g.tiles_n = pipe::round_up((g.Ndim + BNH - 1) / BNH, pipe::GN);
+  g.tiles_n = (g.Ndim + BNH - 1) / BNH;
   const int mt = std::min(g.E, R);  // at most one thin tile per expert with rows
   if (mt == 0 || g.tiles_n == 0) return 0;
   g.tiles_m = pipe::round_up(mt, pipe::GM);
@@ -1834,7 +1914,11 @@ int launch_rows(const GemmArgs& g1, int R, const GemmArgs* gw, int64_t n1, bool 
   ga.thin = gt.thin = thin ? 1 : 0;
   const int64_t full = pipe_grid<KR>(ga, R);
   if (n1 < 0) n1 = full;  // no split: one block per full tile of the upper bound
-  const int64_t n2 = thin ? pipe_grid_thin<T, KR>(gt, R) : 0;
+  int64_t n2 = thin ? pipe_grid_thin<T, KR>(gt, R) : 0;
+  if (g1.ksplit > 1) {
+    n1 *= g1.ksplit;
+    n2 *= g1.ksplit;
+  }
   int64_t n3 = 0;
   if constexpr (KW >= 0) {
     n3 = wgrad_blocks<KW>(gc, R);
@@ -1960,14 +2044,6 @@ int launch_pipe_split(const GemmArgs& g, int R, const SplitPlan& plan, float* ws
   return 0;
 }
 
-// A data gradient (KA, row-grouped: the long tiles, then its thin ones) and a
-// weight gradient (KB) in one launch.
-template <int KA, int KB>
-int launch_pipe_pair(const GemmArgs& a, int Ra, const GemmArgs& b, int Rb, hipStream_t s, const char* name) {
-  (void)Rb;
-  return launch_rows<uint16_t, KA, KB>(a, Ra, &b, -1, thin_tiles_pay<uint16_t>(Ra, a.E), s, name);
-}
-
 // The pipelined DMA kernel whenever every dimension it tiles is a whole
 // number of 16-byte chunks.  A fixed reduction that is not a whole number of
 // k-tiles takes the kernel's ragged form (its last k-tile reads zeros past the
@@ -1998,6 +2074,69 @@ bool pipe_ok(int dtype, const GemmArgs& g, int R) {
   }
   if (dtype != kF32 || KIND == kDownDgrad) return false;
   return (int64_t)((R + pipe::BM - 1) / pipe::BM) * ((g.Ndim + BNH - 1) / BNH) >= cu_count();
+}
+
+// Slices of a row-grouped launch (the down projection's forward, the gate/up data
+// gradient).  Their output is D wide and their reduction M or 2M long, so a narrow
+// layer with a long hidden size has few tiles, each a long serial chain, and most
+// CUs idle.  The slice count minimises an estimate of the launch for evenly filled
+// experts: the longest CU's tiles, or the launch's whole work (with `extra_us` of
+// work that other blocks of it do) shared by all CUs if that is more, plus the
+// pass over the fp32 partials.  Measured per k-tile 1.7 us (bf16; 1.1 thin) and 7
+// us (fp32; 1.9 thin), per block 8 us, partials at 4 TB/s; fp32 on the generic
+// kernel 2.4 us per k-tile up to a 128 x 128 tile per CU, 4.2 up to two.  1:
+// unsliced.  Measured (us, unsliced -> sliced): bf16 E 64 D 256 M 11200, 366
+// tokens top-8, down forward 269 -> 115, gate/up backward 787 -> 611; E 8 D 448 M
+// 13632, 1027 tokens top-2, 114 -> 57 and 640 -> 223; fp32 E 4 D 1472 M 2496, 273
+// tokens top-2, 189 -> 97 and 543 -> 331.
+template <typename T, int KIND>
+int row_slices(const GemmArgs& g, int64_t R, double extra_us) {
+  static_assert(KIND == kDownFwd || KIND == kGateUpDgrad, "plain-store row kinds");
+  constexpr bool kF = sizeof(T) == 4;
+  const double cus = cu_count(), per_block = 8.0, per_k = kF ? 7.0 : 1.7, per_k_thin = kF ? 1.9 : 1.1;
+  const int64_t E = std::min<int64_t>(g.E, R), r = (R + E - 1) / E;
+  const int64_t nt = (g.Ndim + pipe::BN - 1) / pipe::BN, nt_thin = (g.Ndim + pipe::kThinN<T> - 1) / pipe::kThinN<T>;
+  // an expert of r rows: rounded full tiles, and in half of the cases a thin one beside them
+  const double full = r <= pipe::THIN ? 0.0 : (double)(E * std::max<int64_t>(1, (r + 128) / 256) * nt);
+  const double thin = (double)(E * nt_thin) * (r <= pipe::THIN ? 1.0 : 0.5);
+  const int64_t kt = (KindTraits<KIND>::DUAL_K ? 2 : 1) * (((int64_t)g.Kdim + pipe::kBKT<T> - 1) / pipe::kBKT<T>);
+  const auto rounds = [&](double blocks) { return std::max(1.0, std::ceil(blocks / cus)); };
+  int best = 1;
+  double best_us = 0.0;
+  for (int s = 1; s <= 16 && (s == 1 || kt / s >= 4); ++s) {
+    const double k = (double)((kt + s - 1) / s), b_full = k * per_k + per_block, b_thin = k * per_k_thin + per_block;
+    const double chain = full > 0.0 ? rounds(full * s) * b_full : rounds(thin * s) * b_thin;
+    const double share = (full * s * b_full + thin * s * b_thin + extra_us) / cus;
+    double us = std::max(chain, share) + (s > 1 ? 6.0 + (double)s * (double)R * g.Ndim * 8.0 / 4e6 : 0.0);
+    if (kF && s == 1 && !pipe_ok<KIND>(kF32, g, (int)R)) {
+      const double tiles = (double)((E + R / 128) * ((g.Ndim + 127) / 128));
+      us = (double)kt * (tiles <= cus ? 2.4 : 4.2 * std::max(1.0, tiles / (2.0 * cus)));
+    }
+    if (s == 1 || us < (best == 1 ? 0.93 : 0.97) * best_us) {
+      best = s;
+      best_us = us;
+    }
+  }
+  return best;
+}
+
+inline int64_t slices_ws_bytes(int slices, int64_t R, int64_t N) { return slices > 1 ? slices * R * N * 4 : 0; }
+
+template <typename T>
+int launch_rows_reduce(const float* ws, int64_t R, int64_t N, int slices, void* out, hipStream_t s, const char* name) {
+  const int64_t n = R * N;
+  hipLaunchKernelGGL(pipe::rows_reduce_kernel<T>, dim3((unsigned)((n / 4 + 255) / 256)), dim3(256), 0, s, ws, n, slices,
+                     (T*)out);
+  ABACUS_CHECK_LAUNCH(name);
+  return 0;
+}
+
+// A data gradient (KA, row-grouped: the long tiles, then its thin ones) and a
+// weight gradient (KB) in one launch.
+template <int KA, int KB>
+int launch_pipe_pair(const GemmArgs& a, int Ra, const GemmArgs& b, int Rb, hipStream_t s, const char* name) {
+  (void)Rb;
+  return launch_rows<uint16_t, KA, KB>(a, Ra, &b, -1, thin_tiles_pay<uint16_t>(Ra, a.E), s, name);
 }
 
 template <int KIND>
@@ -2231,15 +2370,32 @@ static bool down_fwd_split(int64_t R, int64_t M, int64_t E) {
   return !down_fwd_thin(R, E) && M >= kSplitMinReduction;
 }
 
+static int down_fwd_slices(int dtype, const GemmArgs& g, int64_t R) {
+  return dtype == kBF16 ? row_slices<uint16_t, kDownFwd>(g, R, 0.0) : row_slices<float, kDownFwd>(g, R, 0.0);
+}
+
 int64_t abacus_moe_down_fwd_ws_bytes(int64_t R, int64_t M, int64_t D, int64_t E, int dtype) {
   if (check_gemm_shape(R, D, M, E, dtype) || R == 0) return 0;
   const GemmArgs g = args_down_fwd(nullptr, nullptr, nullptr, R, M, D, E, nullptr);
+  const int slices = D % 8 == 0 ? down_fwd_slices(dtype, g, R) : 1;
+  if (slices > 1) return slices_ws_bytes(slices, R, D);
   if (!pipe_ok<kDownFwd>(dtype, g, (int)R) || !down_fwd_split(R, M, E)) return 0;  // no split tail
   return plan_split<kDownFwd>(g, (int)R).ws_bytes();
 }
 
-static int run_down_fwd(int dtype, const GemmArgs& g, int64_t R, int64_t M, int64_t E, void* ws, int64_t ws_bytes,
+static int run_down_fwd(int dtype, GemmArgs g, int64_t R, int64_t M, int64_t E, void* ws, int64_t ws_bytes,
                         hipStream_t s) {
+  const int slices = g.Ndim % 8 == 0 ? down_fwd_slices(dtype, g, R) : 1;
+  if (slices > 1 && ws != nullptr && ws_bytes >= slices_ws_bytes(slices, R, g.Ndim)) {
+    g.ksplit = slices;
+    g.ksplit_ws = (float*)ws;
+    if (dtype == kBF16
+            ? launch_rows<uint16_t, kDownFwd, -1>(g, (int)R, nullptr, -1, true, s, "down_fwd")
+            : launch_rows<float, kDownFwd, -1>(g, (int)R, nullptr, -1, true, s, "down_fwd"))
+      return 1;
+    return dtype == kBF16 ? launch_rows_reduce<uint16_t>((const float*)ws, R, g.Ndim, slices, g.c0, s, "down_fwd")
+                          : launch_rows_reduce<float>((const float*)ws, R, g.Ndim, slices, g.c0, s, "down_fwd");
+  }
   if (pipe_ok<kDownFwd>(dtype, g, (int)R)) {
     if (down_fwd_thin(R, E))
       return dtype == kBF16 ? launch_rows<uint16_t, kDownFwd, -1>(g, (int)R, nullptr, -1, true, s, "down_fwd")
@@ -2377,20 +2533,49 @@ int abacus_experts_down_bwd(const void* dy_RD, const void* w_down_EMD, const voi
                                                "experts_down_bwd", "experts_down_bwd");
 }
 
-int abacus_experts_gateup_bwd(const void* dgate, const void* dup, const void* w_gate_pad, const void* w_up_pad,
+// The data gradient's slices; the weight gradient's tiles beside it (bf16) count
+// as work that fills the CUs it leaves idle.
+static int gateup_bwd_slices(int dtype, const GemmArgs& gd, int64_t R, int64_t D, int64_t ld, int64_t E) {
+  if (D % 8 != 0 || R == 0) return 1;
+  if (dtype == kF32) return row_slices<float, kGateUpDgrad>(gd, R, 0.0);
+  const double tiles = (double)E * (double)((D + 255) / 256) * (double)((ld + 127) / 128);
+  return row_slices<uint16_t, kGateUpDgrad>(gd, R, tiles * (8.0 + 1.9 * (double)R / (double)E / 64.0));
+}
+
+int64_t abacus_experts_gateup_bwd_ws_bytes(int64_t R, int64_t D, int64_t M, int64_t E, int dtype) {
+  if (check_gemm_shape(R, D, M, E, dtype)) return 0;
+  const GemmArgs gd = args_gateup_dgrad(nullptr, nullptr, nullptr, nullptr, nullptr, R, D, M, E, nullptr);
+  return slices_ws_bytes(gateup_bwd_slices(dtype, gd, R, D, M, E), R, D);
+}
+
+int abacus_experts_gateup_bwd(const void* dgate, const void* dup, const void* w_gate, const void* w_up,
                               const void* x_perm_RD, const int32_t* offsets_E1, int64_t R, int64_t D, int64_t M,
-                              int64_t ld, int64_t E, void* dx_perm_RD, void* dw_gate_EDM, void* dw_up_EDM,
-                              int32_t* tile_ctr, void* stream) {
-  if (check_hidden(R, D, M, ld, E)) return 1;
+                              int64_t ld, int64_t E, int dtype, void* dx_perm_RD, void* dw_gate_EDM, void* dw_up_EDM,
+                              int32_t* tile_ctr, void* ws, int64_t ws_bytes, void* stream) {
+  if (dtype == kF32 ? check_gemm_shape(R, D, M, E, dtype) : check_hidden(R, D, M, ld, E)) return 1;
+  ABACUS_CHECK_ARG(dtype != kF32 || ld == M, "fp32: ld %lld must be hidden_dim %lld", (long long)ld, (long long)M);
   ABACUS_CHECK_ARG(tile_ctr != nullptr, "tile_ctr workspace is NULL");
-  const GemmArgs gd = args_gateup_dgrad(dgate, dup, w_gate_pad, w_up_pad, offsets_E1, R, D, ld, E, dx_perm_RD);
+  const hipStream_t s = (hipStream_t)stream;
+  GemmArgs gd = args_gateup_dgrad(dgate, dup, w_gate, w_up, offsets_E1, R, D, ld, E, dx_perm_RD);
   GemmArgs gw = args_gateup_wgrad(x_perm_RD, dgate, dup, offsets_E1, D, ld, E, dw_gate_EDM, dw_up_EDM);
   gw.ldc = M;
   gw.c_estride = D * M;
-  gw.c_cols = (int)M;
+  gw.c_cols = ld == M ? 0 : (int)M;
   gw.tile_ctr = tile_ctr;
-  return dispatch_pair<kGateUpDgrad, kGateUpWgrad>(kBF16, gd, gw, (int)R, (hipStream_t)stream, "experts_gateup_bwd",
-                                                   "experts_gateup_bwd", "experts_gateup_bwd");
+  const char* name = "experts_gateup_bwd";
+  const int slices = gateup_bwd_slices(dtype, gd, R, D, ld, E);
+  if (slices > 1 && ws != nullptr && ws_bytes >= slices_ws_bytes(slices, R, D)) {
+    gd.ksplit = slices;
+    gd.ksplit_ws = (float*)ws;
+    if (dtype == kBF16) {
+      if (launch_rows<uint16_t, kGateUpDgrad, kGateUpWgrad>(gd, (int)R, &gw, -1, true, s, name)) return 1;
+      return launch_rows_reduce<uint16_t>(gd.ksplit_ws, R, D, slices, dx_perm_RD, s, name);
+    }
+    if (launch_rows<float, kGateUpDgrad, -1>(gd, (int)R, nullptr, -1, true, s, name)) return 1;
+    if (launch_rows_reduce<float>(gd.ksplit_ws, R, D, slices, dx_perm_RD, s, name)) return 1;
+    return dispatch_gemm<kGateUpWgrad>(dtype, gw, (int)R, s, name);
+  }
+  return dispatch_pair<kGateUpDgrad, kGateUpWgrad>(dtype, gd, gw, (int)R, s, name, name, name);
 }
 
 }  // extern "C"

@@ -247,23 +247,14 @@ class _MoEFunction(torch.autograd.Function):
         ld = gate.shape[1]
         dgate = torch.empty(R, ld, dtype=x_TD.dtype, device=dev)
         dup = torch.empty(R, ld, dtype=x_TD.dtype, device=dev)
-        if ld != M:  # w_gate and w_up are the forward's padded copies
+        dw_down = None
+        if ld != M:
             dw_down = torch.empty_like(w_down)
-            dw_gate, dw_up = (torch.empty(E, D, M, dtype=x_TD.dtype, device=dev) for _ in range(2))
-            dxp = torch.empty(R, D, dtype=x_TD.dtype, device=dev)
             call(
                 "abacus_experts_down_bwd", ptr(dy), ptr(w_down), ptr(gate), ptr(up), ptr(h), ptr(offsets), R, M, ld, D, E,
                 ptr(dgate), ptr(dup), ptr(dw_down), ptr(_lib.tile_ctr(dev)), s,
             )
-            call(
-                "abacus_experts_gateup_bwd", ptr(dgate), ptr(dup), ptr(w_gate), ptr(w_up), ptr(xp), ptr(offsets), R, D, M,
-                ld, E, ptr(dxp), ptr(dw_gate), ptr(dw_up), ptr(_lib.tile_ctr(dev)), s,
-            )
-            dx, dw_DE = _router_dgrad_wgrad(needs[0], needs[1], x_TD, w_DE, dlogit, idx32, pos, dxp, wt)
-            return (dx, dw_DE, dw_gate if needs[2] else None, dw_up if needs[3] else None,
-                    dw_down if needs[4] else None, None, None, None, None, None, None)
-        dw_down = None
-        if needs[4]:
+        elif needs[4]:
             dw_down = torch.empty_like(w_down)
             call(
                 "abacus_moe_down_bwd", ptr(dy), ptr(w_down), ptr(gate), ptr(up), ptr(h), ptr(offsets), R, M, D, E,
@@ -274,12 +265,19 @@ class _MoEFunction(torch.autograd.Function):
                 "abacus_moe_down_bwd_dgrad", ptr(dy), ptr(w_down), ptr(gate), ptr(up), ptr(offsets), R, M, D, E, dt,
                 ptr(dgate), ptr(dup), s,
             )
-        dxp = torch.empty(R, D, dtype=x_TD.dtype, device=dev) if needs[0] else None
+        dxp = torch.empty(R, D, dtype=x_TD.dtype, device=dev) if needs[0] or ld != M else None
         dw_gate = dw_up = None
-        if needs[2] or needs[3]:
-            dw_gate = torch.empty_like(w_gate)
-            dw_up = torch.empty_like(w_up)
-        if dxp is not None and dw_gate is not None:
+        if needs[2] or needs[3] or ld != M:
+            dw_gate, dw_up = (torch.empty(E, D, M, dtype=x_TD.dtype, device=dev) for _ in range(2))
+        both = dxp is not None and dw_gate is not None
+        ws_bytes = query("abacus_experts_gateup_bwd_ws_bytes", R, D, ld, E, dt) if both and x_TD.is_cuda else 0
+        if ws_bytes > 0 or ld != M:  # (ld != M: w_gate and w_up are the forward's padded copies)
+            ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes > 0 else None
+            call(
+                "abacus_experts_gateup_bwd", ptr(dgate), ptr(dup), ptr(w_gate), ptr(w_up), ptr(xp), ptr(offsets), R, D, M,
+                ld, E, dt, ptr(dxp), ptr(dw_gate), ptr(dw_up), ptr(_lib.tile_ctr(dev)), ptr(ws), ws_bytes, s,
+            )
+        elif both:
             call(
                 "abacus_moe_gateup_bwd", ptr(dgate), ptr(dup), ptr(w_gate), ptr(w_up), ptr(xp), ptr(offsets),
                 R, D, M, E, dt, ptr(dxp), ptr(dw_gate), ptr(dw_up), ptr(_lib.tile_ctr(dev)), s,
@@ -295,7 +293,7 @@ class _MoEFunction(torch.autograd.Function):
                 ptr(dw_gate), ptr(dw_up), ptr(_lib.tile_ctr(dev)), s,
             )
         dx, dw_DE = _router_dgrad_wgrad(needs[0], needs[1], x_TD, w_DE, dlogit, idx32, pos, dxp, wt)
-        return (dx, dw_DE, dw_gate if needs[2] else None, dw_up if needs[3] else None, dw_down,
+        return (dx, dw_DE, dw_gate if needs[2] else None, dw_up if needs[3] else None, dw_down if needs[4] else None,
                 None, None, None, None, None, None)
 
 

@@ -66,8 +66,8 @@ int64_t abacus_moe_router_ws_bytes(int64_t D, int64_t E, int dtype);
 /* bytes of the fp32 partial-sum scratch used by router_wgrad for this dtype
  * (-1 for an unknown dtype). */
 int64_t abacus_moe_router_wgrad_ws_bytes(int64_t T, int64_t D, int64_t E, int dtype);
-/* bytes of the split-tail workspace of down_fwd (0: that shape runs no split, which
- * includes small batches, R <= 128 * E, and short reductions, M < 2560). */
+/* bytes of the workspace of down_fwd: the slices of a launch with too few tiles for
+ * the GPU, else the split tail's (0: that shape runs neither). */
 int64_t abacus_moe_down_fwd_ws_bytes(int64_t R, int64_t M, int64_t D, int64_t E, int dtype);
 /* bytes of the per-block partial sums and counts used by load_balancing_fwd. */
 int64_t abacus_moe_load_balancing_ws_bytes(int64_t T, int64_t E);
@@ -147,17 +147,23 @@ int abacus_experts_decode_fwd(const void* x_perm_RD, const void* w_gate_EDM, con
  * w_up (E*D rows of M) into rows of ld, which abacus_moe_gateup_fwd takes as a
  * hidden size of ld; w_down, and every weight gradient, keep rows and columns of
  * M.  Otherwise as abacus_moe_down_fwd (workspace of abacus_moe_down_fwd_ws_bytes
- * for ld), abacus_moe_down_bwd and abacus_moe_gateup_bwd. */
+ * for ld) and abacus_moe_down_bwd. */
 int abacus_experts_pad_columns(const void* src, int64_t rows, int64_t M, int64_t ld, void* dst, void* stream);
 int abacus_experts_down_fwd(const void* h, const void* w_down_EMD, const int32_t* offsets_E1, int64_t R, int64_t M,
                             int64_t ld, int64_t D, int64_t E, void* y_RD, void* ws, int64_t ws_bytes, void* stream);
 int abacus_experts_down_bwd(const void* dy_RD, const void* w_down_EMD, const void* gate, const void* up, const void* h,
                             const int32_t* offsets_E1, int64_t R, int64_t M, int64_t ld, int64_t D, int64_t E,
                             void* dgate, void* dup, void* dw_down_EMD, int32_t* tile_ctr, void* stream);
-int abacus_experts_gateup_bwd(const void* dgate, const void* dup, const void* w_gate_pad, const void* w_up_pad,
+
+/* abacus_moe_gateup_bwd for any hidden size (bf16; w_gate and w_up with rows of
+ * ld; fp32: ld = M), with a workspace of abacus_experts_gateup_bwd_ws_bytes bytes
+ * (for a hidden size of ld; 0: no use for one) that lets the data gradient run as
+ * slices of its reduction where its tiles are too few for the GPU. */
+int64_t abacus_experts_gateup_bwd_ws_bytes(int64_t R, int64_t D, int64_t M, int64_t E, int dtype);
+int abacus_experts_gateup_bwd(const void* dgate, const void* dup, const void* w_gate, const void* w_up,
                               const void* x_perm_RD, const int32_t* offsets_E1, int64_t R, int64_t D, int64_t M,
-                              int64_t ld, int64_t E, void* dx_perm_RD, void* dw_gate_EDM, void* dw_up_EDM,
-                              int32_t* tile_ctr, void* stream);
+                              int64_t ld, int64_t E, int dtype, void* dx_perm_RD, void* dw_gate_EDM, void* dw_up_EDM,
+                              int32_t* tile_ctr, void* ws, int64_t ws_bytes, void* stream);
 
 /* Replaces moe.py:81-85: out[t] = sum over the token's experts (ascending)
  * of y[pos(t,k)] * weights_TK[t,k]. */

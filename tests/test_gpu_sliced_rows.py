@@ -1,0 +1,75 @@
+"""Launches whose tiles are too few for the GPU run as slices of the reduction (down forward, gate/up data gradient):
+the same products against fp64, repeatable bit for bit, with the weight gradients beside them unchanged."""
+
+import itertools
+
+import pytest
+import torch
+
+from abacus_amd import _lib
+
+pytestmark = pytest.mark.gpu
+
+call, ptr = _lib.call, _lib.ptr
+
+
+@pytest.mark.parametrize("dtype,counts,D,M", [
+    (torch.bfloat16, [300, 0, 129, 70, 1], 200, 6008),   # full and thin tiles, an empty expert, a ragged last k-tile
+    (torch.bfloat16, [5, 0, 33], 64, 4096),              # thin tiles only
+    (torch.bfloat16, [130, 257], 264, 2731),             # a hidden size off the vector (slices cross the gate/up halves)
+    (torch.float32, [300, 0, 129, 70, 1], 200, 2808),
+    (torch.float32, [260, 256], 1024, 1408),
+], ids=["full_thin", "thin", "odd", "fp32", "fp32_dense"])
+def test_sliced_products_match_fp64(dtype, counts, D, M):
+    dev = torch.device("cuda")
+    gen = torch.Generator(device=dev).manual_seed(51)
+    E, R = len(counts), sum(counts)
+    offs = [0] + list(itertools.accumulate(counts))
+    offsets = torch.tensor(offs, dtype=torch.int32, device=dev)
+    dt, s = _lib.dtype_code(dtype), _lib.stream_of(dev)
+    vec = 8 if dtype == torch.bfloat16 else 4
+    ld = -(-M // vec) * vec
+
+    def rn(*shape, scale=1.0):
+        return (torch.randn(*shape, device=dev, generator=gen) * scale).to(dtype)
+
+    def pitched(t):  # rows of ld, zero past M
+        return torch.nn.functional.pad(t, (0, ld - M)).contiguous()
+
+    xp, h, dg, du = rn(R, D), pitched(rn(R, M)), pitched(rn(R, M)), pitched(rn(R, M))
+    wg, wu, wd = rn(E, D, M, scale=0.05), rn(E, D, M, scale=0.05), rn(E, M, D, scale=0.05)
+    wgp, wup = pitched(wg), pitched(wu)
+    outs = []
+    for _ in range(2):
+        nan = lambda *shape: torch.full(shape, float("nan"), dtype=dtype, device=dev)
+        y, dx, dwg, dwu = nan(R, D), nan(R, D), nan(E, D, M), nan(E, D, M)
+        n1 = _lib.query("abacus_moe_down_fwd_ws_bytes", R, ld, D, E, dt)
+        n2 = _lib.query("abacus_experts_gateup_bwd_ws_bytes", R, D, ld, E, dt)
+        assert n1 >= 2 * R * D * 4 and n2 >= 2 * R * D * 4, "these shapes are meant to run sliced"
+        ws = torch.full((max(n1, n2) // 4,), float("nan"), device=dev)
+        if ld != M:
+            call("abacus_experts_down_fwd", ptr(h), ptr(wd), ptr(offsets), R, M, ld, D, E, ptr(y), ptr(ws), n1, s)
+        else:
+            call("abacus_moe_down_fwd", ptr(h), ptr(wd), ptr(offsets), R, M, D, E, dt, ptr(y), ptr(ws), n1, s)
+        call("abacus_experts_gateup_bwd", ptr(dg), ptr(du), ptr(wgp), ptr(wup), ptr(xp), ptr(offsets), R, D, M, ld, E, dt,
+             ptr(dx), ptr(dwg), ptr(dwu), ptr(_lib.tile_ctr(dev)), ptr(ws), n2, s)
+        torch.cuda.synchronize()
+        outs.append((y, dx, dwg, dwu))
+    for a, b in zip(*outs):
+        assert torch.equal(a, b) and not torch.isnan(a).any()
+    y, dx, dwg, dwu = outs[0]
+    # one rounding to bf16 (2^-9); fp32 sums of at most 5616 terms: sqrt(n) 2^-24 of their norm
+    tol = 4e-3 if dtype == torch.bfloat16 else 1e-5
+    for e in range(E):
+        a, b = offs[e], offs[e + 1]
+        if a == b:
+            continue
+        d = lambda t: t[a:b].double()
+        for name, got, want in (
+            ("y", y[a:b], d(h)[:, :M] @ wd[e].double()),
+            ("dx", dx[a:b], d(dg)[:, :M] @ wg[e].double().t() + d(du)[:, :M] @ wu[e].double().t()),
+            ("dwg", dwg[e], d(xp).t() @ d(dg)[:, :M]),
+            ("dwu", dwu[e], d(xp).t() @ d(du)[:, :M]),
+        ):
+            err = float((got.double() - want).norm() / want.norm())
+            assert err < tol, f"{name} expert {e}: {err:.3g}"
