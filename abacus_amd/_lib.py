@@ -62,6 +62,9 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "abacus_moe_router_wgrad_noalloc": (_I, [_P, _P, _P, _I64, _I64, _I64, _I64, _I, _P, _P]),
     "abacus_experts_decode_ws_bytes": (_I64, [_I64, _I64, _I64, _I64, _I]),
     "abacus_experts_decode_fwd": (_I, [_P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _I, _I64, _P, _P, _P, _I64, _P]),
+    "abacus_layer_plan_fields": (_I64, []),
+    "abacus_layer_fwd": (_I, [_P, _P, _P, _P, _P, _P, _P, _D, _D, _I, _P, _P, _P, _P, _P]),
+    "abacus_layer_bwd": (_I, [_P, _P, _P, _P, _P, _P, _D, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P]),
     "abacus_experts_pad_columns": (_I, [_P, _I64, _I64, _I64, _P, _P]),
     "abacus_experts_down_fwd": (_I, [_P, _P, _P, _I64, _I64, _I64, _I64, _I64, _P, _P, _I64, _P]),
     "abacus_experts_down_bwd": (_I, [_P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _P, _P, _P, _P, _P]),
@@ -187,6 +190,12 @@ class KernelTimer:
 _timer: KernelTimer | None = None
 
 
+def timing() -> bool:
+    """Whether a KernelTimer is active: callers that can run several entry points in one call then make
+    them one by one, so that each is timed under its name."""
+    return _timer is not None
+
+
 def call(name: str, *args) -> None:
     """Call an entry point that returns a status code; raise on failure.
 
@@ -262,4 +271,5 @@ def stream_of(device: torch.device):
     """The stream argument for a call on `device`'s tensors: torch's current HIP stream, or HOST."""
     if device.type == "cpu":
         return HOST
-    return torch.cuda.current_stream(device).cuda_stream
+    index = device.index if device.index is not None else torch.cuda.current_device()
+    return torch._C._cuda_getCurrentRawStream(index)  # current_stream(device).cuda_stream without the Stream object

@@ -12,7 +12,9 @@ R = T*K routed rows.
 
 from __future__ import annotations
 
+import ctypes
 import dataclasses
+import functools
 
 import torch
 import torch.distributed as dist
@@ -44,6 +46,156 @@ class Routing:
     offsets_E1: torch.Tensor | None = None
     perm_R: torch.Tensor | None = None
     pos_TK: torch.Tensor | None = None
+
+
+class _PlanRouting(Routing):
+    """A Routing whose tensors are views of the layer's route buffer, made when they are asked for."""
+
+    def __init__(self, route: torch.Tensor, plan: "_LayerPlan", dtype: torch.dtype):
+        self._route, self._at, self._sizes, self._dtype = route, plan.at, plan.sizes, dtype
+
+    def _view(self, name: str, dtype: torch.dtype, *shape: int) -> torch.Tensor:
+        n, a = dtype.itemsize, self._at[name]
+        for d in shape:
+            n *= d
+        return self._route[a:a + n].view(dtype).view(shape)
+
+    @functools.cached_property
+    def logits_TE(self):
+        return self._view("logits", self._dtype, self._sizes[0], self._sizes[2])
+
+    @functools.cached_property
+    def weights_TK(self):
+        return self._view("weights", self._dtype, self._sizes[0], self._sizes[3])
+
+    @functools.cached_property
+    def indices_TK(self):
+        return self._view("indices", torch.int64, self._sizes[0], self._sizes[3])
+
+    @functools.cached_property
+    def counts_E(self):
+        return self._view("counts", torch.int32, self._sizes[2])
+
+    @functools.cached_property
+    def offsets_E1(self):
+        return self._view("offsets", torch.int32, self._sizes[2] + 1)
+
+    @functools.cached_property
+    def perm_R(self):
+        return self._view("perm", torch.int32, self._sizes[0] * self._sizes[3])
+
+    @functools.cached_property
+    def pos_TK(self):
+        return self._view("pos", torch.int32, self._sizes[0], self._sizes[3])
+
+
+# LayerPlan of csrc/layer.hip, field by field.
+_PLAN_FIELDS = ("T", "D", "E", "K", "M", "ld", "dtype", "decode",
+                "logits", "weights", "indices", "counts", "offsets", "pos", "perm",
+                "idx", "score", "wt", "gate_pad", "up_pad", "xp", "gate", "up", "h", "y",
+                "hist", "base", "ws", "ws_bytes",
+                "dy", "dlogit", "dgate", "dup", "dxp", "ctr", "bws", "bws_bytes", "partial")
+
+
+@dataclasses.dataclass(frozen=True)
+class _LayerPlan:
+    """Where one layer call keeps what: byte offsets in its buffers, and their sizes."""
+
+    sizes: tuple[int, int, int, int]  # T, D, E, K
+    at: dict[str, int]
+    fields: ctypes.Array  # the LayerPlan of csrc/layer.hip
+    route_bytes: int
+    keep_bytes: int
+    scratch_bytes: int
+    bwd_bytes: int
+
+
+@functools.lru_cache(maxsize=512)
+def _layer_plan(T: int, D: int, E: int, K: int, M: int, dt: int, need_grad: bool) -> _LayerPlan:
+    """The buffers of the GPU layer for these sizes (and nothing else: no tensor enters)."""
+    R, s = T * K, 2 if dt == _lib.BF16 else 4
+    vec = 16 // s
+    decode_ws = -1 if need_grad else query("abacus_experts_decode_ws_bytes", R, D, M, E, dt)
+    ld = -(-M // vec) * vec
+    if decode_ws < 0 and dt != _lib.BF16:
+        ld = M
+    at = dict(T=T, D=D, E=E, K=K, M=M, ld=ld, dtype=dt, decode=int(decode_ws >= 0))
+
+    def lay(**sizes: int) -> int:
+        end = 0
+        for name, nbytes in sizes.items():
+            if nbytes < 0:
+                at[name] = -1
+                continue
+            at[name] = end
+            end += (nbytes + 255) // 256 * 256  # each buffer 256-byte aligned
+        return max(end, 256)
+
+    rows, hidden = R * D * s, R * ld * s
+    pad = E * D * ld * s if decode_ws < 0 and ld != M else -1
+    ws = decode_ws if decode_ws >= 0 else query("abacus_moe_down_fwd_ws_bytes", R, ld, D, E, dt)
+    hist = query("abacus_moe_hist_len", T, E) * 4
+    route_bytes = lay(logits=T * E * s, weights=R * s, indices=R * 8, counts=E * 4, offsets=(E + 1) * 4, pos=R * 4,
+                      perm=R * 4)
+    keep_bytes = lay(idx=R * 4, score=R * 4, wt=query("abacus_moe_router_ws_bytes", D, E, dt), gate_pad=pad, up_pad=pad,
+                     xp=rows, gate=hidden if need_grad else -1, up=hidden if need_grad else -1, h=hidden, y=rows)
+    scratch_bytes = lay(hist=hist, base=hist, ws=ws if ws > 0 else -1)
+    at["ws_bytes"] = max(ws, 0)
+    bws = query("abacus_experts_gateup_bwd_ws_bytes", R, D, ld, E, dt) if need_grad else 0
+    bwd_bytes = lay(dy=rows, dlogit=R * 4, dgate=hidden, dup=hidden, dxp=rows, ctr=_lib.TILE_CTR_INTS * 4,
+                    bws=bws if bws > 0 else -1,
+                    partial=query("abacus_moe_router_wgrad_ws_bytes", T, D, E, dt))
+    at["bws_bytes"] = bws
+    assert query("abacus_layer_plan_fields") == len(_PLAN_FIELDS)
+    fields = (ctypes.c_int64 * len(_PLAN_FIELDS))(*[at[f] for f in _PLAN_FIELDS])
+    return _LayerPlan((T, D, E, K), at, fields, route_bytes, keep_bytes, scratch_bytes, bwd_bytes)
+
+
+def _layer_forward(ctx, x_TD, w_DE, w_gate, w_up, w_down, bias_E, top_k, route_scale, bias_speed, need_grad, record):
+    """_MoEFunction.forward on the GPU: every kernel from one call (abacus_layer_fwd)."""
+    T, D = x_TD.shape
+    E, _, M = w_gate.shape
+    dev = x_TD.device
+    plan = _layer_plan(T, D, E, top_k, M, _lib.dtype_code(x_TD.dtype), need_grad)
+    route = torch.empty(plan.route_bytes, dtype=torch.uint8, device=dev)
+    keep = torch.empty(plan.keep_bytes, dtype=torch.uint8, device=dev)
+    scratch = torch.empty(plan.scratch_bytes, dtype=torch.uint8, device=dev)
+    out = torch.empty_like(x_TD)
+    update = bias_speed is not None and bias_speed != 0
+    call(
+        "abacus_layer_fwd", plan.fields, ptr(x_TD), ptr(w_DE), ptr(w_gate), ptr(w_up), ptr(w_down), ptr(bias_E),
+        route_scale, bias_speed if update else 0.0, int(update), route.data_ptr(), keep.data_ptr(), scratch.data_ptr(),
+        out.data_ptr(), _lib.stream_of(dev),
+    )
+    if need_grad:
+        ctx.save_for_backward(x_TD, w_DE, w_gate, w_up, w_down, route, keep)
+        ctx.plan = plan
+    ctx.route_scale = float(route_scale)
+    if record is not None:
+        record["routing"] = _PlanRouting(route, plan, x_TD.dtype)
+    return out
+
+
+def _layer_backward(ctx, dout):
+    """_MoEFunction.backward after _layer_forward: every kernel from one call (abacus_layer_bwd)."""
+    x_TD, w_DE, w_gate, w_up, w_down, route, keep = ctx.saved_tensors
+    plan, needs, dev = ctx.plan, ctx.needs_input_grad, x_TD.device
+    dout = _contig(dout.to(x_TD.dtype))
+    pitched = plan.at["ld"] != plan.at["M"]
+    scratch = torch.empty(plan.bwd_bytes, dtype=torch.uint8, device=dev)
+    dx = torch.empty_like(x_TD) if needs[0] else None
+    dw_DE = torch.empty_like(w_DE) if needs[1] else None
+    dw_gate = dw_up = None
+    if needs[2] or needs[3] or pitched:
+        dw_gate, dw_up = torch.empty_like(w_gate), torch.empty_like(w_up)
+    dw_down = torch.empty_like(w_down) if needs[4] or pitched else None
+    call(
+        "abacus_layer_bwd", plan.fields, ptr(x_TD), ptr(w_DE), ptr(w_gate), ptr(w_up), ptr(w_down), ctx.route_scale,
+        route.data_ptr(), keep.data_ptr(), ptr(dout), scratch.data_ptr(), ptr(dx), ptr(dw_DE), ptr(dw_gate), ptr(dw_up),
+        ptr(dw_down), _lib.stream_of(dev),
+    )
+    return (dx, dw_DE, dw_gate if needs[2] else None, dw_up if needs[3] else None, dw_down if needs[4] else None,
+            None, None, None, None, None, None)
 
 
 def _check_device(x: torch.Tensor, what: str) -> None:
@@ -161,10 +313,17 @@ def _decode_ws_bytes(x_TD: torch.Tensor, R: int, M: int, E: int) -> int:
 
 
 class _MoEFunction(torch.autograd.Function):
-    """MoE.forward (moe.py:60-86) fused: router -> dispatch -> grouped SwiGLU -> combine."""
+    """MoE.forward (moe.py:60-86) fused: router -> dispatch -> grouped SwiGLU -> combine.
+
+    On the GPU one call runs all kernels of a direction; on the CPU, and while a KernelTimer
+    wants each entry point by its name, they are called one by one."""
 
     @staticmethod
     def forward(ctx, x_TD, w_DE, w_gate, w_up, w_down, bias_E, top_k, route_scale, bias_speed, need_grad, record):
+        ctx.plan = None
+        if x_TD.is_cuda and not _lib.timing():
+            return _layer_forward(ctx, x_TD, w_DE, w_gate, w_up, w_down, bias_E, top_k, route_scale, bias_speed,
+                                  need_grad, record)
         T, D = x_TD.shape
         E, _, M = w_gate.shape
         K = top_k
@@ -226,6 +385,8 @@ class _MoEFunction(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, dout):
+        if ctx.plan is not None:
+            return _layer_backward(ctx, dout)
         (x_TD, w_DE, w_gate, w_up, w_down, xp, gate, up, h, y, weights, score, idx32, pos,
          offsets, wt) = ctx.saved_tensors
         T, D = x_TD.shape

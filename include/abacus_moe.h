@@ -342,6 +342,21 @@ int abacus_attention_any_bwd(const void* q_BLHK, const void* k_BLHK, const void*
                              float scale, int dtype, void* dq_BLHK, void* dk_BLHK, void* dv_BLHK, float* ws,
                              int64_t ws_bytes, void* stream);
 
+/* The MoE layer as one call per direction (GPU only): the entry points above in
+ * the order of moe.py:60-86 and its autograd.  plan: abacus_layer_plan_fields()
+ * int64 values (sizes, and byte offsets of every buffer in route, keep and scratch;
+ * abacus_amd/moe.py lays them out).  Null gradients are not computed (dw_gate_EDM
+ * and dw_up_EDM come together). */
+int64_t abacus_layer_plan_fields(void);
+int abacus_layer_fwd(const int64_t* plan, const void* x_TD, const void* w_DE, const void* w_gate_EDM,
+                     const void* w_up_EDM, const void* w_down_EMD, void* bias_E, double route_scale,
+                     double bias_update_speed, int update_bias, void* route, void* keep, void* scratch, void* out_TD,
+                     void* stream);
+int abacus_layer_bwd(const int64_t* plan, const void* x_TD, const void* w_DE, const void* w_gate_EDM,
+                     const void* w_up_EDM, const void* w_down_EMD, double route_scale, const void* route,
+                     const void* keep, const void* dout_TD, void* scratch, void* dx_TD, void* dw_DE,
+                     void* dw_gate_EDM, void* dw_up_EDM, void* dw_down_EMD, void* stream);
+
 /* Cross-entropy of the decoder's logits (kernels/liger.py:12-47, called at
  * trainer.py:81-85), forward: for the N rows of logits_NV ((N, V), `dtype`)
  * with int64 targets_N, lse_N[i] = log(sum_j exp(x_ij)) and
