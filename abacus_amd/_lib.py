@@ -87,6 +87,8 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
                                       _P]),
     "abacus_cross_entropy_fwd": (_I, [_P, _P, _I64, _I64, _I64, _I, _P, _P, _P]),
     "abacus_cross_entropy_bwd": (_I, [_P, _P, _P, _P, _F, _I64, _I64, _I64, _I, _P, _P]),
+    "abacus_cross_entropy_mean_fwd": (_I, [_P, _P, _I64, _I64, _I64, _I, _P, _P, _P, _P, _P]),
+    "abacus_cross_entropy_mean_bwd": (_I, [_P, _P, _P, _P, _P, _I64, _I64, _I64, _I, _P, _P]),
     "abacus_adamw_step": (_I, [_P, _P, _P, _P, _P, _P, _I, _D, _D, _D, _D, _D, _I, _P]),
 }
 

@@ -63,6 +63,35 @@ class _CrossEntropyFunction(torch.autograd.Function):
         return d_logits, None, None, None
 
 
+class _MeanCrossEntropyFunction(torch.autograd.Function):
+    """The mean loss in the logits' dtype, its row count taken and used on the device
+    (_CrossEntropyFunction where the caller does not know the count)."""
+
+    @staticmethod
+    def forward(ctx, logits_NV, targets_N, ignore_index: int):
+        N, V = logits_NV.shape
+        dev = logits_NV.device
+        rows = torch.empty(2, N, dtype=torch.float32, device=dev)  # log-sum-exp and loss per row
+        loss = torch.empty((), dtype=logits_NV.dtype, device=dev)
+        count = torch.empty((), dtype=torch.float32, device=dev)
+        _lib.call("abacus_cross_entropy_mean_fwd", _lib.ptr(logits_NV), _lib.ptr(targets_N), N, V, ignore_index,
+                  _lib.dtype_code(logits_NV.dtype), rows.data_ptr(), rows[1].data_ptr(), _lib.ptr(loss),
+                  _lib.ptr(count), _lib.stream_of(dev))
+        ctx.save_for_backward(logits_NV, targets_N, rows, count)
+        ctx.ignore_index = ignore_index
+        return loss
+
+    @staticmethod
+    def backward(ctx, g):
+        logits_NV, targets_N, rows, count = ctx.saved_tensors
+        N, V = logits_NV.shape
+        d_logits = torch.empty_like(logits_NV)
+        _lib.call("abacus_cross_entropy_mean_bwd", _lib.ptr(logits_NV), _lib.ptr(targets_N), rows.data_ptr(),
+                  g.contiguous().data_ptr(), count.data_ptr(), N, V, ctx.ignore_index,
+                  _lib.dtype_code(logits_NV.dtype), d_logits.data_ptr(), _lib.stream_of(logits_NV.device))
+        return d_logits, None, None
+
+
 _use_liger = False
 
 
@@ -94,8 +123,7 @@ def cross_entropy(input: torch.Tensor, target: torch.Tensor, weight: torch.Tenso
         return F.cross_entropy(input, target, weight=weight, size_average=size_average, ignore_index=ignore_index,
                                reduce=reduce, reduction=reduction, label_smoothing=label_smoothing)
     t = target.to(torch.int64).contiguous()
-    count = (t != ignore_index).sum().to(torch.float32)
-    return _CrossEntropyFunction.apply(input.contiguous(), t, count, int(ignore_index)).to(input.dtype)
+    return _MeanCrossEntropyFunction.apply(input.contiguous(), t, int(ignore_index))
 
 
 def make_optimizer(model: torch.nn.Module, lr: float = 1e-3) -> AdamW:

@@ -374,6 +374,16 @@ int abacus_cross_entropy_bwd(const void* logits_NV, const int64_t* targets_N, co
                              const float* grad_loss, float scale, int64_t N, int64_t V, int64_t ignore_index,
                              int dtype, void* dlogits_NV, void* stream);
 
+/* The same with the mean: loss (one value of `dtype`) = sum of the rows' losses /
+ * count, count (fp32, device) = rows not ignored; the backward takes the loss's
+ * gradient in `dtype` and divides it by count, both read on the device. */
+int abacus_cross_entropy_mean_fwd(const void* logits_NV, const int64_t* targets_N, int64_t N, int64_t V,
+                                  int64_t ignore_index, int dtype, float* lse_N, float* loss_N, void* loss,
+                                  float* count, void* stream);
+int abacus_cross_entropy_mean_bwd(const void* logits_NV, const int64_t* targets_N, const float* lse_N,
+                                  const void* grad_loss, const float* count, int64_t N, int64_t V,
+                                  int64_t ignore_index, int dtype, void* dlogits_NV, void* stream);
+
 /* One AdamW step (optimizers/adamw.py:85-119, AdamW.step) over n tensors in
  * as few launches as possible: for tensor i, params[i], grads[i], exp_avgs[i]
  * and exp_avg_sqs[i] hold numels[i] contiguous elements of `dtype` (16-byte

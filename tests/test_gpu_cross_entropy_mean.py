@@ -1,0 +1,42 @@
+"""cross_entropy's mean on the device: row sums and counts of one and several passes of the mean kernel, vocabularies
+off the vector (rows at any alignment), an ignore index of its own, no rows left, against fp64."""
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+from abacus_amd.train import cross_entropy
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["bf16", "fp32"])
+@pytest.mark.parametrize("N,V,ignore", [(1, 7, -100), (1024, 64, 3), (1025, 65, -100), (3001, 50257, -100),
+                                        (5000, 129, 0), (37, 1030, -100)])
+def test_mean_matches_fp64(dtype, N, V, ignore):
+    g = torch.Generator(device="cuda").manual_seed(N + V)
+    x = (torch.randn(N, V, device="cuda", generator=g) * 3).to(dtype).requires_grad_()
+    t = torch.randint(0, V, (N,), device="cuda", generator=g)
+    t[1::5] = ignore
+    loss = cross_entropy(x, t, ignore_index=ignore)
+    upstream = torch.tensor(0.75, device="cuda", dtype=dtype)
+    (grad,) = torch.autograd.grad(loss, x, upstream)
+    ref_x = x.detach().double().requires_grad_()
+    ref = F.cross_entropy(ref_x, t, ignore_index=ignore)
+    (ref_grad,) = torch.autograd.grad(ref, ref_x, upstream.double())
+    # one rounding to the dtype (bf16 2^-9) over fp32 sums
+    assert loss.dtype == dtype and loss.shape == ()
+    assert abs(float(loss.detach()) - float(ref.detach())) <= (2 ** -8 if dtype == torch.bfloat16 else 1e-5) * abs(float(ref.detach()))
+    err = float((grad.double() - ref_grad).norm() / ref_grad.norm())
+    assert err <= (4e-3 if dtype == torch.bfloat16 else 1e-5), err
+    assert torch.count_nonzero(grad[t == ignore]) == 0
+
+
+def test_no_rows_left_is_nan():
+    x = torch.randn(4, 16, device="cuda").requires_grad_()
+    loss = cross_entropy(x, torch.full((4,), -100, device="cuda"))
+    assert torch.isnan(loss.detach())
+    loss.backward()
+    assert torch.count_nonzero(x.grad) == 0
+    assert torch.isnan(cross_entropy(torch.randn(0, 16, device="cuda"), torch.zeros(0, dtype=torch.int64, device="cuda")))
+
