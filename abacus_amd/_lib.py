@@ -83,8 +83,13 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "abacus_attention_bwd": (_I, [_P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _F, _I, _P, _P, _P, _P, _I64,
                                   _P]),
     "abacus_attention_any_fwd": (_I, [_P, _P, _P, _I64, _I64, _I64, _I64, _F, _I, _P, _P, _P]),
-    "abacus_attention_any_bwd": (_I, [_P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _F, _I, _P, _P, _P, _P, _I64,
-                                      _P]),
+    "abacus_attention_any_bwd": (_I, [_P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _F, _I, _P, _P, _P, _I64, _P,
+                                      _I64, _P]),
+    "abacus_qk_norm_rope_fwd": (_I, [_P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _F, _I, _P, _P, _P, _P]),
+    "abacus_qk_norm_rope_bwd": (_I, [_P, _P, _P, _P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _I, _P, _P, _I64, _P,
+                                     _P, _P, _I64, _P]),
+    "abacus_join3": (_I, [_P, _P, _P, _I64, _I64, _P, _P]),
+    "abacus_split3": (_I, [_P, _I64, _I64, _P, _P, _P, _P]),
     "abacus_cross_entropy_fwd": (_I, [_P, _P, _I64, _I64, _I64, _I, _P, _P, _P]),
     "abacus_cross_entropy_bwd": (_I, [_P, _P, _P, _P, _F, _I64, _I64, _I64, _I, _P, _P]),
     "abacus_cross_entropy_mean_fwd": (_I, [_P, _P, _I64, _I64, _I64, _I, _P, _P, _P, _P, _P]),

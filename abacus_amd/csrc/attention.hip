@@ -482,7 +482,7 @@ template <int HD>
 __device__ __attribute__((always_inline)) inline void attn_bwd_dkdv_block(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
     const uint16_t* __restrict__ dout, const float* __restrict__ lse2, const float* __restrict__ dvec, int L, int H,
-    float scale_log2, float scale, uint16_t* __restrict__ dk, uint16_t* __restrict__ dv, int kb,
+    float scale_log2, float scale, uint16_t* __restrict__ dk, uint16_t* __restrict__ dv, int64_t dv_stride, int kb,
     AttnRing<HD>& lds, AttnStats& stats) {  // [stage][Q, dO], [stage][lse2, D]
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, h = lane >> 5;
   const int head = blockIdx.y, batch = blockIdx.z;
@@ -597,7 +597,7 @@ __device__ __attribute__((always_inline)) inline void attn_bwd_dkdv_block(
   }
   if (my_k >= L) return;
   uint16_t* krow = dk + base + (int64_t)my_k * row_stride;
-  uint16_t* vrow = dv + base + (int64_t)my_k * row_stride;
+  uint16_t* vrow = dv + ((int64_t)batch * L + my_k) * dv_stride + head * HD;
 #pragma unroll
   for (int t = 0; t < HD / 32; ++t)
 #pragma unroll
@@ -616,14 +616,14 @@ template <int HD>
 __global__ __launch_bounds__(kAttnThreads, HD == 64 ? 2 : 1) void attn_bwd_dkdv_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
     const uint16_t* __restrict__ dout, const float* __restrict__ lse2, const float* __restrict__ dvec, int L, int H,
-    float scale_log2, float scale, uint16_t* __restrict__ dk, uint16_t* __restrict__ dv) {
+    float scale_log2, float scale, uint16_t* __restrict__ dk, uint16_t* __restrict__ dv, int64_t dv_stride) {
   __shared__ __attribute__((aligned(1024))) AttnRing<HD> lds;
   __shared__ __attribute__((aligned(16))) AttnStats stats;
   const int nk = (L + kQRows - 1) / kQRows, p = blockIdx.x;
-  attn_bwd_dkdv_block<HD>(q, k, v, dout, lse2, dvec, L, H, scale_log2, scale, dk, dv, p, lds, stats);
+  attn_bwd_dkdv_block<HD>(q, k, v, dout, lse2, dvec, L, H, scale_log2, scale, dk, dv, dv_stride, p, lds, stats);
   if (p != nk - 1 - p) {
     __syncthreads();
-    attn_bwd_dkdv_block<HD>(q, k, v, dout, lse2, dvec, L, H, scale_log2, scale, dk, dv, nk - 1 - p, lds, stats);
+    attn_bwd_dkdv_block<HD>(q, k, v, dout, lse2, dvec, L, H, scale_log2, scale, dk, dv, dv_stride, nk - 1 - p, lds, stats);
   }
 }
 
@@ -649,7 +649,7 @@ int launch_fwd(const uint16_t* q, const uint16_t* k, const uint16_t* v, int64_t 
 template <int HD>
 int launch_bwd(const uint16_t* q, const uint16_t* k, const uint16_t* v, const uint16_t* o, const uint16_t* dout,
                const float* lse, int64_t B, int64_t L, int64_t H, float scale, uint16_t* dq, uint16_t* dk, uint16_t* dv,
-               float* ws, hipStream_t s) {
+               int64_t dv_stride, float* ws, hipStream_t s) {
   const int64_t rows = B * L * H, nq = (L + kQRows - 1) / kQRows;
   const float scale_log2 = scale * 1.4426950408889634f;
   constexpr int kDotRows = 256 / (HD / 8);
@@ -658,7 +658,7 @@ int launch_bwd(const uint16_t* q, const uint16_t* k, const uint16_t* v, const ui
   ABACUS_CHECK_LAUNCH("attention_bwd (dot)");
   const dim3 grid((unsigned)((nq + 1) / 2), (unsigned)H, (unsigned)B);  // block pairs
   hipLaunchKernelGGL(attn_bwd_dkdv_kernel<HD>, grid, dim3(kAttnThreads), 0, s, q, k, v, dout, lse, ws, (int)L, (int)H,
-                     scale_log2, scale, dk, dv);
+                     scale_log2, scale, dk, dv, dv_stride);
   ABACUS_CHECK_LAUNCH("attention_bwd (dk, dv)");
   hipLaunchKernelGGL(attn_bwd_dq_kernel<HD>, grid, dim3(kAttnThreads), 0, s, q, k, v, dout, lse, ws, (int)L, (int)H,
                      scale_log2, scale, dq);
@@ -698,7 +698,9 @@ extern "C" int64_t abacus_attention_bwd_ws_bytes(int64_t B, int64_t L, int64_t H
 extern "C" int abacus_attention_any_bwd(const void* q_BLHK, const void* k_BLHK, const void* v_BLHK, const void* o_BLHK,
                                         const void* dout_BLHK, const float* lse_BHL, int64_t B, int64_t L, int64_t H,
                                         int64_t K, float scale, int dtype, void* dq_BLHK, void* dk_BLHK, void* dv_BLHK,
-                                        float* ws, int64_t ws_bytes, void* stream) {
+                                        int64_t dv_stride, float* ws, int64_t ws_bytes, void* stream) {
+  ABACUS_CHECK_ARG(dv_stride >= H * K && dv_stride % 8 == 0, "attention_bwd: dv's token stride %lld for %lld x %lld",
+                   (long long)dv_stride, (long long)H, (long long)K);
   if (check_attention(B, L, H, K, dtype)) return 1;
   ABACUS_CHECK_ARG(q_BLHK && k_BLHK && v_BLHK && o_BLHK && dout_BLHK && lse_BHL && dq_BLHK && dk_BLHK && dv_BLHK && ws,
                    "attention: null pointer");
@@ -711,7 +713,7 @@ extern "C" int abacus_attention_any_bwd(const void* q_BLHK, const void* k_BLHK, 
   return (K == 64 ? launch_bwd<64> : launch_bwd<128>)(
       (const uint16_t*)q_BLHK, (const uint16_t*)k_BLHK, (const uint16_t*)v_BLHK, (const uint16_t*)o_BLHK,
       (const uint16_t*)dout_BLHK, lse_BHL, B, L, H, scale, (uint16_t*)dq_BLHK, (uint16_t*)dk_BLHK, (uint16_t*)dv_BLHK,
-      ws, (hipStream_t)stream);
+      dv_stride, ws, (hipStream_t)stream);
 }
 
 extern "C" int abacus_attention_bwd(const void* q_BLHK, const void* k_BLHK, const void* v_BLHK, const void* o_BLHK,
@@ -723,5 +725,5 @@ extern "C" int abacus_attention_bwd(const void* q_BLHK, const void* k_BLHK, cons
   ABACUS_CHECK_ARG(L >= kQRows && L % kQRows == 0, "attention: seq_len %lld must be a positive multiple of %d",
                    (long long)L, kQRows);
   return abacus_attention_any_bwd(q_BLHK, k_BLHK, v_BLHK, o_BLHK, dout_BLHK, lse_BHL, B, L, H, K, scale, dtype, dq_BLHK,
-                                  dk_BLHK, dv_BLHK, ws, ws_bytes, stream);
+                                  dk_BLHK, dv_BLHK, H * K, ws, ws_bytes, stream);
 }

@@ -48,8 +48,7 @@ __device__ inline Vec16 pack(const float* f) {
   Vec16 v;
   if constexpr (sizeof(T) == 2) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      v.w[i] = (uint32_t)f32_to_bf16(f[2 * i]) | ((uint32_t)f32_to_bf16(f[2 * i + 1]) << 16);
+    for (int i = 0; i < 4; ++i) v.w[i] = pack_bf16x2(f[2 * i], f[2 * i + 1]);
   } else {
 #pragma unroll
     for (int i = 0; i < 4; ++i) v.w[i] = f32_bits(f[i]);
@@ -63,14 +62,32 @@ __device__ inline float row_sum(float v, int lpr) {
   return v;
 }
 
+// The tensors of a launch: one norm, or (grid.y = 2) the attention's q and k
+// norms side by side.
+struct NormFwd {
+  const void *x[2], *gamma[2];
+  void* y[2];
+  float* rstd[2];
+};
+struct NormBwd {
+  const void *dy[2], *x[2], *gamma[2];
+  const float* rstd[2];
+  void* dx[2];
+  int64_t dx_stride;  // elements between dx's tokens of H rows (0: rows contiguous)
+  float* partial[2];
+  void* dgamma[2];
+};
+
 template <typename T, int VPL, bool ROPE>
-__global__ __launch_bounds__(norm_waves(VPL * VecTraits<T>::kN) * 64) void rmsnorm_fwd_kernel(const T* __restrict__ x,
-                                                                      const T* __restrict__ gamma, int64_t rows,
-                                                                      int D, int lpr, float eps, T* __restrict__ y,
-                                                                      float* __restrict__ rstd,
+__global__ __launch_bounds__(norm_waves(VPL * VecTraits<T>::kN) * 64) void rmsnorm_fwd_kernel(NormFwd a, int64_t rows,
+                                                                      int D, int lpr, float eps,
                                                                       const T* __restrict__ cosv,
                                                                       const T* __restrict__ sinv, int L, int H) {
   static_assert(!ROPE || VPL == 1, "the rotary pairs sit on partner lanes");
+  const T* __restrict__ x = (const T*)(blockIdx.y ? a.x[1] : a.x[0]);
+  const T* __restrict__ gamma = (const T*)(blockIdx.y ? a.gamma[1] : a.gamma[0]);
+  T* __restrict__ y = (T*)(blockIdx.y ? a.y[1] : a.y[0]);
+  float* __restrict__ rstd = blockIdx.y ? a.rstd[1] : a.rstd[0];
   constexpr int EPV = VecTraits<T>::kN;
   constexpr int W = norm_waves(VPL * EPV);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -128,15 +145,16 @@ __global__ __launch_bounds__(norm_waves(VPL * VecTraits<T>::kN) * 64) void rmsno
 }
 
 template <typename T, int VPL, bool ROPE>
-__global__ __launch_bounds__(norm_waves(VPL * VecTraits<T>::kN) * 64) void rmsnorm_bwd_kernel(const T* __restrict__ dy,
-                                                                      const T* __restrict__ x,
-                                                                      const T* __restrict__ gamma,
-                                                                      const float* __restrict__ rstd, int64_t rows,
-                                                                      int D, int lpr, T* __restrict__ dx,
-                                                                      float* __restrict__ partial,
-                                                                      const T* __restrict__ cosv,
+__global__ __launch_bounds__(norm_waves(VPL * VecTraits<T>::kN) * 64) void rmsnorm_bwd_kernel(NormBwd a, int64_t rows,
+                                                                      int D, int lpr, const T* __restrict__ cosv,
                                                                       const T* __restrict__ sinv, int L, int H) {
   static_assert(!ROPE || VPL == 1, "the rotary pairs sit on partner lanes");
+  const T* __restrict__ dy = (const T*)(blockIdx.y ? a.dy[1] : a.dy[0]);
+  const T* __restrict__ x = (const T*)(blockIdx.y ? a.x[1] : a.x[0]);
+  const T* __restrict__ gamma = (const T*)(blockIdx.y ? a.gamma[1] : a.gamma[0]);
+  const float* __restrict__ rstd = blockIdx.y ? a.rstd[1] : a.rstd[0];
+  T* __restrict__ dx = (T*)(blockIdx.y ? a.dx[1] : a.dx[0]);
+  float* __restrict__ partial = blockIdx.y ? a.partial[1] : a.partial[0];
   constexpr int EPV = VecTraits<T>::kN;
   constexpr int NE = VPL * EPV;  // elements per lane
   constexpr int W = norm_waves(NE);
@@ -187,7 +205,8 @@ __global__ __launch_bounds__(norm_waves(VPL * VecTraits<T>::kN) * 64) void rmsno
         float o[EPV];
 #pragma unroll
         for (int i = 0; i < EPV; ++i) o[i] = inv * gf[v * EPV + i] * df[v * EPV + i] - xf[v * EPV + i] * c;
-        st16(dx + r * D + (li + v * lpr) * EPV, pack<T>(o));
+        const int64_t at = ROPE && a.dx_stride ? r / H * a.dx_stride + r % H * D : r * D;
+        st16(dx + at + (li + v * lpr) * EPV, pack<T>(o));
       }
     }
   }
@@ -221,9 +240,9 @@ __global__ __launch_bounds__(norm_waves(VPL * VecTraits<T>::kN) * 64) void rmsno
 // adds them pairwise; the 16 wave sums are added in wave order.
 constexpr int kDgammaWaves = 16;
 template <typename T>
-__global__ __launch_bounds__(kDgammaWaves * 64) void rmsnorm_dgamma_kernel(const float* __restrict__ partial,
-                                                                           int nblocks, int D,
-                                                                           T* __restrict__ dgamma) {
+__global__ __launch_bounds__(kDgammaWaves * 64) void rmsnorm_dgamma_kernel(NormBwd a, int nblocks, int D) {
+  const float* __restrict__ partial = blockIdx.y ? a.partial[1] : a.partial[0];
+  T* __restrict__ dgamma = (T*)(blockIdx.y ? a.dgamma[1] : a.dgamma[0]);
   __shared__ float s_part[kDgammaWaves][64];
   const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int col = blockIdx.x * 64 + l;
@@ -275,6 +294,20 @@ int check_norm(int64_t rows, int64_t D, int dtype, int* lpr, int* vpl) {
 
 int64_t norm_groups(int64_t rows, int lpr) { return (rows + 64 / lpr - 1) / (64 / lpr); }
 
+// Three (rows, vecs) matrices of 16-byte vectors and one of (rows, 3 vecs), in
+// either direction: one launch for the attention's joint weight and its gradient.
+template <bool SPLIT>
+__global__ __launch_bounds__(256) void join3_kernel(char* __restrict__ a, char* __restrict__ b, char* __restrict__ c,
+                                                    int64_t n, int vecs, char* __restrict__ joint) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= n) return;
+  const int64_t row = i / (3 * vecs);
+  const int col = (int)(i - row * 3 * vecs), part = col / vecs;
+  char* p = (part == 0 ? a : part == 1 ? b : c) + (row * vecs + col - part * vecs) * 16;
+  if (SPLIT) st16(p, ld16(joint + i * 16));
+  else st16(joint + i * 16, ld16(p));
+}
+
 }  // namespace
 
 }  // namespace abacus
@@ -283,8 +316,21 @@ using namespace abacus;
 
 namespace {
 
-int norm_fwd(const void* x, const void* gamma, int64_t rows, int64_t D, float eps, int dtype, void* y, float* rstd,
-             const void* cosv, const void* sinv, int64_t L, int64_t H, bool rope, void* stream) {
+template <bool SPLIT>
+int join_or_split(void* a, void* b, void* c, int64_t rows, int64_t row_bytes, void* joint, void* stream) {
+  ABACUS_CHECK_ARG(rows >= 0 && row_bytes >= 16 && row_bytes % 16 == 0 && row_bytes < (1ll << 30) &&
+                       rows * (row_bytes / 16) < (1ll << 36),
+                   "join3: %lld rows of %lld bytes", (long long)rows, (long long)row_bytes);
+  if (rows == 0) return 0;
+  const int64_t n = rows * 3 * (row_bytes / 16);
+  hipLaunchKernelGGL(join3_kernel<SPLIT>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, (hipStream_t)stream, (char*)a,
+                     (char*)b, (char*)c, n, (int)(row_bytes / 16), (char*)joint);
+  ABACUS_CHECK_LAUNCH("join3");
+  return 0;
+}
+
+int norm_fwd(const NormFwd& a, int pairs, int64_t rows, int64_t D, float eps, int dtype, const void* cosv,
+             const void* sinv, int64_t L, int64_t H, bool rope, void* stream) {
   int lpr, vpl;
   if (check_norm(rows, D, dtype, &lpr, &vpl)) return 1;
   if (rope) {
@@ -297,9 +343,8 @@ int norm_fwd(const void* x, const void* gamma, int64_t rows, int64_t D, float ep
   const unsigned grid = (unsigned)std::min<int64_t>(kNormMaxBlocks, (groups + W - 1) / W);
   hipStream_t s = (hipStream_t)stream;
 #define ABACUS_NORM_FWD(TT, V, R)                                                                                 \
-  hipLaunchKernelGGL((rmsnorm_fwd_kernel<TT, V, R>), dim3(grid), dim3(W * 64), 0, s, (const TT*)x,                \
-                     (const TT*)gamma, rows, (int)D, lpr, eps, (TT*)y, rstd, (const TT*)cosv, (const TT*)sinv,   \
-                     (int)L, (int)H)
+  hipLaunchKernelGGL((rmsnorm_fwd_kernel<TT, V, R>), dim3(grid, pairs), dim3(W * 64), 0, s, a, rows, (int)D, lpr,  \
+                     eps, (const TT*)cosv, (const TT*)sinv, (int)L, (int)H)
   if (dtype == kBF16) {
     if (rope) ABACUS_NORM_FWD(uint16_t, 1, true);
     else if (vpl == 1) ABACUS_NORM_FWD(uint16_t, 1, false);
@@ -318,9 +363,8 @@ int norm_fwd(const void* x, const void* gamma, int64_t rows, int64_t D, float ep
   return 0;
 }
 
-int norm_bwd(const void* dy, const void* x, const void* gamma, const float* rstd, int64_t rows, int64_t D, int dtype,
-             void* dx, void* dgamma, float* ws, int64_t ws_bytes, const void* cosv, const void* sinv, int64_t L,
-             int64_t H, bool rope, void* stream) {
+int norm_bwd(NormBwd a, int pairs, int64_t rows, int64_t D, int dtype, float* ws, int64_t ws_bytes, const void* cosv,
+             const void* sinv, int64_t L, int64_t H, bool rope, void* stream) {
   int lpr, vpl;
   if (check_norm(rows, D, dtype, &lpr, &vpl)) return 1;
   if (rope) {
@@ -331,23 +375,24 @@ int norm_bwd(const void* dy, const void* x, const void* gamma, const float* rstd
   const int64_t groups = norm_groups(rows, lpr);
   const int W = norm_waves(vpl * (dtype == kBF16 ? 8 : 4));
   const int nb = (int)std::max<int64_t>(1, std::min<int64_t>(kNormBwdBlocks, (groups + W - 1) / W));
-  ABACUS_CHECK_ARG(rows == 0 || ws_bytes >= (int64_t)nb * D * 4, "rmsnorm_bwd: workspace of %lld bytes, need %lld",
-                   (long long)ws_bytes, (long long)nb * D * 4);
+  ABACUS_CHECK_ARG(rows == 0 || ws_bytes >= (int64_t)pairs * nb * D * 4,
+                   "rmsnorm_bwd: workspace of %lld bytes, need %lld", (long long)ws_bytes,
+                   (long long)pairs * nb * D * 4);
+  a.partial[0] = ws;
+  a.partial[1] = pairs > 1 ? ws + (int64_t)nb * D : nullptr;
+  const dim3 dg_grid((unsigned)((D + 63) / 64), (unsigned)pairs);
   if (rows == 0) {
     // no rows: dgamma is zero
     if (dtype == kBF16)
-      hipLaunchKernelGGL(rmsnorm_dgamma_kernel<uint16_t>, dim3((unsigned)((D + 63) / 64)), dim3(kDgammaWaves * 64), 0, s, ws, 0,
-                         (int)D, (uint16_t*)dgamma);
+      hipLaunchKernelGGL(rmsnorm_dgamma_kernel<uint16_t>, dg_grid, dim3(kDgammaWaves * 64), 0, s, a, 0, (int)D);
     else
-      hipLaunchKernelGGL(rmsnorm_dgamma_kernel<float>, dim3((unsigned)((D + 63) / 64)), dim3(kDgammaWaves * 64), 0, s, ws, 0,
-                         (int)D, (float*)dgamma);
+      hipLaunchKernelGGL(rmsnorm_dgamma_kernel<float>, dg_grid, dim3(kDgammaWaves * 64), 0, s, a, 0, (int)D);
     ABACUS_CHECK_LAUNCH("rmsnorm_dgamma");
     return 0;
   }
 #define ABACUS_NORM_BWD(TT, V, R)                                                                                  \
-  hipLaunchKernelGGL((rmsnorm_bwd_kernel<TT, V, R>), dim3(nb), dim3(W * 64), 0, s, (const TT*)dy,                  \
-                     (const TT*)x, (const TT*)gamma, rstd, rows, (int)D, lpr, (TT*)dx, ws, (const TT*)cosv,        \
-                     (const TT*)sinv, (int)L, (int)H)
+  hipLaunchKernelGGL((rmsnorm_bwd_kernel<TT, V, R>), dim3(nb, pairs), dim3(W * 64), 0, s, a, rows, (int)D, lpr,    \
+                     (const TT*)cosv, (const TT*)sinv, (int)L, (int)H)
   if (dtype == kBF16) {
     if (rope) ABACUS_NORM_BWD(uint16_t, 1, true);
     else if (vpl == 1) ABACUS_NORM_BWD(uint16_t, 1, false);
@@ -364,11 +409,9 @@ int norm_bwd(const void* dy, const void* x, const void* gamma, const float* rstd
 #undef ABACUS_NORM_BWD
   ABACUS_CHECK_LAUNCH("rmsnorm_bwd");
   if (dtype == kBF16)
-    hipLaunchKernelGGL(rmsnorm_dgamma_kernel<uint16_t>, dim3((unsigned)((D + 63) / 64)), dim3(kDgammaWaves * 64), 0, s, ws, nb,
-                       (int)D, (uint16_t*)dgamma);
+    hipLaunchKernelGGL(rmsnorm_dgamma_kernel<uint16_t>, dg_grid, dim3(kDgammaWaves * 64), 0, s, a, nb, (int)D);
   else
-    hipLaunchKernelGGL(rmsnorm_dgamma_kernel<float>, dim3((unsigned)((D + 63) / 64)), dim3(kDgammaWaves * 64), 0, s, ws, nb,
-                       (int)D, (float*)dgamma);
+    hipLaunchKernelGGL(rmsnorm_dgamma_kernel<float>, dg_grid, dim3(kDgammaWaves * 64), 0, s, a, nb, (int)D);
   ABACUS_CHECK_LAUNCH("rmsnorm_dgamma");
   return 0;
 }
@@ -384,24 +427,58 @@ int64_t abacus_rmsnorm_bwd_ws_bytes(int64_t rows, int64_t D) {
 
 int abacus_rmsnorm_fwd(const void* x, const void* gamma, int64_t rows, int64_t D, float eps, int dtype, void* y,
                        float* rstd, void* stream) {
-  return norm_fwd(x, gamma, rows, D, eps, dtype, y, rstd, nullptr, nullptr, 1, 1, false, stream);
+  const NormFwd a{{x, nullptr}, {gamma, nullptr}, {y, nullptr}, {rstd, nullptr}};
+  return norm_fwd(a, 1, rows, D, eps, dtype, nullptr, nullptr, 1, 1, false, stream);
 }
 
 int abacus_rmsnorm_bwd(const void* dy, const void* x, const void* gamma, const float* rstd, int64_t rows, int64_t D,
                        int dtype, void* dx, void* dgamma, float* ws, int64_t ws_bytes, void* stream) {
-  return norm_bwd(dy, x, gamma, rstd, rows, D, dtype, dx, dgamma, ws, ws_bytes, nullptr, nullptr, 1, 1, false, stream);
+  const NormBwd a{{dy, nullptr}, {x, nullptr}, {gamma, nullptr}, {rstd, nullptr}, {dx, nullptr}, 0, {nullptr, nullptr},
+                  {dgamma, nullptr}};
+  return norm_bwd(a, 1, rows, D, dtype, ws, ws_bytes, nullptr, nullptr, 1, 1, false, stream);
 }
 
 int abacus_rmsnorm_rope_fwd(const void* x, const void* gamma, const void* cos_LK, const void* sin_LK, int64_t rows,
                             int64_t L, int64_t H, int64_t K, float eps, int dtype, void* y, float* rstd,
                             void* stream) {
-  return norm_fwd(x, gamma, rows, K, eps, dtype, y, rstd, cos_LK, sin_LK, L, H, true, stream);
+  const NormFwd a{{x, nullptr}, {gamma, nullptr}, {y, nullptr}, {rstd, nullptr}};
+  return norm_fwd(a, 1, rows, K, eps, dtype, cos_LK, sin_LK, L, H, true, stream);
 }
 
 int abacus_rmsnorm_rope_bwd(const void* dy, const void* x, const void* gamma, const float* rstd, const void* cos_LK,
                             const void* sin_LK, int64_t rows, int64_t L, int64_t H, int64_t K, int dtype, void* dx,
                             void* dgamma, float* ws, int64_t ws_bytes, void* stream) {
-  return norm_bwd(dy, x, gamma, rstd, rows, K, dtype, dx, dgamma, ws, ws_bytes, cos_LK, sin_LK, L, H, true, stream);
+  const NormBwd a{{dy, nullptr}, {x, nullptr}, {gamma, nullptr}, {rstd, nullptr}, {dx, nullptr}, 0, {nullptr, nullptr},
+                  {dgamma, nullptr}};
+  return norm_bwd(a, 1, rows, K, dtype, ws, ws_bytes, cos_LK, sin_LK, L, H, true, stream);
+}
+
+int abacus_qk_norm_rope_fwd(const void* q, const void* k, const void* gamma_q, const void* gamma_k, const void* cos_LK,
+                            const void* sin_LK, int64_t rows, int64_t L, int64_t H, int64_t K, float eps, int dtype,
+                            void* y_q, void* y_k, float* rstd, void* stream) {
+  const NormFwd a{{q, k}, {gamma_q, gamma_k}, {y_q, y_k}, {rstd, rstd + rows}};
+  return norm_fwd(a, 2, rows, K, eps, dtype, cos_LK, sin_LK, L, H, true, stream);
+}
+
+int abacus_qk_norm_rope_bwd(const void* dy_q, const void* dy_k, const void* q, const void* k, const void* gamma_q,
+                            const void* gamma_k, const float* rstd, const void* cos_LK, const void* sin_LK,
+                            int64_t rows, int64_t L, int64_t H, int64_t K, int dtype, void* dq, void* dk,
+                            int64_t token_stride, void* dgamma_q, void* dgamma_k, float* ws, int64_t ws_bytes,
+                            void* stream) {
+  ABACUS_CHECK_ARG(token_stride >= H * K && token_stride % 8 == 0, "qk_norm_rope_bwd: token stride %lld for %lld x %lld",
+                   (long long)token_stride, (long long)H, (long long)K);
+  const NormBwd a{{dy_q, dy_k}, {q, k}, {gamma_q, gamma_k}, {rstd, rstd + rows}, {dq, dk}, token_stride,
+                  {nullptr, nullptr}, {dgamma_q, dgamma_k}};
+  return norm_bwd(a, 2, rows, K, dtype, ws, ws_bytes, cos_LK, sin_LK, L, H, true, stream);
+}
+
+int abacus_join3(const void* a, const void* b, const void* c, int64_t rows, int64_t row_bytes, void* out, void* stream) {
+  return join_or_split<false>(const_cast<void*>(a), const_cast<void*>(b), const_cast<void*>(c), rows, row_bytes, out,
+                              stream);
+}
+
+int abacus_split3(const void* in, int64_t rows, int64_t row_bytes, void* a, void* b, void* c, void* stream) {
+  return join_or_split<true>(a, b, c, rows, row_bytes, const_cast<void*>(in), stream);
 }
 
 }  // extern "C"

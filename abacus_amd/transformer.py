@@ -329,9 +329,11 @@ class _FlashAttentionFunction(torch.autograd.Function):
         dq, dk, dv = (torch.empty_like(q) for _ in range(3))
         nbytes = _lib.query("abacus_attention_bwd_ws_bytes", B, L, H)
         ws = torch.empty(nbytes // 4, dtype=torch.float32, device=q.device)
-        _lib.call(_flash_entry(q, "bwd"), _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(o), _lib.ptr(d_o),
+        entry = _flash_entry(q, "bwd")
+        stride = (H * K,) if entry == "abacus_attention_any_bwd" else ()
+        _lib.call(entry, _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(o), _lib.ptr(d_o),
                   _lib.ptr(lse), B, L, H, K, 1.0 / math.sqrt(K), _lib.BF16, _lib.ptr(dq), _lib.ptr(dk), _lib.ptr(dv),
-                  _lib.ptr(ws), nbytes, _lib.stream_of(q.device))
+                  *stride, _lib.ptr(ws), nbytes, _lib.stream_of(q.device))
         return dq, dk, dv
 
 
@@ -380,6 +382,85 @@ class _QKVProjection(torch.autograd.Function):
             dwq, dwk, dwv = (dw_D3[:, i * HK:(i + 1) * HK].contiguous().view(D, H, K) if ctx.needs_input_grad[1 + i]
                              else None for i in range(3))
         return dx, dwq, dwk, dwv
+
+
+class _AttentionFunction(torch.autograd.Function):
+    """_QKVProjection, the q and k norms with the rotary embedding and causal attention as one node
+    (bf16 on the GPU): the same products and kernels, with the q and k norms in one launch each
+    way and dq, dk, dv written by their kernels as columns of the joint (T, 3HK) gradient that the
+    projection's two backward products read, so nothing is concatenated on the way.  At B 4,
+    L 2048, H 16, K 64 the attention block's forward + backward went 623 -> 565 us.
+    """
+
+    @staticmethod
+    def forward(ctx, x_BLD, w_q, w_k, w_v, gamma_q, gamma_k, cos_LK, sin_LK, eps: float):
+        B, L, D = x_BLD.shape
+        _, H, K = w_q.shape
+        rows, dev = B * L * H, x_BLD.device
+        s = _lib.stream_of(dev)
+        x_TD = x_BLD.reshape(B * L, D)
+        q, k, v = ((x_TD @ w.reshape(D, H * K)).view(B, L, H, K) for w in (w_q, w_k, w_v))
+        gamma_q, gamma_k, cos_c, sin_c = (t.contiguous() for t in (gamma_q, gamma_k, cos_LK, sin_LK))
+        qn, kn, o = torch.empty_like(q), torch.empty_like(k), torch.empty_like(q)
+        rstd = torch.empty(2, rows, dtype=torch.float32, device=dev)
+        lse = torch.empty(B, H, L, dtype=torch.float32, device=dev)
+        _lib.call("abacus_qk_norm_rope_fwd", _lib.ptr(q), _lib.ptr(k), _lib.ptr(gamma_q), _lib.ptr(gamma_k),
+                  _lib.ptr(cos_c), _lib.ptr(sin_c), rows, L, H, K, eps, _lib.BF16, _lib.ptr(qn), _lib.ptr(kn),
+                  _lib.ptr(rstd), s)
+        _lib.call("abacus_attention_any_fwd", _lib.ptr(qn), _lib.ptr(kn), _lib.ptr(v), B, L, H, K,
+                  1.0 / math.sqrt(K), _lib.BF16, _lib.ptr(o), _lib.ptr(lse), s)
+        ctx.save_for_backward(x_TD, w_q, w_k, w_v, gamma_q, gamma_k, cos_c, sin_c, q, k, v, qn, kn, o, rstd, lse)
+        ctx.x_shape = (B, L, D)
+        return o
+
+    @staticmethod
+    def backward(ctx, d_o):
+        x_TD, w_q, w_k, w_v, gamma_q, gamma_k, cos_c, sin_c, q, k, v, qn, kn, o, rstd, lse = ctx.saved_tensors
+        B, L, D = ctx.x_shape
+        _, H, K = w_q.shape
+        HK, rows, dev = H * K, B * L * H, q.device
+        s = _lib.stream_of(dev)
+        d_o = d_o.contiguous()
+        dqn, dkn = torch.empty_like(q), torch.empty_like(k)
+        joint = torch.empty(B * L, 3 * HK, dtype=q.dtype, device=dev)
+        dgamma_q, dgamma_k = torch.empty_like(gamma_q), torch.empty_like(gamma_k)
+        nbytes = _lib.query("abacus_attention_bwd_ws_bytes", B, L, H)
+        norm_bytes = 2 * _lib.query("abacus_rmsnorm_bwd_ws_bytes", rows, K)
+        ws = torch.empty(max(nbytes, norm_bytes) // 4, dtype=torch.float32, device=dev)
+        at, col = joint.data_ptr(), HK * joint.element_size()
+        _lib.call("abacus_attention_any_bwd", _lib.ptr(qn), _lib.ptr(kn), _lib.ptr(v), _lib.ptr(o), _lib.ptr(d_o),
+                  _lib.ptr(lse), B, L, H, K, 1.0 / math.sqrt(K), _lib.BF16, _lib.ptr(dqn), _lib.ptr(dkn), at + 2 * col,
+                  3 * HK, _lib.ptr(ws), nbytes, s)
+        _lib.call("abacus_qk_norm_rope_bwd", _lib.ptr(dqn), _lib.ptr(dkn), _lib.ptr(q), _lib.ptr(k), _lib.ptr(gamma_q),
+                  _lib.ptr(gamma_k), _lib.ptr(rstd), _lib.ptr(cos_c), _lib.ptr(sin_c), rows, L, H, K, _lib.BF16, at,
+                  at + col, 3 * HK, _lib.ptr(dgamma_q), _lib.ptr(dgamma_k), _lib.ptr(ws), norm_bytes, s)
+        needs = ctx.needs_input_grad
+        dx = None
+        dws = [None, None, None]
+        if needs[0]:
+            w_D3 = torch.empty(D, 3 * HK, dtype=q.dtype, device=dev)
+            w_c = [w.contiguous() for w in (w_q, w_k, w_v)]
+            _lib.call("abacus_join3", *map(_lib.ptr, w_c), D, col, _lib.ptr(w_D3), s)
+            dx = (joint @ w_D3.t()).view(B, L, D)
+        if any(needs[1:4]):
+            dw_D3 = x_TD.t() @ joint
+            dws = [torch.empty(D, H, K, dtype=q.dtype, device=dev) for _ in range(3)]
+            _lib.call("abacus_split3", _lib.ptr(dw_D3), D, col, *map(_lib.ptr, dws), s)
+            dws = [g if need else None for g, need in zip(dws, needs[1:4])]
+        return (dx, *dws, dgamma_q if needs[4] else None, dgamma_k if needs[5] else None, None, None, None)
+
+
+def _joint_ok(x: torch.Tensor, weights, gammas, rotary) -> bool:
+    """_AttentionFunction takes what the flash kernels and the norm + rotary kernel take (bf16 on the
+    GPU, heads of 64 or 128), with this module's own Rotary, outside autocast.  While a KernelTimer
+    wants each entry point by its name, the separate nodes run."""
+    H, K = weights[0].shape[1:]
+    return (flash_attention_enabled and not _lib.timing() and x.is_cuda and x.dim() == 3 and x.numel() > 0
+            and x.dtype == torch.bfloat16 and K in (64, 128) and x.shape[0] <= 65535 and H <= 65535 and H * K < 1 << 24
+            and all(t.dtype == x.dtype and t.device == x.device for t in (*weights, *gammas))
+            and type(rotary) is Rotary and not rotary._forward_hooks and not rotary._forward_pre_hooks
+            and rotary.inv_freq.dtype == x.dtype and rotary.inv_freq.shape[0] * 2 == K
+            and not torch.is_autocast_enabled())
 
 
 class MultiHeadAttention(torch.nn.Module):
@@ -438,6 +519,11 @@ class MultiHeadAttention(torch.nn.Module):
             _single_process("attention parallelism")
         B, L, _ = x_BLD.shape
         H, K = self.local_heads, self.head_dim
+        weights, gammas = (self.w_q_DHK, self.w_k_DHK, self.w_v_DHK), (self.q_norm.w_gamma_D, self.k_norm.w_gamma_D)
+        if _joint_ok(x_BLD, weights, gammas, rotary):
+            cos, sin = rotary(x_BLD, seq_dim=1)  # (1, 1, L, K)
+            out = _AttentionFunction.apply(x_BLD, *weights, *gammas, cos.reshape(L, K), sin.reshape(L, K), 1e-5)
+            return out.reshape(B, L, H * K) @ self.w_o_HKD.reshape(H * K, self.dim)
         q_heads, k_heads, v_heads = _QKVProjection.apply(x_BLD, self.w_q_DHK, self.w_k_DHK, self.w_v_DHK)
         cos = sin = None
         if rotary is not None:

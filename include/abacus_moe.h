@@ -306,6 +306,23 @@ int abacus_rmsnorm_rope_bwd(const void* dy, const void* x, const void* gamma, co
                             const void* sin_LK, int64_t rows, int64_t L, int64_t H, int64_t K, int dtype, void* dx,
                             void* dgamma, float* ws, int64_t ws_bytes, void* stream);
 
+/* abacus_rmsnorm_rope_fwd / _bwd for q and k in one launch: rstd holds q's rows,
+ * then k's; dq and dk have tokens of H rows token_stride elements apart (so that
+ * they can be columns of one wider matrix); ws: twice abacus_rmsnorm_bwd_ws_bytes. */
+int abacus_qk_norm_rope_fwd(const void* q, const void* k, const void* gamma_q, const void* gamma_k, const void* cos_LK,
+                            const void* sin_LK, int64_t rows, int64_t L, int64_t H, int64_t K, float eps, int dtype,
+                            void* y_q, void* y_k, float* rstd, void* stream);
+int abacus_qk_norm_rope_bwd(const void* dy_q, const void* dy_k, const void* q, const void* k, const void* gamma_q,
+                            const void* gamma_k, const float* rstd, const void* cos_LK, const void* sin_LK,
+                            int64_t rows, int64_t L, int64_t H, int64_t K, int dtype, void* dq, void* dk,
+                            int64_t token_stride, void* dgamma_q, void* dgamma_k, float* ws, int64_t ws_bytes,
+                            void* stream);
+
+/* out = [a b c] row by row, and the reverse: rows of row_bytes (whole 16-byte
+ * vectors) in a, b and c, of three times that in the joint matrix. */
+int abacus_join3(const void* a, const void* b, const void* c, int64_t rows, int64_t row_bytes, void* out, void* stream);
+int abacus_split3(const void* in, int64_t rows, int64_t row_bytes, void* a, void* b, void* c, void* stream);
+
 /* Causal attention forward (attention.py:136-141), flash style: for the
  * B*H (batch, head) pairs of q, k, v in (B, L, H, K) layout (token rows of
  * H*K contiguous elements, bf16, K = 64, L a multiple of 128),
@@ -336,10 +353,11 @@ int abacus_attention_bwd(const void* q_BLHK, const void* k_BLHK, const void* v_B
                          float scale, int dtype, void* dq_BLHK, void* dk_BLHK, void* dv_BLHK, float* ws,
                          int64_t ws_bytes, void* stream);
 
-/* The same for any L >= 1 and K = 64 or 128 (abacus_attention_any_fwd's o and lse_BHL). */
+/* The same for any L >= 1 and K = 64 or 128 (abacus_attention_any_fwd's o and lse_BHL);
+ * dv's tokens are dv_stride elements apart (H*K: contiguous). */
 int abacus_attention_any_bwd(const void* q_BLHK, const void* k_BLHK, const void* v_BLHK, const void* o_BLHK,
                              const void* dout_BLHK, const float* lse_BHL, int64_t B, int64_t L, int64_t H, int64_t K,
-                             float scale, int dtype, void* dq_BLHK, void* dk_BLHK, void* dv_BLHK, float* ws,
+                             float scale, int dtype, void* dq_BLHK, void* dk_BLHK, void* dv_BLHK, int64_t dv_stride, float* ws,
                              int64_t ws_bytes, void* stream);
 
 /* The MoE layer as one call per direction (GPU only): the entry points above in

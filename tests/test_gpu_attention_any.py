@@ -36,7 +36,7 @@ def test_any_length_matches_fp64(B, L, H, K):
     nbytes = _lib.query("abacus_attention_bwd_ws_bytes", B, L, H)
     ws = torch.empty(nbytes // 4, dtype=torch.float32, device="cuda")
     _lib.call("abacus_attention_any_bwd", _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(o), _lib.ptr(dout),
-              _lib.ptr(lse2), B, L, H, K, scale, 1, _lib.ptr(dq), _lib.ptr(dk), _lib.ptr(dv), _lib.ptr(ws), nbytes, s)
+              _lib.ptr(lse2), B, L, H, K, scale, 1, _lib.ptr(dq), _lib.ptr(dk), _lib.ptr(dv), H * K, _lib.ptr(ws), nbytes, s)
     torch.cuda.synchronize()
     leaves = [t.double().requires_grad_() for t in (q, k, v)]
     want, want_lse = _exact(*leaves, scale)
@@ -62,6 +62,39 @@ def test_module_runs_any_kernels(L, K):
         attn(x, rot).sum().backward()
     assert {"abacus_attention_any_fwd", "abacus_attention_any_bwd"} <= set(timer.totals_ms())
     assert torch.isfinite(x.grad.float()).all()
+
+
+@pytest.mark.parametrize("B,L,H,K", [(2, 256, 3, 64), (1, 75, 2, 128), (3, 1, 1, 64)])
+def test_joint_node_equals_separate_nodes(B, L, H, K):
+    """The attention as one node against the separate nodes (which run while a KernelTimer is active): the same
+    kernels on the same operands, so every output and gradient agrees bit for bit; frozen parameters get none."""
+    torch.manual_seed(8)
+    dim = 96
+    attn = tr.MultiHeadAttention(dim, H, K).to(torch.bfloat16).cuda()
+    rot = tr.Rotary(K).to(torch.bfloat16).cuda()
+    x = torch.randn(B, L, dim, device="cuda").to(torch.bfloat16)
+    dy = torch.randn(B, L, dim, device="cuda").to(torch.bfloat16)
+
+    def run():
+        xi = x.clone().requires_grad_()
+        attn.zero_grad(set_to_none=True)
+        y = attn(xi, rot)
+        y.backward(dy)
+        return [y.detach(), xi.grad] + [p.grad for p in attn.parameters()]
+
+    joint = run()
+    with _lib.KernelTimer():
+        separate = run()
+    for name, a, b in zip(["out", "dx"] + [n for n, _ in attn.named_parameters()], joint, separate):
+        assert torch.equal(a, b), name
+    with torch.no_grad():
+        assert torch.equal(attn(x, rot), joint[0])
+    attn.w_k_DHK.requires_grad_(False)
+    attn.q_norm.w_gamma_D.requires_grad_(False)
+    attn.zero_grad(set_to_none=True)
+    attn(x, rot).backward(dy)  # x needs no gradient either
+    assert attn.w_k_DHK.grad is None and attn.q_norm.w_gamma_D.grad is None
+    assert torch.equal(attn.w_q_DHK.grad, joint[2]) and torch.equal(attn.w_v_DHK.grad, joint[4])
 
 
 def test_any_rejects_head_dims():
