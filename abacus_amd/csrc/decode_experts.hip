@@ -276,6 +276,273 @@ __global__ __launch_bounds__(W * 64, 2) void decode_down_kernel(const T* __restr
   }
 }
 
+// More rows per expert (bf16): blocks of up to 64 rows of one expert, so that
+// most experts' weights still stream once.  Block b's tile comes from the
+// offsets: (expert, columns, rows), the rows fastest, numbered over the
+// real ones only, an equal contiguous share to each XCD (block b runs on XCD b % 8),
+// so that the blocks that read the same weights run beside each other on one L2
+// (weights that are read nontemporal miss it: E 64 D 2048 M 1408, 682 tokens 346 -> 410 us).
+// What bounds them is the weight stream as long as an expert's rows are one block's.
+// 64 rows: more would not fit the registers (128 of 256 hold the sums), fewer stream
+// the weights more often.
+constexpr int kMidRows = 64;
+
+struct MidTile {
+  int e, row0, row1, col;  // row1: the expert's end or row0 + kMidRows
+};
+
+// Every wave finds the tile by itself; false: this block has none.
+__device__ __forceinline__ bool mid_tile(const int32_t* __restrict__ offsets, int E, int cols, int lane, MidTile& t) {
+  auto chunks = [&](int e) { return e < E ? (offsets[e + 1] - offsets[e] + kMidRows - 1) / kMidRows : 0; };
+  int total = 0;
+  for (int e0 = 0; e0 < E; e0 += 64) {
+    int c = chunks(e0 + lane);
+#pragma unroll
+    for (int o = 32; o; o >>= 1) c += __shfl_xor(c, o, 64);
+    total += c;
+  }
+  const int per = (total * cols + 7) / 8, b = (int)blockIdx.x;
+  const int L = (b & 7) * per + (b >> 3);
+  if ((b >> 3) >= per || L >= total * cols) return false;
+  int before = 0;
+  for (int e0 = 0; e0 < E; e0 += 64) {
+    const int c = chunks(e0 + lane);
+    int end = c;  // inclusive scan over the lanes
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int u = __shfl_up(end, o, 64);
+      if (lane >= o) end += u;
+    }
+    const uint64_t past = __ballot((before + end) * cols > L);
+    if (past) {
+      const int l = __builtin_ctzll(past);
+      const int n = __builtin_amdgcn_readlane(c, l);
+      const int at = L - (before + __builtin_amdgcn_readlane(end, l) - n) * cols;
+      t.e = e0 + l;
+      t.col = at / n;
+      t.row0 = offsets[t.e] + at % n * kMidRows;
+      t.row1 = min(t.row0 + kMidRows, offsets[t.e + 1]);
+      return true;
+    }
+    before += __builtin_amdgcn_readlane(end, 63);
+  }
+  return false;
+}
+
+// acc[r][j] += step_mfma's product for G groups of 16 rows, each column transposed once.
+template <int G>
+__device__ inline void step_groups(dec_f32x4 (&acc)[G][8], const Vec16 (&w)[8], const Vec16 (&x)[G]) {
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    Vec16 b;
+#pragma unroll
+    for (int p = 0; p < 4; ++p)
+      b.w[p] = __builtin_amdgcn_perm(w[2 * p + 1].w[j >> 1], w[2 * p].w[j >> 1], (j & 1) ? 0x07060302u : 0x05040100u);
+#pragma unroll
+    for (int r = 0; r < G; ++r)
+      acc[r][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(dec_bf16x8, x[r]),
+                                                          __builtin_bit_cast(dec_bf16x8, b), acc[r][j], 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);  // one column's transpose live at a time
+  }
+}
+
+// A wave-uniform pointer kept in scalar registers, for loops whose accumulators
+// leave no room: else the compiler steps one 64-bit vector address per load
+// through the loop, some 50 registers (64 rows a pass then spill in it).
+typedef const __attribute__((address_space(1))) char* global_bytes;
+__device__ inline global_bytes scalar_base(const void* p) {
+  uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)(uint64_t)p);
+  uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)((uint64_t)p >> 32));
+  asm("" : "+s"(lo), "+s"(hi));
+  return (global_bytes)(((uint64_t)hi << 32) | lo);
+}
+// The 16 bytes at base + off, aligned or at any element.
+template <bool UNALIGNED>
+__device__ inline Vec16 load_at(global_bytes base, uint32_t off) {
+  typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+  typedef uint32_t u32x4_ua __attribute__((ext_vector_type(4), aligned(2)));
+  typedef const __attribute__((address_space(1))) u32x4_t* whole_ptr;
+  typedef const __attribute__((address_space(1))) u32x4_ua* any_ptr;
+  u32x4_t v;
+  if constexpr (UNALIGNED) {
+    v = *(any_ptr)(base + off);
+  } else {
+    v = *(whole_ptr)(base + off);
+  }
+  Vec16 r;
+  r.w[0] = v.x; r.w[1] = v.y; r.w[2] = v.z; r.w[3] = v.w;
+  return r;
+}
+
+// acc += x[rows] * w over the k-blocks kb0, kb0 + kstride, ... < kb1, as
+// stream_rows, for G groups of rows that are all computed (no branches between
+// the loads and products), the weights at any element.
+template <bool UNALIGNED, int G>
+__device__ __forceinline__ void stream_groups(const uint16_t* __restrict__ w, int64_t ldw, const uint16_t* __restrict__ x,
+                                              int64_t pitch, int n_rows, int K, int kb0, int kb1, int kstride, int lane,
+                                              dec_f32x4 (&acc)[G][8]) {
+  struct Operands {
+    Vec16 w[8], x[G];
+  };
+  const int kl = 8 * (lane >> 4);
+  const uint32_t woff = 2 * ((uint32_t)kl * (uint32_t)ldw + 8 * (lane & 15));  // bytes
+  uint32_t xoff[G];
+#pragma unroll
+  for (int r = 0; r < G; ++r) xoff[r] = 2 * ((uint32_t)min(r * kGroup + (lane & 15), n_rows - 1) * (uint32_t)pitch + kl);
+  auto load = [&](Operands& s, int kb) __attribute__((always_inline)) {
+    const uint16_t* wb = w + (int64_t)kb * kKB * ldw;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) s.w[i] = load_at<UNALIGNED>(scalar_base(wb + i * ldw), woff);
+    const global_bytes xb = scalar_base(x + (int64_t)kb * kKB);
+#pragma unroll
+    for (int r = 0; r < G; ++r) s.x[r] = load_at<false>(xb, xoff[r]);
+  };
+  const int whole = min(kb1, K / kKB);  // k-blocks without a tail
+  Operands a, b;
+  int kb = kb0;
+  if (kb < whole) load(a, kb);
+  while (kb < whole) {  // the next block's loads go out before this one's products
+    if (kb + kstride < whole) load(b, kb + kstride);
+    step_groups<G>(acc, a.w, a.x);
+    kb += kstride;
+    if (kb >= whole) break;
+    if (kb + kstride < whole) load(a, kb + kstride);
+    step_groups<G>(acc, b.w, b.x);
+    kb += kstride;
+  }
+  if (kb < kb1) {  // the tail block: rows from K on read row K - 1 and count as zero
+    const int k = kb * kKB + kl;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      a.w[i] = load_weights<uint16_t, UNALIGNED, false>(w + (int64_t)min(k + i, K - 1) * ldw + 8 * (lane & 15));
+      if (k + i >= K) a.w[i] = zero16();
+    }
+#pragma unroll
+    for (int r = 0; r < G; ++r) a.x[r] = k < K ? ld16(x + (int64_t)kb * kKB + xoff[r] / 2) : zero16();
+    step_groups<G>(acc, a.w, a.x);
+  }
+}
+
+// H = silu(x w_gate) (x w_up) for rows r0 .. min(r0 + 16 G, row1) - 1 of one
+// expert and the kCols columns from n0.  The first half of the block's W waves
+// share w_gate's k-blocks, the second half w_up's (w: this wave's matrix at n0);
+// the partial products meet in LDS and are added in wave order.  pads: this
+// block also writes H's pad columns.
+template <int W, int G>
+__device__ __forceinline__ void mid_gateup_pass(float* part, const uint16_t* __restrict__ w, const uint16_t* __restrict__ xp, int r0, int row1, int n0,
+                                   bool pads, int D, int M, int64_t ldh, uint16_t* __restrict__ h, int tid) {
+  constexpr int HW = W / 2;  // waves per matrix
+  constexpr int NC = kCols<uint16_t>, PART = kGroup * NC;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  dec_f32x4 acc[G][8] = {};
+  stream_groups<true, G>(w, M, xp + (int64_t)r0 * D, D, row1 - r0, D, wave % HW, (D + kKB - 1) / kKB, HW, lane, acc);
+#pragma unroll
+  for (int r = 0; r < G; ++r) {
+    const int rg0 = r0 + r * kGroup;
+    if (rg0 >= row1) break;
+    __syncthreads();  // the previous group's sums are read
+    store_partial<uint16_t>(part + wave * PART, acc[r], lane);
+    __syncthreads();
+    for (int v = tid; v < PART / 4; v += W * 64) {
+      const int row = rg0 + v / (NC / 4), c = (v % (NC / 4)) * 4;
+      if (row >= row1) continue;
+      float s[2][4];
+#pragma unroll
+      for (int hf = 0; hf < 2; ++hf) {
+        float4 t = *reinterpret_cast<const float4*>(part + HW * hf * PART + 4 * v);
+#pragma unroll
+        for (int p = 1; p < HW; ++p) {
+          const float4 u = *reinterpret_cast<const float4*>(part + (HW * hf + p) * PART + 4 * v);
+          t.x += u.x; t.y += u.y; t.z += u.z; t.w += u.w;
+        }
+        s[hf][0] = t.x; s[hf][1] = t.y; s[hf][2] = t.z; s[hf][3] = t.w;
+      }
+      float o[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {  // each product rounded to the dtype, as the separate products are
+        const float g = round_to<uint16_t>(s[0][i]), u = round_to<uint16_t>(s[1][i]);
+        o[i] = round_to<uint16_t>(silu_f32(g)) * u;
+      }
+      store4<uint16_t>(h + (int64_t)row * ldh + n0 + c, o[0], o[1], o[2], o[3]);
+    }
+    if (pads && tid < kGroup && rg0 + tid < row1)
+      for (int64_t c = M; c < ldh; ++c) h[(int64_t)(rg0 + tid) * ldh + c] = 0;
+  }
+}
+
+// Y = H w_down for rows r0 .. min(r0 + 16 G, row1) - 1 of one expert, the
+// kCols columns from n0 and the k-blocks kb0 .. kb1 - 1, shared by the block's W
+// waves.  One slice: Y itself; more: fp32 partials [slice][R][D] for
+// decode_reduce_kernel.
+template <int W, int G>
+__device__ __forceinline__ void mid_down_pass(float* part, const uint16_t* __restrict__ w, const uint16_t* __restrict__ h, int r0, int row1, int n0,
+                                 int M, int D, int64_t ldh, int64_t R, int kb0, int kb1, int slice, int slices,
+                                 uint16_t* __restrict__ y, float* __restrict__ ws, int tid) {
+  constexpr int NC = kCols<uint16_t>, PART = kGroup * NC;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  dec_f32x4 acc[G][8] = {};
+  stream_groups<false, G>(w, D, h + (int64_t)r0 * ldh, ldh, row1 - r0, M, kb0 + wave, kb1, W, lane, acc);
+#pragma unroll
+  for (int r = 0; r < G; ++r) {
+    const int rg0 = r0 + r * kGroup;
+    if (rg0 >= row1) break;
+    __syncthreads();
+    store_partial<uint16_t>(part + wave * PART, acc[r], lane);
+    __syncthreads();
+    for (int v = tid; v < PART / 4; v += W * 64) {
+      const int row = rg0 + v / (NC / 4), c = (v % (NC / 4)) * 4;
+      if (row >= row1) continue;
+      float4 t = *reinterpret_cast<const float4*>(part + 4 * v);
+#pragma unroll
+      for (int p = 1; p < W; ++p) {
+        const float4 u = *reinterpret_cast<const float4*>(part + p * PART + 4 * v);
+        t.x += u.x; t.y += u.y; t.z += u.z; t.w += u.w;
+      }
+      if (slices == 1) store4<uint16_t>(y + (int64_t)row * D + n0 + c, t.x, t.y, t.z, t.w);
+      else *reinterpret_cast<float4*>(ws + ((int64_t)slice * R + row) * D + n0 + c) = t;
+    }
+  }
+}
+
+__global__ __launch_bounds__(256, 2) void mid_gateup_kernel(const uint16_t* __restrict__ xp,
+                                                            const uint16_t* __restrict__ w_gate,
+                                                            const uint16_t* __restrict__ w_up,
+                                                            const int32_t* __restrict__ offsets, int E, int D, int M,
+                                                            int64_t ldh, uint16_t* __restrict__ h) {
+  constexpr int NC = kCols<uint16_t>;
+  __shared__ __attribute__((aligned(16))) float part[4 * kGroup * NC];
+  const int tid = threadIdx.x, cols = (M + NC - 1) / NC;
+  MidTile t;
+  if (!mid_tile(offsets, E, cols, tid & 63, t)) return;
+  const int half = __builtin_amdgcn_readfirstlane(tid >> 7), n0 = min(t.col * NC, M - NC);
+  const uint16_t* w = (half ? w_up : w_gate) + (int64_t)t.e * D * M + n0;
+  const bool pads = t.col == cols - 1;
+  if (t.row1 - t.row0 > kRows)
+    mid_gateup_pass<4, kMidRows / kGroup>(part, w, xp, t.row0, t.row1, n0, pads, D, M, ldh, h, tid);
+  else
+    mid_gateup_pass<4, RG>(part, w, xp, t.row0, t.row1, n0, pads, D, M, ldh, h, tid);
+}
+
+__global__ __launch_bounds__(256, 2) void mid_down_kernel(const uint16_t* __restrict__ h,
+                                                          const uint16_t* __restrict__ w_down,
+                                                          const int32_t* __restrict__ offsets, int E, int M, int D,
+                                                          int64_t ldh, int64_t R, int kb_per, uint16_t* __restrict__ y,
+                                                          float* __restrict__ ws) {
+  constexpr int NC = kCols<uint16_t>;
+  __shared__ __attribute__((aligned(16))) float part[4 * kGroup * NC];
+  const int tid = threadIdx.x, slice = (int)blockIdx.y, slices = (int)gridDim.y;
+  MidTile t;
+  if (!mid_tile(offsets, E, (D + NC - 1) / NC, tid & 63, t)) return;
+  const int n0 = min(t.col * NC, D - NC);
+  const int kb0 = slice * kb_per, kb1 = min(kb0 + kb_per, (M + kKB - 1) / kKB);
+  const uint16_t* w = w_down + (int64_t)t.e * M * D + n0;
+  if (t.row1 - t.row0 > kRows)
+    mid_down_pass<4, kMidRows / kGroup>(part, w, h, t.row0, t.row1, n0, M, D, ldh, R, kb0, kb1, slice, slices,
+                                                  y, ws, tid);
+  else
+    mid_down_pass<4, RG>(part, w, h, t.row0, t.row1, n0, M, D, ldh, R, kb0, kb1, slice, slices, y, ws, tid);
+}
+
 // Y = the slices' partials added in slice order, four elements a thread.
 template <typename T>
 __global__ __launch_bounds__(256) void decode_reduce_kernel(const float* __restrict__ ws, int64_t n, int slices,
@@ -313,10 +580,38 @@ void launch_gateup(dim3 grid, hipStream_t s, const void* xp, const void* wg, con
                      (const T*)wu, offsets, (int)D, (int)M, ldh, (T*)h);
 }
 
+template <typename T>
+int launch_reduce(const float* ws, int64_t n, int slices, void* y, hipStream_t s) {
+  if (slices <= 1) return 0;
+  hipLaunchKernelGGL(decode_reduce_kernel<T>, dim3((unsigned)((n / 4 + 255) / 256)), dim3(256), 0, s, ws, n, slices, (T*)y);
+  ABACUS_CHECK_LAUNCH("experts_decode_fwd (reduce)");
+  return 0;
+}
+
+// Rows per expert from which the blocks of 64 rows run (taken for unaligned
+// hidden sizes only).
+bool mid_rows(int64_t R, int64_t E, int dtype) { return dtype == kBF16 && R > 16 * E; }
+
+int launch_mid(const void* xp, const void* wg, const void* wu, const void* wd, const int32_t* offsets, int64_t R, int64_t D,
+               int64_t M, int64_t E, int64_t ldh, void* h, void* y, float* ws, hipStream_t s) {
+  constexpr int NC = kCols<uint16_t>;
+  const int64_t tiles = R / kMidRows + std::min(E, R);  // at most, and whole turns of the 8 XCDs
+  const int64_t t1 = (tiles * ((M + NC - 1) / NC) + 7) / 8 * 8, t2 = (tiles * ((D + NC - 1) / NC) + 7) / 8 * 8;
+  const DownPlan p = plan_down(R, D, M, E, NC);
+  hipLaunchKernelGGL(mid_gateup_kernel, dim3((unsigned)t1), dim3(256), 0, s, (const uint16_t*)xp, (const uint16_t*)wg,
+                     (const uint16_t*)wu, offsets, (int)E, (int)D, (int)M, ldh, (uint16_t*)h);
+  ABACUS_CHECK_LAUNCH("experts_decode_fwd (gate/up)");
+  hipLaunchKernelGGL(mid_down_kernel, dim3((unsigned)t2, (unsigned)p.slices), dim3(256), 0, s, (const uint16_t*)h,
+                     (const uint16_t*)wd, offsets, (int)E, (int)M, (int)D, ldh, R, p.kb_per, (uint16_t*)y, ws);
+  ABACUS_CHECK_LAUNCH("experts_decode_fwd (down)");
+  return launch_reduce<uint16_t>(ws, R * D, p.slices, y, s);
+}
+
 template <typename T, bool NT>
 int launch(const void* xp, const void* wg, const void* wu, const void* wd, const int32_t* offsets, int64_t R, int64_t D,
            int64_t M, int64_t E, int64_t ldh, void* h, void* y, float* ws, hipStream_t s) {
   constexpr int NC = kCols<T>;
+  if (mid_rows(R, E, sizeof(T) == 2 ? kBF16 : kF32)) return launch_mid(xp, wg, wu, wd, offsets, R, D, M, E, ldh, h, y, ws, s);
   // An expert's passes of 32 rows run beside each other, up to four: one expert
   // may hold many of the rows (E 4 D 512 M 1024, 128 tokens top-1: 26 -> 19 us).
   // They are the slowest grid dimension, so that the blocks without rows come
@@ -339,14 +634,17 @@ int launch(const void* xp, const void* wg, const void* wu, const void* wd, const
     hipLaunchKernelGGL((decode_down_kernel<T, 8, NT>), g2, dim3(512), 0, s, (const T*)h, (const T*)wd, offsets, (int)M,
                        (int)D, ldh, R, p.kb_per, p.slices, (T*)y, ws);
   ABACUS_CHECK_LAUNCH("experts_decode_fwd (down)");
-  if (p.slices > 1) {
-    const int64_t n = R * D;
-    hipLaunchKernelGGL(decode_reduce_kernel<T>, dim3((unsigned)((n / 4 + 255) / 256)), dim3(256), 0, s, ws, n, p.slices,
-                       (T*)y);
-    ABACUS_CHECK_LAUNCH("experts_decode_fwd (reduce)");
-  }
-  return 0;
+  return launch_reduce<T>(ws, R * D, p.slices, y, s);
 }
+
+// bf16 hidden sizes that are not whole vectors: the tiles of grouped_gemm.hip
+// need every weight copied to an aligned pitch first, so the weights are streamed as
+// they are up to 128 rows per expert on average.  Eval layer, copies + tiles against
+// this (us): E 64 D 2048 M 1406 top-6, 513 tokens 549 -> 310 (skewed routing 554 -> 332), 1366
+// tokens 617 -> 500; E 8 D 4096 M 14330, 68 tokens 1180 -> 548, 512 tokens 1270 -> 1118, 768 tokens
+// (192 rows per expert) 1359 -> 1392; E 16 D 1024 M 2730, 136 tokens 156 -> 82, 1024 tokens 195 ->
+// 164.  Whole vectors stay with the tiles: E 64 D 2048 M 1408, 512 tokens 276 against 299 here.
+constexpr int kMidMax = 128;
 
 // Shapes taken: up to 16 rows per expert on average in bf16 (E 64 D 2048 M 1408:
 // 12 rows 225 -> 186 us, 24 rows 222 either way, 48 rows 239 -> 387, where most
@@ -356,7 +654,7 @@ bool takes(int64_t R, int64_t D, int64_t M, int64_t E, int dtype) {
   if (dtype != kBF16 && dtype != kF32) return false;
   const int vec = dtype == kBF16 ? 8 : 4, cols = 16 * vec;
   return R >= 1 && E >= 1 && E <= 1024 && D % vec == 0 && D >= cols && M >= cols && D < (1 << 24) && M < (1 << 24) &&
-         R <= (dtype == kBF16 ? 16 : 64) * E;
+         R <= (dtype == kF32 ? 64 : M % vec == 0 ? 16 : kMidMax) * E;
 }
 
 // Weights that reach well past what the 256 MB last-level cache can hold from

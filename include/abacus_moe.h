@@ -130,9 +130,10 @@ int abacus_moe_down_fwd(const void* h_RM, const void* w_down_EMD, const int32_t*
 
 /* Replaces moe.py:78-80 for a small batch without gradients (GPU only): gate,
  * up, silu(gate) * up and the down projection by kernels that stream each
- * touched expert's weights once.  Takes R <= 16 E (bf16) or 64 E (fp32), D a multiple of the 16-byte
- * vector, D and M at least 16 vectors; M may be any such size (the weight rows
- * of M elements need no alignment).  h: (R, ld_h) scratch, ld_h = M rounded up
+ * touched expert's weights once.  Takes R <= 16 E (bf16; 128 E where M is not
+ * whole vectors) or 64 E (fp32), D a multiple of the 16-byte vector, D and M at
+ * least 16 vectors; M may be any such size (the weight rows of M elements need
+ * no alignment).  h: (R, ld_h) scratch, ld_h = M rounded up
  * to whole vectors.  ws: abacus_experts_decode_ws_bytes bytes (-1: the shape is
  * not taken; 0: none needed), the slices of the down projection's reduction. */
 int64_t abacus_experts_decode_ws_bytes(int64_t R, int64_t D, int64_t M, int64_t E, int dtype);
