@@ -33,7 +33,7 @@ import math
 import torch
 
 from . import _lib
-from .moe import MoE, MoEExpertParallel, _rank_and_world_size
+from .moe import MoE, MoEExpertParallel, _contig, _rank_and_world_size
 
 __all__ = [
     "Embedding",
@@ -439,7 +439,7 @@ class _AttentionFunction(torch.autograd.Function):
         dws = [None, None, None]
         if needs[0]:
             w_D3 = torch.empty(D, 3 * HK, dtype=q.dtype, device=dev)
-            w_c = [w.contiguous() for w in (w_q, w_k, w_v)]
+            w_c = [_contig(w) for w in (w_q, w_k, w_v)]  # (views into a flat buffer may start at any element)
             _lib.call("abacus_join3", *map(_lib.ptr, w_c), D, col, _lib.ptr(w_D3), s)
             dx = (joint @ w_D3.t()).view(B, L, D)
         if any(needs[1:4]):
