@@ -88,6 +88,9 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "abacus_qk_norm_rope_fwd": (_I, [_P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _F, _I, _P, _P, _P, _P]),
     "abacus_qk_norm_rope_bwd": (_I, [_P, _P, _P, _P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _I, _P, _P, _I64, _P,
                                      _P, _P, _I64, _P]),
+    "abacus_token_wgrad_ws_bytes": (_I64, [_I64, _I64, _I64]),
+    "abacus_token_wgrad_pays": (_I64, [_I64, _I64, _I64]),
+    "abacus_token_wgrad": (_I, [_P, _P, _I64, _I64, _I64, _I, _P, _P, _P, _P, _I64, _P]),
     "abacus_join3": (_I, [_P, _P, _P, _I64, _I64, _P, _P]),
     "abacus_split3": (_I, [_P, _I64, _I64, _P, _P, _P, _P]),
     "abacus_cross_entropy_fwd": (_I, [_P, _P, _I64, _I64, _I64, _I, _P, _P, _P]),

@@ -39,6 +39,7 @@ enum GemmKind : int {
   kGateUpDgrad = 3,
   kDownWgrad = 4,
   kGateUpWgrad = 5,
+  kTokenWgrad = 6,  // A^T B of two token-major matrices, sliced over the tokens
 };
 
 template <int KIND> struct KindTraits;
@@ -52,6 +53,7 @@ template <> struct KindTraits<kDownDgrad> { static constexpr bool A_MC = false, 
 template <> struct KindTraits<kGateUpDgrad> { static constexpr bool A_MC = false, B_NC = false, DUAL_B = false, DUAL_K = true, WGRAD = false; };
 template <> struct KindTraits<kDownWgrad> { static constexpr bool A_MC = true, B_NC = true, DUAL_B = false, DUAL_K = false, WGRAD = true; };
 template <> struct KindTraits<kGateUpWgrad> { static constexpr bool A_MC = true, B_NC = true, DUAL_B = true, DUAL_K = false, WGRAD = true; };
+template <> struct KindTraits<kTokenWgrad> { static constexpr bool A_MC = true, B_NC = true, DUAL_B = false, DUAL_K = false, WGRAD = true; };
 
 // Tile counters of a persistent weight-gradient launch (caller workspace).
 constexpr int kTileCtrInts = ABACUS_MOE_TILE_CTR_INTS;
@@ -96,6 +98,7 @@ struct GemmArgs {
   // epilogue): every tile runs as ksplit slices of the reduction, each writing
   // its rows of an fp32 (ksplit, R, Ndim) workspace, which rows_reduce_kernel
   // adds in slice order.  <= 1: none.
+  // (kTokenWgrad: E slices of `ksplit` tokens each, of Kdim in all.)
   int ksplit;
   float* ksplit_ws;
   // Pipelined kernel, row-grouped kinds: nonzero when expert remainders of at
@@ -944,6 +947,14 @@ __device__ __attribute__((always_inline)) inline void gemm_tile(const GemmArgs& 
     if (!block_to_row_tile(g, b, total, r, part, kslice)) return;
     row_tile(r, mt_real, g.tiles_n, tl.mt, tl.nt);
     if (part >= 0) slot = r - total / g.split_cus * g.split_cus;
+  } else if constexpr (KIND == kTokenWgrad) {
+    // (slice, row tile, column tile), an equal contiguous share to each XCD
+    const int per_slice = g.tiles_m * g.tiles_n, total = g.E * per_slice, per = (total + 7) / 8;
+    const int L = (b & 7) * per + (b >> 3);
+    if ((b >> 3) >= per || L >= total) return;
+    tl.e = L / per_slice;
+    tl.mt = L % per_slice / g.tiles_n;
+    tl.nt = L % g.tiles_n;
   } else {
     // per-expert tile space (E x tiles_m x tiles_n), XCD-contiguous
     // (fp32: the groups dealt to the XCDs in turn; its blocks are not
@@ -961,9 +972,9 @@ __device__ __attribute__((always_inline)) inline void gemm_tile(const GemmArgs& 
     row0 = tl.mt * BM;
     if (e >= g.E || row0 >= g.Mdim) return;
     row_end = g.Mdim;
-    k_len = g.offsets[e + 1] - g.offsets[e];
+    k_len = KIND == kTokenWgrad ? min(g.ksplit, g.Kdim - e * g.ksplit) : g.offsets[e + 1] - g.offsets[e];
   }
-  const int seg0 = KT::WGRAD ? g.offsets[e] : 0;
+  const int seg0 = KIND == kTokenWgrad ? e * g.ksplit : KT::WGRAD ? g.offsets[e] : 0;
 
   const T* A0 = (const T*)g.a0;
   const T* A1 = (const T*)g.a1;
@@ -1161,9 +1172,9 @@ __device__ __attribute__((always_inline)) inline void gemm_tile(const GemmArgs& 
               make_float4(acc[i][j][4 * gq], acc[i][j][4 * gq + 1], acc[i][j][4 * gq + 2], acc[i][j][4 * gq + 3]);
     return;
   }
-  if constexpr (KIND == kDownFwd || KIND == kGateUpDgrad) {
-    if (g.ksplit > 1) {  // a slice of the whole launch: its fp32 rows, for rows_reduce_kernel
-      float* ws = g.ksplit_ws + (int64_t)kslice * g.Mdim * g.Ndim;
+  if constexpr (KIND == kDownFwd || KIND == kGateUpDgrad || KIND == kTokenWgrad) {
+    if (KIND == kTokenWgrad || g.ksplit > 1) {  // a slice of the whole launch: its fp32 rows, for the adding pass
+      float* ws = g.ksplit_ws + (int64_t)(KIND == kTokenWgrad ? e : kslice) * g.Mdim * g.Ndim;
       const int rl = lane & 31, ch = 4 * (lane >> 5);
 #pragma unroll
       for (int i = 0; i < FM; ++i) {
@@ -1771,6 +1782,41 @@ __global__ __launch_bounds__(256) void rows_reduce_kernel(const float* __restric
     w.y = pack_bf16x2(t.z, t.w);
     *reinterpret_cast<uint2*>(out + i) = w;
   }
+}
+
+// A weight gradient of a plain projection, C = A^T B over T tokens (A (T, Mdim), B
+// (T, Ndim), bf16).  What bounds it is that C has few tiles (16 of 256 x 256 for
+// 1024 x 1024, on 256 CUs) with the whole batch as their reduction, so the tokens are cut into
+// slices and every (slice, tile) is a block.  The slices' fp32 products meet in
+// token_reduce_kernel.
+__global__ __launch_bounds__(NT, 1) void token_wgrad_kernel(GemmArgs g) {
+  __shared__ __attribute__((aligned(1024))) char lds[LDS_ALLOC];
+  gemm_tile<uint16_t, kTokenWgrad, BM>(g, (int)blockIdx.x, (int)gridDim.x, lds, nullptr);
+}
+
+// C's slices added in slice order and rounded once, four elements a thread; C's
+// columns are cut into equal parts (1 or 3) that go to tensors of their own.
+__global__ __launch_bounds__(256) void token_reduce_kernel(const float* __restrict__ ws, int64_t n, int N, int slices,
+                                                           int part_cols, uint16_t* __restrict__ c0,
+                                                           uint16_t* __restrict__ c1, uint16_t* __restrict__ c2) {
+  const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
+  if (i >= n) return;
+  float4 t = *reinterpret_cast<const float4*>(ws + i);
+#pragma unroll 4
+  for (int s = 1; s < slices; ++s) {
+    const float4 u = *reinterpret_cast<const float4*>(ws + s * n + i);
+    t.x += u.x;
+    t.y += u.y;
+    t.z += u.z;
+    t.w += u.w;
+  }
+  const uint32_t row = (uint32_t)((uint32_t)(i >> 2) / (uint32_t)(N >> 2)), col = (uint32_t)(i - (int64_t)row * N);
+  const uint32_t part = col / (uint32_t)part_cols;
+  uint16_t* c = part == 0 ? c0 : part == 1 ? c1 : c2;
+  uint2 w;
+  w.x = pack_bf16x2(t.x, t.y);
+  w.y = pack_bf16x2(t.z, t.w);
+  *reinterpret_cast<uint2*>(c + (int64_t)row * part_cols + (col - part * part_cols)) = w;
 }
 
 // Adds the slices of each split tail tile in slice order and writes the tile
@@ -2579,3 +2625,86 @@ int abacus_experts_gateup_bwd(const void* dgate, const void* dup, const void* w_
 }
 
 }  // extern "C"
+
+namespace {
+
+// Slices of whole k-tiles: the count that minimises an estimate of the launch, 1.7 us
+// per k-tile and 8 per block (as row_slices) in rounds over the CUs, plus the
+// partials written and read at 4 TB/s.
+struct TokenPlan {
+  int tiles_m, tiles_n, rows, slices;
+};
+TokenPlan plan_token_wgrad(int64_t T, int64_t M, int64_t N) {
+  const int64_t tm = (M + pipe::BM - 1) / pipe::BM, tn = (N + pipe::BN - 1) / pipe::BN, kt = (T + 63) / 64;
+  int64_t best = 1;
+  double best_us = 0.0;
+  for (int64_t s = 1; s <= std::min<int64_t>(16, kt); ++s) {
+    const double rounds = (double)((tm * tn * s + cu_count() - 1) / cu_count());
+    const double us = rounds * (1.7 * (double)((kt + s - 1) / s) + 8.0) + (double)(s * M * N) * 8.0 / 4e6;
+    if (s == 1 || us < best_us) {
+      best = s;
+      best_us = us;
+    }
+  }
+  const int64_t rows = (kt + best - 1) / best * 64;
+  return {(int)tm, (int)tn, (int)rows, (int)((T + rows - 1) / rows)};
+}
+
+bool token_wgrad_takes(int64_t T, int64_t M, int64_t N) {
+  return T >= 1 && T < (1ll << 24) && M < (1ll << 24) && N < (1ll << 24) && M >= 8 && N >= 8 && M % 8 == 0 && N % 8 == 0 && M * N < (1ll << 31);
+}
+
+}  // namespace
+
+// Where it is faster than the library's product: from about 4096 tokens, as long as C's
+// tiles leave CUs for a second slice.  Measured (us, library -> this, D x N outputs): 1024 x
+// 3072 in three parts, T 3072 40 -> 41, 4500 56 -> 49, 8192 85 -> 67, 12288 122 -> 87; 1024 x 1024,
+// T 3072 23 -> 31, 4500 33 -> 32, 8192 53 -> 39, 12288 77 -> 45; 512 x 512, T 4500 33 -> 28, 12288 76
+// -> 35; 2048 x 2048 (64 tiles), T 4500 54 -> 55, 6000 71 -> 64; 1536 x 4608 (108 tiles), T 8192 125 -> 118;
+// 2048 x 6144 (192 tiles, one slice), T 8192 195 -> 207.
+extern "C" int64_t abacus_token_wgrad_pays(int64_t T, int64_t M, int64_t N) {
+  return token_wgrad_takes(T, M, N) && T >= 4096 && plan_token_wgrad(T, M, N).slices >= 2 ? 1 : 0;
+}
+
+extern "C" int64_t abacus_token_wgrad_ws_bytes(int64_t T, int64_t M, int64_t N) {
+  if (!token_wgrad_takes(T, M, N)) return -1;
+  return plan_token_wgrad(T, M, N).slices * M * N * 4;
+}
+
+extern "C" int abacus_token_wgrad(const void* a_TM, const void* b_TN, int64_t T, int64_t M, int64_t N, int parts, void* c0,
+                                  void* c1, void* c2, float* ws, int64_t ws_bytes, void* stream) {
+  ABACUS_CHECK_ARG(token_wgrad_takes(T, M, N), "token_wgrad: T %lld, M %lld, N %lld not taken", (long long)T, (long long)M,
+                   (long long)N);
+  ABACUS_CHECK_ARG((parts == 1 || parts == 3) && N % (4 * parts) == 0, "token_wgrad: %d parts of %lld columns", parts,
+                   (long long)N);
+  ABACUS_CHECK_ARG(a_TM && b_TN && c0 && ws && (parts == 1 || (c1 && c2)), "token_wgrad: null pointer");
+  ABACUS_CHECK_ARG(((uintptr_t)a_TM | (uintptr_t)b_TN | (uintptr_t)ws) % 16 == 0 &&
+                       ((uintptr_t)c0 | (uintptr_t)c1 | (uintptr_t)c2) % 8 == 0,
+                   "token_wgrad: misaligned tensor");
+  const TokenPlan p = plan_token_wgrad(T, M, N);
+  ABACUS_CHECK_ARG(ws_bytes >= p.slices * M * N * 4, "token_wgrad: workspace of %lld bytes, need %lld", (long long)ws_bytes,
+                   (long long)(p.slices * M * N * 4));
+  const int64_t blocks = ((int64_t)p.slices * p.tiles_m * p.tiles_n + 7) / 8 * 8;
+  ABACUS_CHECK_ARG(blocks < (1ll << 31), "token_wgrad: tile grid too large");
+  GemmArgs g{};
+  g.a0 = a_TM;
+  g.b0 = b_TN;
+  g.lda = M;
+  g.ldb = N;
+  g.E = p.slices;
+  g.Mdim = (int)M;
+  g.Ndim = (int)N;
+  g.Kdim = (int)T;
+  g.tiles_m = p.tiles_m;
+  g.tiles_n = p.tiles_n;
+  g.ksplit = p.rows;
+  g.ksplit_ws = ws;
+  hipStream_t s = (hipStream_t)stream;
+  hipLaunchKernelGGL(pipe::token_wgrad_kernel, dim3((unsigned)blocks), dim3(pipe::NT), 0, s, g);
+  ABACUS_CHECK_LAUNCH("token_wgrad");
+  const int64_t n = M * N;
+  hipLaunchKernelGGL(pipe::token_reduce_kernel, dim3((unsigned)((n / 4 + 255) / 256)), dim3(256), 0, s, ws, n, (int)N,
+                     p.slices, (int)(N / parts), (uint16_t*)c0, (uint16_t*)c1, (uint16_t*)c2);
+  ABACUS_CHECK_LAUNCH("token_wgrad (add)");
+  return 0;
+}

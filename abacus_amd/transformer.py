@@ -342,6 +342,42 @@ class _FlashAttentionFunction(torch.autograd.Function):
 flash_attention_enabled = True
 
 
+def _token_wgrad(a_TM: torch.Tensor, b_TN: torch.Tensor, parts: int) -> list[torch.Tensor] | None:
+    """a^T b over the tokens, its columns in `parts` tensors (M, N / parts), by the sliced HIP kernel;
+    None where the library's product is to form it (few tokens, wide outputs, other types)."""
+    T, M = a_TM.shape
+    N = b_TN.shape[1]
+    if not (a_TM.is_cuda and a_TM.dtype == b_TN.dtype == torch.bfloat16 and N % (4 * parts) == 0
+            and all(t.is_contiguous() and t.data_ptr() % 16 == 0 for t in (a_TM, b_TN))
+            and _lib.query("abacus_token_wgrad_pays", T, M, N)):
+        return None
+    nbytes = _lib.query("abacus_token_wgrad_ws_bytes", T, M, N)
+    ws = torch.empty(nbytes // 4, dtype=torch.float32, device=a_TM.device)
+    out = [torch.empty(M, N // parts, dtype=a_TM.dtype, device=a_TM.device) for _ in range(parts)]
+    _lib.call("abacus_token_wgrad", _lib.ptr(a_TM), _lib.ptr(b_TN), T, M, N, parts,
+              *map(_lib.ptr, out + [None] * (3 - parts)), _lib.ptr(ws), nbytes, _lib.stream_of(a_TM.device))
+    return out
+
+
+class _OutProjection(torch.autograd.Function):
+    """o_TN @ w_ND, its weight gradient by _token_wgrad where that pays."""
+
+    @staticmethod
+    def forward(ctx, o_TN, w_ND):
+        ctx.save_for_backward(o_TN, w_ND)
+        return o_TN @ w_ND
+
+    @staticmethod
+    def backward(ctx, dy_TD):
+        o_TN, w_ND = ctx.saved_tensors
+        d_o = dy_TD @ w_ND.t() if ctx.needs_input_grad[0] else None
+        dw = None
+        if ctx.needs_input_grad[1]:
+            own = _token_wgrad(o_TN, dy_TD.contiguous(), 1)
+            dw = o_TN.t() @ dy_TD if own is None else own[0]
+        return d_o, dw
+
+
 class _QKVProjection(torch.autograd.Function):
     """q, k, v = x W_q, x W_k, x W_v (attention.py:129-131) with one backward for the three.
 
@@ -378,9 +414,11 @@ class _QKVProjection(torch.autograd.Function):
             w_D3 = torch.cat([w.reshape(D, HK) for w in (w_q, w_k, w_v)], dim=1)
             dx = (g_T3 @ w_D3.t()).view(B, L, D)
         if any(ctx.needs_input_grad[1:]):
-            dw_D3 = x_TD.t() @ g_T3
-            dwq, dwk, dwv = (dw_D3[:, i * HK:(i + 1) * HK].contiguous().view(D, H, K) if ctx.needs_input_grad[1 + i]
-                             else None for i in range(3))
+            dws = _token_wgrad(x_TD, g_T3, 3)
+            if dws is None:
+                dw_D3 = x_TD.t() @ g_T3
+                dws = [dw_D3[:, i * HK:(i + 1) * HK].contiguous() for i in range(3)]
+            dwq, dwk, dwv = (g.view(D, H, K) if need else None for g, need in zip(dws, ctx.needs_input_grad[1:]))
         return dx, dwq, dwk, dwv
 
 
@@ -443,10 +481,12 @@ class _AttentionFunction(torch.autograd.Function):
             _lib.call("abacus_join3", *map(_lib.ptr, w_c), D, col, _lib.ptr(w_D3), s)
             dx = (joint @ w_D3.t()).view(B, L, D)
         if any(needs[1:4]):
-            dw_D3 = x_TD.t() @ joint
-            dws = [torch.empty(D, H, K, dtype=q.dtype, device=dev) for _ in range(3)]
-            _lib.call("abacus_split3", _lib.ptr(dw_D3), D, col, *map(_lib.ptr, dws), s)
-            dws = [g if need else None for g, need in zip(dws, needs[1:4])]
+            dws = _token_wgrad(x_TD, joint, 3)
+            if dws is None:
+                dw_D3 = x_TD.t() @ joint
+                dws = [torch.empty(D, HK, dtype=q.dtype, device=dev) for _ in range(3)]
+                _lib.call("abacus_split3", _lib.ptr(dw_D3), D, col, *map(_lib.ptr, dws), s)
+            dws = [g.view(D, H, K) if need else None for g, need in zip(dws, needs[1:4])]
         return (dx, *dws, dgamma_q if needs[4] else None, dgamma_k if needs[5] else None, None, None, None)
 
 
@@ -514,6 +554,14 @@ class MultiHeadAttention(torch.nn.Module):
         self.q_norm = RMSNorm(head_dim, sync_grads=sync_qk)
         self.k_norm = RMSNorm(head_dim, sync_grads=sync_qk)
 
+    def _out_projection(self, out_BLHK: torch.Tensor) -> torch.Tensor:
+        """The HIP attention's output through w_o (its type and device checked by the product)."""
+        B, L, H, K = out_BLHK.shape
+        w_ND = self.w_o_HKD.reshape(H * K, self.dim)
+        if torch.is_autocast_enabled():
+            return out_BLHK.reshape(B, L, H * K) @ w_ND
+        return _OutProjection.apply(out_BLHK.reshape(B * L, H * K), w_ND).view(B, L, self.dim)
+
     def forward(self, x_BLD: torch.Tensor, rotary: Rotary | None = None) -> torch.Tensor:
         if self.context_parallel or self.world_size > 1:
             _single_process("attention parallelism")
@@ -523,7 +571,7 @@ class MultiHeadAttention(torch.nn.Module):
         if _joint_ok(x_BLD, weights, gammas, rotary):
             cos, sin = rotary(x_BLD, seq_dim=1)  # (1, 1, L, K)
             out = _AttentionFunction.apply(x_BLD, *weights, *gammas, cos.reshape(L, K), sin.reshape(L, K), 1e-5)
-            return out.reshape(B, L, H * K) @ self.w_o_HKD.reshape(H * K, self.dim)
+            return self._out_projection(out)
         q_heads, k_heads, v_heads = _QKVProjection.apply(x_BLD, self.w_q_DHK, self.w_k_DHK, self.w_v_DHK)
         cos = sin = None
         if rotary is not None:
@@ -537,7 +585,7 @@ class MultiHeadAttention(torch.nn.Module):
             if flash_attention_enabled and _flash_ok(q_blhk, k_blhk, v_heads):
                 # the HIP flash kernels on the (B, L, H, K) layout: no permuted copies
                 out = _FlashAttentionFunction.apply(q_blhk, k_blhk, v_heads)
-                return out.reshape(B, L, H * K) @ self.w_o_HKD.reshape(H * K, self.dim)
+                return self._out_projection(out)
             q, k = q_blhk.permute(0, 2, 1, 3), k_blhk.permute(0, 2, 1, 3)
         else:
             q = self.q_norm(q_heads).permute(0, 2, 1, 3)  # (B, H, L, K)

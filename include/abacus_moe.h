@@ -319,6 +319,16 @@ int abacus_qk_norm_rope_bwd(const void* dy_q, const void* dy_k, const void* q, c
                             int64_t token_stride, void* dgamma_q, void* dgamma_k, float* ws, int64_t ws_bytes,
                             void* stream);
 
+/* C = A^T B over T tokens (the weight gradient of a projection), A (T, M) and B
+ * (T, N) bf16, M and N multiples of 8; fp32 sums, rounded once.  parts 1: C (M, N)
+ * in c0; 3: C's columns in three equal parts, c0, c1, c2 (M, N / 3).  ws:
+ * abacus_token_wgrad_ws_bytes bytes (-1: the shape is not taken).
+ * abacus_token_wgrad_pays: 1 where this is faster than a library product. */
+int64_t abacus_token_wgrad_pays(int64_t T, int64_t M, int64_t N);
+int64_t abacus_token_wgrad_ws_bytes(int64_t T, int64_t M, int64_t N);
+int abacus_token_wgrad(const void* a_TM, const void* b_TN, int64_t T, int64_t M, int64_t N, int parts, void* c0, void* c1,
+                       void* c2, float* ws, int64_t ws_bytes, void* stream);
+
 /* out = [a b c] row by row, and the reverse: rows of row_bytes (whole 16-byte
  * vectors) in a, b and c, of three times that in the joint matrix. */
 int abacus_join3(const void* a, const void* b, const void* c, int64_t rows, int64_t row_bytes, void* out, void* stream);
