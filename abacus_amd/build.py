@@ -27,8 +27,8 @@ HOST_LIB_NAME = "libabacus_moe_host.so"
 HOST_FLAGS = ["-O3", "-std=c++17", "-fPIC", "-fopenmp", "-shared", "-Wall", "-Wno-unused-parameter"]
 ARCH = "gfx950"
 
-# -packed-fp32-ops: never emit v_pk_{add,mul,fma}_f32 (see DESIGN notes on
-# packed fp32); hipcc's host pass warns that it does not know the feature.
+# -packed-fp32-ops: never emit v_pk_{add,mul,fma}_f32 (some of their forms have
+# given wrong results); hipcc's host pass warns that it does not know the feature.
 HIPCC_FLAGS = [
     f"--offload-arch={ARCH}",
     "-O3",
