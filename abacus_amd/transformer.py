@@ -344,10 +344,11 @@ flash_attention_enabled = True
 
 def _token_wgrad(a_TM: torch.Tensor, b_TN: torch.Tensor, parts: int) -> list[torch.Tensor] | None:
     """a^T b over the tokens, its columns in `parts` tensors (M, N / parts), by the sliced HIP kernel;
-    None where the library's product is to form it (few tokens, wide outputs, other types)."""
+    None where the library's product is to form it (few tokens, wide outputs, other types, or a
+    backward that is to be differentiated again, which the kernel is not)."""
     T, M = a_TM.shape
     N = b_TN.shape[1]
-    if not (a_TM.is_cuda and a_TM.dtype == b_TN.dtype == torch.bfloat16 and N % (4 * parts) == 0
+    if not (not torch.is_grad_enabled() and a_TM.is_cuda and a_TM.dtype == b_TN.dtype == torch.bfloat16 and N % (4 * parts) == 0
             and all(t.is_contiguous() and t.data_ptr() % 16 == 0 for t in (a_TM, b_TN))
             and _lib.query("abacus_token_wgrad_pays", T, M, N)):
         return None

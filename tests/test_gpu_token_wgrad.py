@@ -53,3 +53,14 @@ def test_attention_block_weight_gradients(monkeypatch):
     monkeypatch.setattr(tr, "_token_wgrad", lambda *_: None)
     for name, want in grads().items():
         assert float((own[name] - want).norm()) <= 2 ** -7 * float(want.norm()), name  # a bf16 rounding on each side
+
+
+def test_second_derivative_of_the_output_projection():
+    """A backward with create_graph keeps the differentiable product."""
+    o, dy = (torch.randn(4096, 64, device="cuda").to(torch.bfloat16).requires_grad_() for _ in range(2))
+    w = torch.randn(64, 64, device="cuda").to(torch.bfloat16).requires_grad_()
+    assert _lib.query("abacus_token_wgrad_pays", 4096, 64, 64) == 1
+    (dw,) = torch.autograd.grad(tr._OutProjection.apply(o, w), w, dy, create_graph=True)
+    (got,) = torch.autograd.grad(dw.float().sum(), dy)
+    want = o.detach().float().sum(dim=1, keepdim=True).expand(4096, 64)  # d/d dy of sum(o^T dy)
+    assert float((got.float() - want).norm()) <= 2 ** -8 * float(want.norm())
