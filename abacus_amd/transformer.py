@@ -108,10 +108,16 @@ def apply_rotary_pos_emb(q, k, cos, sin):
     return (q * cos) + (rotate_half(q) * sin), (k * cos) + (rotate_half(k) * sin)
 
 
+def _of_kind(x: torch.Tensor, *tensors: torch.Tensor) -> bool:
+    """Whether the tensors have x's dtype and device.  Rotary's tables may not: they are cached by
+    length alone, so a module cast or moved after a forward hands on the old ones."""
+    return all(t.dtype == x.dtype and t.device == x.device for t in tensors)
+
+
 def _fused_norm_ok(x: torch.Tensor, gamma: torch.Tensor) -> bool:
-    """The HIP RMSNorm takes x: GPU, fp32/bf16, gamma of the same dtype, and rows whose
+    """The HIP RMSNorm takes x: GPU, fp32/bf16, gamma of the same dtype and device, and rows whose
     16-byte vectors split evenly over a power-of-two number of lanes (at most 8 each)."""
-    if not (x.is_cuda and x.dtype in (torch.float32, torch.bfloat16) and gamma.dtype == x.dtype):
+    if not (x.is_cuda and x.dtype in (torch.float32, torch.bfloat16) and _of_kind(x, gamma)):
         return False
     D = x.shape[-1]
     epv = 8 if x.dtype == torch.bfloat16 else 4
@@ -157,8 +163,8 @@ class _RMSNormFunction(torch.autograd.Function):
 
 def _fused_rope_ok(x: torch.Tensor, gamma: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> bool:
     """The HIP norm + rotary kernel takes what the fused norm takes, with cos/sin of
-    x's dtype and a row of 2..64 16-byte vectors, a power of two (one per lane)."""
-    if not (_fused_norm_ok(x, gamma) and cos.dtype == x.dtype and sin.dtype == x.dtype):
+    x's dtype and device and a row of 2..64 16-byte vectors, a power of two (one per lane)."""
+    if not (_fused_norm_ok(x, gamma) and _of_kind(x, cos, sin)):
         return False
     nvec = x.shape[-1] // (8 if x.dtype == torch.bfloat16 else 4)
     return 2 <= nvec <= 64 and nvec & (nvec - 1) == 0
@@ -494,11 +500,12 @@ class _AttentionFunction(torch.autograd.Function):
 def _joint_ok(x: torch.Tensor, weights, gammas, rotary) -> bool:
     """_AttentionFunction takes what the flash kernels and the norm + rotary kernel take (bf16 on the
     GPU, heads of 64 or 128), with this module's own Rotary, outside autocast.  While a KernelTimer
-    wants each entry point by its name, the separate nodes run."""
+    wants each entry point by its name, the separate nodes run.  (The tables that rotary returns
+    are looked at after the call.)"""
     H, K = weights[0].shape[1:]
     return (flash_attention_enabled and not _lib.timing() and x.is_cuda and x.dim() == 3 and x.numel() > 0
             and x.dtype == torch.bfloat16 and K in (64, 128) and x.shape[0] <= 65535 and H <= 65535 and H * K < 1 << 24
-            and all(t.dtype == x.dtype and t.device == x.device for t in (*weights, *gammas))
+            and _of_kind(x, *weights, *gammas)
             and type(rotary) is Rotary and not rotary._forward_hooks and not rotary._forward_pre_hooks
             and rotary.inv_freq.dtype == x.dtype and rotary.inv_freq.shape[0] * 2 == K
             and not torch.is_autocast_enabled())
@@ -571,8 +578,9 @@ class MultiHeadAttention(torch.nn.Module):
         weights, gammas = (self.w_q_DHK, self.w_k_DHK, self.w_v_DHK), (self.q_norm.w_gamma_D, self.k_norm.w_gamma_D)
         if _joint_ok(x_BLD, weights, gammas, rotary):
             cos, sin = rotary(x_BLD, seq_dim=1)  # (1, 1, L, K)
-            out = _AttentionFunction.apply(x_BLD, *weights, *gammas, cos.reshape(L, K), sin.reshape(L, K), 1e-5)
-            return self._out_projection(out)
+            if _of_kind(x_BLD, cos, sin):
+                out = _AttentionFunction.apply(x_BLD, *weights, *gammas, cos.reshape(L, K), sin.reshape(L, K), 1e-5)
+                return self._out_projection(out)
         q_heads, k_heads, v_heads = _QKVProjection.apply(x_BLD, self.w_q_DHK, self.w_k_DHK, self.w_v_DHK)
         cos = sin = None
         if rotary is not None:

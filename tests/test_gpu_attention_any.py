@@ -122,6 +122,19 @@ def test_joint_node_takes_weights_at_any_element():
         assert float((a.double() - b.double()).norm()) <= 1.2e-2 * float(b.double().norm())
 
 
+def test_block_cast_after_a_forward_refuses_the_old_tables():
+    """Rotary's tables of an fp32 forward at this length do not fit the block once it is cast to bf16."""
+    torch.manual_seed(10)
+    attn, rot = tr.MultiHeadAttention(64, 1, 64).cuda(), tr.Rotary(64).cuda()
+    x = torch.randn(2, 70, 64, device="cuda")
+    with torch.no_grad():
+        attn(x, rot)
+        attn, rot = attn.to(torch.bfloat16), rot.to(torch.bfloat16)
+        with pytest.raises(RuntimeError):
+            attn(x.to(torch.bfloat16), rot)
+        assert torch.isfinite(attn(x[:, :69].to(torch.bfloat16), rot).float()).all()
+
+
 def test_any_rejects_head_dims():
     q = torch.zeros(1, 100, 1, 32, dtype=torch.bfloat16, device="cuda")
     with pytest.raises(RuntimeError, match="head_dim"):
