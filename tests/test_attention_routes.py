@@ -1,6 +1,8 @@
 """Which attention inputs reach the GPU kernels, decided on the host: checked without a GPU on fake CUDA tensors, with
 the library's calls recorded instead of made."""
 
+import contextlib
+
 import pytest
 import torch
 from torch._subclasses.fake_tensor import FakeTensorMode
@@ -40,10 +42,11 @@ def test_tables_of_the_inputs_type_take_the_joint_node(calls):
 
 @pytest.mark.parametrize("stale", [dict(dtype=torch.float32), dict(device="cpu")])
 def test_tables_cached_for_another_type_or_device_are_refused(calls, stale):
-    """Rotary caches its tables by length alone, so a module cast or moved afterwards hands on the old ones."""
+    """Rotary caches its tables by length alone, so a module cast or moved afterwards hands on the old ones: no kernel
+    reads them (torch's products refuse them on the GPU; fake tensors let a type through)."""
     attn, rot = _block()
     rot(_x(), seq_dim=1)
     rot.cos_cached, rot.sin_cached = rot.cos_cached.to(**stale), rot.sin_cached.to(**stale)
-    with pytest.raises(RuntimeError):
+    with contextlib.suppress(RuntimeError):
         attn(_x(), rot)
     assert not any("rope" in name for name in calls)
