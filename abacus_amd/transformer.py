@@ -497,15 +497,15 @@ class _AttentionFunction(torch.autograd.Function):
         return (dx, *dws, dgamma_q if needs[4] else None, dgamma_k if needs[5] else None, None, None, None)
 
 
-def _joint_ok(x: torch.Tensor, weights, gammas, rotary) -> bool:
+def _joint_ok(x: torch.Tensor, weights, rotary) -> bool:
     """_AttentionFunction takes what the flash kernels and the norm + rotary kernel take (bf16 on the
     GPU, heads of 64 or 128), with this module's own Rotary, outside autocast.  While a KernelTimer
-    wants each entry point by its name, the separate nodes run.  (The tables that rotary returns
-    are looked at after the call.)"""
+    wants each entry point by its name, the separate nodes run.  (The norms' weights and the tables
+    that rotary returns are looked at by the caller.)"""
     H, K = weights[0].shape[1:]
     return (flash_attention_enabled and not _lib.timing() and x.is_cuda and x.dim() == 3 and x.numel() > 0
             and x.dtype == torch.bfloat16 and K in (64, 128) and x.shape[0] <= 65535 and H <= 65535 and H * K < 1 << 24
-            and _of_kind(x, *weights, *gammas)
+            and _of_kind(x, *weights)
             and type(rotary) is Rotary and not rotary._forward_hooks and not rotary._forward_pre_hooks
             and rotary.inv_freq.dtype == x.dtype and rotary.inv_freq.shape[0] * 2 == K
             and not torch.is_autocast_enabled())
@@ -575,10 +575,11 @@ class MultiHeadAttention(torch.nn.Module):
             _single_process("attention parallelism")
         B, L, _ = x_BLD.shape
         H, K = self.local_heads, self.head_dim
-        weights, gammas = (self.w_q_DHK, self.w_k_DHK, self.w_v_DHK), (self.q_norm.w_gamma_D, self.k_norm.w_gamma_D)
-        if _joint_ok(x_BLD, weights, gammas, rotary):
+        weights = (self.w_q_DHK, self.w_k_DHK, self.w_v_DHK)
+        if rotary is not None and _joint_ok(x_BLD, weights, rotary):
+            gammas = (self.q_norm.w_gamma_D, self.k_norm.w_gamma_D)
             cos, sin = rotary(x_BLD, seq_dim=1)  # (1, 1, L, K)
-            if _of_kind(x_BLD, cos, sin):
+            if _of_kind(x_BLD, *gammas, cos, sin):
                 out = _AttentionFunction.apply(x_BLD, *weights, *gammas, cos.reshape(L, K), sin.reshape(L, K), 1e-5)
                 return self._out_projection(out)
         q_heads, k_heads, v_heads = _QKVProjection.apply(x_BLD, self.w_q_DHK, self.w_k_DHK, self.w_v_DHK)

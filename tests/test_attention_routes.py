@@ -50,3 +50,10 @@ def test_tables_cached_for_another_type_or_device_are_refused(calls, stale):
     with contextlib.suppress(RuntimeError):
         attn(_x(), rot)
     assert not any("rope" in name for name in calls)
+
+
+def test_block_without_rotary_takes_any_norms():
+    """Without a rotary embedding the q and k norms are only called: any module will do."""
+    attn = tr.MultiHeadAttention(16, 2, 8)
+    attn.q_norm, attn.k_norm = torch.nn.Identity(), torch.nn.LayerNorm(8)
+    assert attn(torch.randn(2, 5, 16)).shape == (2, 5, 16)
