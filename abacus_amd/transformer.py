@@ -115,9 +115,10 @@ def _of_kind(x: torch.Tensor, *tensors: torch.Tensor) -> bool:
 
 
 def _fused_norm_ok(x: torch.Tensor, gamma: torch.Tensor) -> bool:
-    """The HIP RMSNorm takes x: GPU, fp32/bf16, gamma of the same dtype and device, and rows whose
-    16-byte vectors split evenly over a power-of-two number of lanes (at most 8 each)."""
-    if not (x.is_cuda and x.dtype in (torch.float32, torch.bfloat16) and _of_kind(x, gamma)):
+    """The HIP RMSNorm takes x: GPU, fp32/bf16, a row of gamma of the same dtype and device, and rows
+    whose 16-byte vectors split evenly over a power-of-two number of lanes (at most 8 each)."""
+    if not (x.is_cuda and x.dtype in (torch.float32, torch.bfloat16) and _of_kind(x, gamma)
+            and gamma.shape == x.shape[-1:]):
         return False
     D = x.shape[-1]
     epv = 8 if x.dtype == torch.bfloat16 else 4
@@ -579,7 +580,7 @@ class MultiHeadAttention(torch.nn.Module):
         if rotary is not None and _joint_ok(x_BLD, weights, rotary):
             gammas = (self.q_norm.w_gamma_D, self.k_norm.w_gamma_D)
             cos, sin = rotary(x_BLD, seq_dim=1)  # (1, 1, L, K)
-            if _of_kind(x_BLD, *gammas, cos, sin):
+            if _of_kind(x_BLD, *gammas, cos, sin) and all(g.shape == (K,) for g in gammas):
                 out = _AttentionFunction.apply(x_BLD, *weights, *gammas, cos.reshape(L, K), sin.reshape(L, K), 1e-5)
                 return self._out_projection(out)
         q_heads, k_heads, v_heads = _QKVProjection.apply(x_BLD, self.w_q_DHK, self.w_k_DHK, self.w_v_DHK)

@@ -57,3 +57,12 @@ def test_block_without_rotary_takes_any_norms():
     attn = tr.MultiHeadAttention(16, 2, 8)
     attn.q_norm, attn.k_norm = torch.nn.Identity(), torch.nn.LayerNorm(8)
     assert attn(torch.randn(2, 5, 16)).shape == (2, 5, 16)
+
+
+def test_norm_weights_of_another_length_stay_with_torch(calls):
+    """A weight that broadcasts over the row is not the row of weights that the kernels read."""
+    attn, rot = _block()
+    attn.q_norm.w_gamma_D = torch.nn.Parameter(torch.empty(1, device="cuda", dtype=torch.bfloat16))
+    assert attn(_x(), rot).shape == (2, 9, 128)
+    assert "abacus_rmsnorm_fwd" in calls and not any("rope" in name for name in calls)  # k_norm's kernel only
+    assert calls.count("abacus_rmsnorm_fwd") == 1
