@@ -31,6 +31,7 @@ from __future__ import annotations
 import math
 
 import torch
+from torch.autograd.function import once_differentiable
 
 from . import _lib
 from .moe import MoE, MoEExpertParallel, _contig, _rank_and_world_size
@@ -108,6 +109,51 @@ def apply_rotary_pos_emb(q, k, cos, sin):
     return (q * cos) + (rotate_half(q) * sin), (k * cos) + (rotate_half(k) * sin)
 
 
+class _KernelGradient(torch.autograd.Function):
+    """The gradients that a kernel backward has formed, where that backward is itself recorded
+    (create_graph): their derivative is taken through `op`, the same forward in torch's operations
+    on fp32 copies, and only once it is asked for."""
+
+    @staticmethod
+    def forward(ctx, op, grads, d_out, *inputs):
+        ctx.op = op
+        ctx.save_for_backward(d_out, *inputs)
+        return grads
+
+    @staticmethod
+    @once_differentiable
+    def backward(ctx, *gg):
+        saved = ctx.saved_tensors
+        with torch.enable_grad():
+            d_out, *leaves = (t.detach().float().requires_grad_() for t in saved)
+            first = torch.autograd.grad(ctx.op(*leaves), leaves, d_out, create_graph=True)
+            asked = [(f, g.float()) for f, g in zip(first, gg) if g is not None]
+            second = torch.autograd.grad([f for f, _ in asked], (d_out, *leaves), [g for _, g in asked],
+                                         allow_unused=True)
+        return (None, None, *(None if g is None else g.to(t.dtype) for g, t in zip(second, saved)))
+
+
+def _recorded(op, grads, d_out, *inputs):
+    """grads, tied to d_out and the inputs where the running backward is recorded."""
+    return _KernelGradient.apply(op, grads, d_out, *inputs) if torch.is_grad_enabled() else grads
+
+
+def _norm_op(x, gamma, eps):
+    return gamma * x * torch.rsqrt(x.square().mean(dim=-1, keepdim=True) + eps)
+
+
+def _norm_rope_op(x_BLHK, gamma, cos_LK, sin_LK, eps):
+    y = _norm_op(x_BLHK, gamma, eps)
+    return y * cos_LK.float()[:, None] + rotate_half(y) * sin_LK.float()[:, None]
+
+
+def _causal_op(q_BLHK, k_BLHK, v_BLHK):
+    q, k, v = (t.transpose(1, 2).contiguous() for t in (q_BLHK, k_BLHK, v_BLHK))
+    s = q @ k.transpose(2, 3).contiguous() / math.sqrt(q.shape[-1])
+    s = s.masked_fill(torch.ones_like(s[0, 0], dtype=torch.bool).triu(1), float("-inf"))
+    return (torch.softmax(s, dim=-1) @ v).transpose(1, 2)
+
+
 def _of_kind(x: torch.Tensor, *tensors: torch.Tensor) -> bool:
     """Whether the tensors have x's dtype and device.  Rotary's tables may not: they are cached by
     length alone, so a module cast or moved after a forward hands on the old ones."""
@@ -143,12 +189,19 @@ class _RMSNormFunction(torch.autograd.Function):
         rstd = torch.empty(rows, dtype=torch.float32, device=x.device)
         _lib.call("abacus_rmsnorm_fwd", _lib.ptr(xc), _lib.ptr(gamma.contiguous()), rows, D, eps,
                   _lib.dtype_code(x.dtype), _lib.ptr(y), _lib.ptr(rstd), _lib.stream_of(x.device))
-        ctx.save_for_backward(xc, gamma, rstd)
+        ctx.save_for_backward(x, gamma, rstd)
+        ctx.eps = eps
         return y.view(x.shape)
 
     @staticmethod
     def backward(ctx, dy):
-        xc, gamma, rstd = ctx.saved_tensors
+        x, gamma, rstd = ctx.saved_tensors
+        with torch.no_grad():
+            grads = _RMSNormFunction.gradients(dy, x.contiguous(), gamma, rstd)
+        return (*_recorded(lambda x, g: _norm_op(x, g, ctx.eps), grads, dy, x, gamma), None)
+
+    @staticmethod
+    def gradients(dy, xc, gamma, rstd):
         D = xc.shape[-1]
         rows = xc.numel() // D
         dyc = dy.contiguous()
@@ -159,7 +212,7 @@ class _RMSNormFunction(torch.autograd.Function):
         _lib.call("abacus_rmsnorm_bwd", _lib.ptr(dyc), _lib.ptr(xc), _lib.ptr(gamma.contiguous()), _lib.ptr(rstd),
                   rows, D, _lib.dtype_code(xc.dtype), _lib.ptr(dx), _lib.ptr(dgamma), _lib.ptr(ws), nbytes,
                   _lib.stream_of(dy.device))
-        return dx.view(dy.shape), dgamma, None
+        return dx.view(dy.shape), dgamma
 
 
 def _fused_rope_ok(x: torch.Tensor, gamma: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> bool:
@@ -186,12 +239,20 @@ class _RMSNormRopeFunction(torch.autograd.Function):
         _lib.call("abacus_rmsnorm_rope_fwd", _lib.ptr(xc), _lib.ptr(gamma.contiguous()), _lib.ptr(cos_c),
                   _lib.ptr(sin_c), rows, L, H, K, eps, _lib.dtype_code(xc.dtype), _lib.ptr(y), _lib.ptr(rstd),
                   _lib.stream_of(xc.device))
-        ctx.save_for_backward(xc, gamma, rstd, cos_c, sin_c)
+        ctx.save_for_backward(x_BLHK, gamma, rstd, cos_c, sin_c)
+        ctx.eps = eps
         return y
 
     @staticmethod
     def backward(ctx, dy):
-        xc, gamma, rstd, cos_c, sin_c = ctx.saved_tensors
+        x, gamma, rstd, cos_c, sin_c = ctx.saved_tensors
+        with torch.no_grad():
+            grads = _RMSNormRopeFunction.gradients(dy, x.contiguous(), gamma, rstd, cos_c, sin_c)
+        op = lambda x, g: _norm_rope_op(x, g, cos_c, sin_c, ctx.eps)
+        return (*_recorded(op, grads, dy, x, gamma), None, None, None)
+
+    @staticmethod
+    def gradients(dy, xc, gamma, rstd, cos_c, sin_c):
         B, L, H, K = xc.shape
         rows = B * L * H
         dyc = dy.contiguous()
@@ -202,7 +263,7 @@ class _RMSNormRopeFunction(torch.autograd.Function):
         _lib.call("abacus_rmsnorm_rope_bwd", _lib.ptr(dyc), _lib.ptr(xc), _lib.ptr(gamma.contiguous()),
                   _lib.ptr(rstd), _lib.ptr(cos_c), _lib.ptr(sin_c), rows, L, H, K, _lib.dtype_code(xc.dtype),
                   _lib.ptr(dx), _lib.ptr(dgamma), _lib.ptr(ws), nbytes, _lib.stream_of(dy.device))
-        return dx, dgamma, None, None, None
+        return dx, dgamma
 
 
 class RMSNorm(torch.nn.Module):
@@ -330,7 +391,13 @@ class _FlashAttentionFunction(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, d_o):
-        q, k, v, o, lse = ctx.saved_tensors
+        saved = ctx.saved_tensors
+        with torch.no_grad():
+            grads = _FlashAttentionFunction.gradients(d_o, *saved)
+        return _recorded(_causal_op, grads, d_o, *saved[:3])
+
+    @staticmethod
+    def gradients(d_o, q, k, v, o, lse):
         B, L, H, K = q.shape
         d_o = d_o.contiguous()
         dq, dk, dv = (torch.empty_like(q) for _ in range(3))
@@ -404,14 +471,14 @@ class _QKVProjection(torch.autograd.Function):
         _, H, K = w_q_DHK.shape
         x_TD = x_BLD.reshape(B * L, D)
         outs = [(x_TD @ w.reshape(D, H * K)).view(B, L, H, K) for w in (w_q_DHK, w_k_DHK, w_v_DHK)]
-        ctx.save_for_backward(x_TD, w_q_DHK, w_k_DHK, w_v_DHK)
-        ctx.x_shape = (B, L, D)
+        ctx.save_for_backward(x_BLD, w_q_DHK, w_k_DHK, w_v_DHK)
         return tuple(outs)
 
     @staticmethod
     def backward(ctx, dq, dk, dv):
-        x_TD, w_q, w_k, w_v = ctx.saved_tensors
-        B, L, D = ctx.x_shape
+        x_BLD, w_q, w_k, w_v = ctx.saved_tensors
+        B, L, D = x_BLD.shape
+        x_TD = x_BLD.reshape(B * L, D)
         _, H, K = w_q.shape
         HK = H * K
         grads = [torch.zeros(B, L, H, K, dtype=x_TD.dtype, device=x_TD.device) if g is None else g
@@ -446,24 +513,39 @@ class _AttentionFunction(torch.autograd.Function):
         s = _lib.stream_of(dev)
         x_TD = x_BLD.reshape(B * L, D)
         q, k, v = ((x_TD @ w.reshape(D, H * K)).view(B, L, H, K) for w in (w_q, w_k, w_v))
-        gamma_q, gamma_k, cos_c, sin_c = (t.contiguous() for t in (gamma_q, gamma_k, cos_LK, sin_LK))
+        cos_c, sin_c = cos_LK.contiguous(), sin_LK.contiguous()
         qn, kn, o = torch.empty_like(q), torch.empty_like(k), torch.empty_like(q)
         rstd = torch.empty(2, rows, dtype=torch.float32, device=dev)
         lse = torch.empty(B, H, L, dtype=torch.float32, device=dev)
-        _lib.call("abacus_qk_norm_rope_fwd", _lib.ptr(q), _lib.ptr(k), _lib.ptr(gamma_q), _lib.ptr(gamma_k),
-                  _lib.ptr(cos_c), _lib.ptr(sin_c), rows, L, H, K, eps, _lib.BF16, _lib.ptr(qn), _lib.ptr(kn),
+        _lib.call("abacus_qk_norm_rope_fwd", _lib.ptr(q), _lib.ptr(k), _lib.ptr(gamma_q.contiguous()),
+                  _lib.ptr(gamma_k.contiguous()), _lib.ptr(cos_c), _lib.ptr(sin_c), rows, L, H, K, eps, _lib.BF16, _lib.ptr(qn), _lib.ptr(kn),
                   _lib.ptr(rstd), s)
         _lib.call("abacus_attention_any_fwd", _lib.ptr(qn), _lib.ptr(kn), _lib.ptr(v), B, L, H, K,
                   1.0 / math.sqrt(K), _lib.BF16, _lib.ptr(o), _lib.ptr(lse), s)
-        ctx.save_for_backward(x_TD, w_q, w_k, w_v, gamma_q, gamma_k, cos_c, sin_c, q, k, v, qn, kn, o, rstd, lse)
-        ctx.x_shape = (B, L, D)
+        ctx.save_for_backward(x_BLD, w_q, w_k, w_v, gamma_q, gamma_k, cos_c, sin_c, q, k, v, qn, kn, o, rstd, lse)
+        ctx.eps = eps
         return o
 
     @staticmethod
     def backward(ctx, d_o):
-        x_TD, w_q, w_k, w_v, gamma_q, gamma_k, cos_c, sin_c, q, k, v, qn, kn, o, rstd, lse = ctx.saved_tensors
-        B, L, D = ctx.x_shape
+        saved = ctx.saved_tensors
+        *inputs, cos_c, sin_c = saved[:8]
+        with torch.no_grad():
+            grads = _AttentionFunction.gradients(ctx.needs_input_grad, d_o, *saved)
+
+        def op(x, w_q, w_k, w_v, gamma_q, gamma_k):
+            q, k, v = ((x @ w.flatten(1)).unflatten(2, w.shape[1:]) for w in (w_q, w_k, w_v))
+            return _causal_op(_norm_rope_op(q, gamma_q, cos_c, sin_c, ctx.eps),
+                              _norm_rope_op(k, gamma_k, cos_c, sin_c, ctx.eps), v)
+
+        return (*_recorded(op, grads, d_o, *inputs), None, None, None)
+
+    @staticmethod
+    def gradients(needs, d_o, x_BLD, w_q, w_k, w_v, gamma_q, gamma_k, cos_c, sin_c, q, k, v, qn, kn, o, rstd, lse):
+        B, L, D = x_BLD.shape
         _, H, K = w_q.shape
+        x_TD = x_BLD.reshape(B * L, D)
+        gamma_q, gamma_k = gamma_q.contiguous(), gamma_k.contiguous()
         HK, rows, dev = H * K, B * L * H, q.device
         s = _lib.stream_of(dev)
         d_o = d_o.contiguous()
@@ -480,7 +562,6 @@ class _AttentionFunction(torch.autograd.Function):
         _lib.call("abacus_qk_norm_rope_bwd", _lib.ptr(dqn), _lib.ptr(dkn), _lib.ptr(q), _lib.ptr(k), _lib.ptr(gamma_q),
                   _lib.ptr(gamma_k), _lib.ptr(rstd), _lib.ptr(cos_c), _lib.ptr(sin_c), rows, L, H, K, _lib.BF16, at,
                   at + col, 3 * HK, _lib.ptr(dgamma_q), _lib.ptr(dgamma_k), _lib.ptr(ws), norm_bytes, s)
-        needs = ctx.needs_input_grad
         dx = None
         dws = [None, None, None]
         if needs[0]:
@@ -495,7 +576,7 @@ class _AttentionFunction(torch.autograd.Function):
                 dws = [torch.empty(D, HK, dtype=q.dtype, device=dev) for _ in range(3)]
                 _lib.call("abacus_split3", _lib.ptr(dw_D3), D, col, *map(_lib.ptr, dws), s)
             dws = [g.view(D, H, K) if need else None for g, need in zip(dws, needs[1:4])]
-        return (dx, *dws, dgamma_q if needs[4] else None, dgamma_k if needs[5] else None, None, None, None)
+        return dx, *dws, dgamma_q if needs[4] else None, dgamma_k if needs[5] else None
 
 
 def _joint_ok(x: torch.Tensor, weights, rotary) -> bool:
