@@ -6,6 +6,7 @@
 // per expert), as the grouped GEMMs of grouped_gemm.hip; rows are the same
 // expert-contiguous rows.
 #include <algorithm>
+#include <type_traits>
 
 #include "common.h"
 
@@ -78,8 +79,9 @@ struct Step {
 // first column; x: the first of n_rows rows (16 per group are taken, those past
 // the last one repeating it), pitch elements apart and zero from K to the next
 // whole vector.  Everything but w, x and the lane is wave-uniform, so a load is
-// a scalar base plus one of two lane offsets.
-template <typename T, bool UNALIGNED, bool NT>
+// a scalar base plus one of two lane offsets.  HOLD: for a caller without a loop
+// around it.
+template <typename T, bool UNALIGNED, bool NT, bool HOLD>
 __device__ inline void stream_rows(const T* __restrict__ w, int64_t ldw, const T* __restrict__ x, int64_t pitch,
                                    int n_rows, int K, int kb0, int kb1, int kstride, int lane,
                                    dec_f32x4 (&acc)[RG][kVec<T>]) {
@@ -92,19 +94,28 @@ __device__ inline void stream_rows(const T* __restrict__ w, int64_t ldw, const T
   auto load = [&](S& s, int kb) __attribute__((always_inline)) {
     const T* wb = w + (int64_t)kb * kKB * ldw;
     const T* xb = x + (int64_t)kb * kKB;
+    const T* wp[8];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) s.w[i] = load_weights<T, UNALIGNED, NT>(wb + i * ldw + woff);
+    for (int i = 0; i < 8; ++i) {
+      wp[i] = wb + i * ldw + woff;
+      s.w[i] = load_weights<T, UNALIGNED, NT>(wp[i]);
+    }
 #pragma unroll
     for (int r = 0; r < RG; ++r)
-      if (r * kGroup < n_rows) {
+      if ((HOLD && r == 0) || r * kGroup < n_rows) {
 #pragma unroll
         for (int v = 0; v < S::XV; ++v) s.x[r][v] = ld16(xb + v * kVec<T> + xoff[r]);
       }
+    // The addresses outlive their loads: else the compiler forms them in the loads' own destinations,
+    // which waits for the loads still in flight there (E 64 D 2048 M 1408, 64 tokens: 205 -> 231 us).
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if constexpr (HOLD) asm volatile("" : : "v"(wp[i]));
   };
   auto use = [&](const S& s) __attribute__((always_inline)) {
 #pragma unroll
     for (int r = 0; r < RG; ++r)
-      if (r * kGroup < n_rows) step_mfma(acc[r], s.w, s.x[r]);
+      if ((HOLD && r == 0) || r * kGroup < n_rows) step_mfma(acc[r], s.w, s.x[r]);
   };
   const int whole = min(kb1, K / kKB);  // k-blocks without a tail
   S a, b;
@@ -163,6 +174,53 @@ __device__ inline void store4(T* p, float a, float b, float c, float d) {
   }
 }
 
+// Tiles numbered over the rows that exist: (expert, columns, rows), ROWS rows each and
+// the rows fastest, an expert's first SKIP row tiles not counted.  Block b takes
+// its tile from an equal contiguous share for each XCD (it runs on XCD b % 8), so
+// that the blocks that read the same weights run beside each other on one L2.
+// Every wave finds the tile by itself; false: this block has none.
+struct RowTile {
+  int e, row0, row1, col;  // row1: the expert's end or row0 + ROWS
+};
+template <int ROWS, int SKIP>
+__device__ __forceinline__ bool row_tile(const int32_t* __restrict__ offsets, int E, int cols, int b, int lane,
+                                         RowTile& t) {
+  auto chunks = [&](int e) { return e < E ? max(0, (offsets[e + 1] - offsets[e] + ROWS - 1) / ROWS - SKIP) : 0; };
+  int total = 0;
+  for (int e0 = 0; e0 < E; e0 += 64) {
+    int c = chunks(e0 + lane);
+#pragma unroll
+    for (int o = 32; o; o >>= 1) c += __shfl_xor(c, o, 64);
+    total += __builtin_amdgcn_readfirstlane(c);
+  }
+  const int per = (total * cols + 7) / 8;
+  const int L = (b & 7) * per + (b >> 3);
+  if ((b >> 3) >= per || L >= total * cols) return false;
+  int before = 0;
+  for (int e0 = 0; e0 < E; e0 += 64) {
+    const int c = chunks(e0 + lane);
+    int end = c;  // inclusive scan over the lanes
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int u = __shfl_up(end, o, 64);
+      if (lane >= o) end += u;
+    }
+    const uint64_t past = __ballot((before + end) * cols > L);
+    if (past) {
+      const int l = __builtin_ctzll(past);
+      const int n = __builtin_amdgcn_readlane(c, l);
+      const int at = L - (before + __builtin_amdgcn_readlane(end, l) - n) * cols;
+      t.e = e0 + l;
+      t.col = at / n;
+      t.row0 = offsets[t.e] + (at % n + SKIP) * ROWS;
+      t.row1 = min(t.row0 + ROWS, offsets[t.e + 1]);
+      return true;
+    }
+    before += __builtin_amdgcn_readlane(end, 63);
+  }
+  return false;
+}
+
 // What bounds these kernels is the weight stream, so the weights go from HBM to
 // registers to MFMA with no LDS and no barrier on the way, each wave keeping 8 KB
 // of loads in flight under its products, and a tile's reduction is split over
@@ -175,28 +233,59 @@ __device__ inline void store4(T* p, float a, float b, float c, float d) {
 // token 352 -> 31, 128 tokens 493 -> 136.  Nontemporal weight loads 8% of it; a
 // third step in flight spills (+15%); 64 rows a pass spills too.
 
+// This block's tile of up to kRows rows.  First a block for each (expert, columns), which
+// takes the expert's first kRows rows: all there is where routing is even.  After
+// them (`more`) come the numbered tiles of the rows past those, as many blocks as
+// R / kRows row tiles need, wherever the rows are: one expert may hold all of them.
+// MANY (more than 8 rows per expert on average): those blocks read the weights, which
+// the blocks beside them read too, through the caches.  It costs the others 3-4%, as two
+// streams share the registers, so a smaller batch reads all of them in the one way.
+// us with at most four passes of an expert side by side -> here, every token on the same
+// experts, beside the 256-row tiles: bf16 E 128 D 1024 M 2816, 2048 tokens top-1 1077 ->
+// 160 (149), E 64 D 2048 M 1408, 170 tokens top-6 191 -> 108 (112), 64 tokens 113 -> 117 (87); fp32
+// E 64 D 1024 M 1408, 4096 tokens top-1 2816 -> 424 (537).  The second and the last of them
+// with even routing 221 -> 231 (259), 660 -> 588 (705), Zipf-skewed 260 -> 246 (239), 1363 -> 484 (696).
+__device__ __forceinline__ bool block_tile(const int32_t* __restrict__ offsets, int E, int cols, int lane, RowTile& t,
+                                           bool& more) {
+  more = (int)blockIdx.y >= E;
+  if (more) return row_tile<kRows, 1>(offsets, E, cols, ((int)blockIdx.y - E) * cols + (int)blockIdx.x, lane, t);
+  t.e = blockIdx.y;
+  t.col = blockIdx.x;
+  t.row0 = offsets[t.e];
+  t.row1 = min(t.row0 + kRows, offsets[t.e + 1]);
+  return t.row0 < t.row1;
+}
+// Its grid: (columns, experts, then whole turns of the 8 XCDs for R / kRows row tiles).
+int64_t grid_rows(int64_t R, int64_t E, int64_t cols) { return E + (R > kRows ? R / kRows + (7 + cols - 1) / cols : 0); }
+
 // H = silu(x w_gate) (x w_up) for one expert's rows and kCols columns per
 // block.  The first half of the W waves share w_gate's k-blocks, the second
 // half w_up's; the partial products meet in LDS and are added in wave order.
-template <typename T, int W, bool UNALIGNED, bool NT>
+template <typename T, int W, bool UNALIGNED, bool NT, bool MANY>
 __global__ __launch_bounds__(W * 64, 2) void decode_gateup_kernel(const T* __restrict__ xp,
                                                                     const T* __restrict__ w_gate,
                                                                     const T* __restrict__ w_up,
-                                                                    const int32_t* __restrict__ offsets, int D, int M,
-                                                                    int64_t ldh, T* __restrict__ h) {
+                                                                    const int32_t* __restrict__ offsets, int E, int D,
+                                                                    int M, int64_t ldh, T* __restrict__ h) {
   constexpr int HW = W / 2;  // waves per matrix
   constexpr int NC = kCols<T>, PART = kGroup * NC;
   __shared__ __attribute__((aligned(16))) float part[W * PART];
-  const int e = blockIdx.y;
-  const int row0 = offsets[e], row1 = offsets[e + 1];
-  if (row0 == row1) return;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), half = wave / HW;
-  const int n0 = min((int)blockIdx.x * NC, M - NC);  // the last tile overlaps its neighbour: the same sums, written twice
-  const T* w = (half ? w_up : w_gate) + (int64_t)e * D * M + n0;
-  for (int r0 = row0 + (int)blockIdx.z * kRows; r0 < row1; r0 += (int)gridDim.z * kRows) {
+  const int cols = (M + NC - 1) / NC;
+  RowTile tile;
+  bool more;
+  if (!block_tile(offsets, E, cols, lane, tile, more)) return;
+  const int row1 = tile.row1;
+  const int n0 = min(tile.col * NC, M - NC);  // the last tile overlaps its neighbour: the same sums, written twice
+  const T* w = (half ? w_up : w_gate) + (int64_t)tile.e * D * M + n0;
+  auto pass = [&](int r0) __attribute__((always_inline)) {
     dec_f32x4 acc[RG][kVec<T>] = {};
-    stream_rows<T, UNALIGNED, NT>(w, M, xp + (int64_t)r0 * D, D, row1 - r0, D, wave % HW, (D + kKB - 1) / kKB, HW, lane,
-                                  acc);
+    auto stream = [&](auto nt) __attribute__((always_inline)) {
+      stream_rows<T, UNALIGNED, decltype(nt)::value, MANY>(w, M, xp + (int64_t)r0 * D, D, row1 - r0, D, wave % HW,
+                                                     (D + kKB - 1) / kKB, HW, lane, acc);
+    };
+    if (!(MANY && NT && more)) stream(std::bool_constant<NT>{});
+    else if constexpr (MANY && NT) stream(std::false_type{});
 #pragma unroll
     for (int r = 0; r < RG; ++r) {
       const int rg0 = r0 + r * kGroup;
@@ -226,33 +315,45 @@ __global__ __launch_bounds__(W * 64, 2) void decode_gateup_kernel(const T* __res
         }
         store4<T>(h + (int64_t)row * ldh + n0 + c, o[0], o[1], o[2], o[3]);
       }
-      if (blockIdx.x == gridDim.x - 1 && tid < kGroup && rg0 + tid < row1)  // H's pad columns
+      if (tile.col == cols - 1 && tid < kGroup && rg0 + tid < row1)  // H's pad columns
         for (int64_t c = M; c < ldh; ++c) h[(int64_t)(rg0 + tid) * ldh + c] = (T)0;
     }
+  };
+  if constexpr (MANY) {
+    pass(tile.row0);
+  } else {
+    int step = kRows;  // one pass, in a loop as far as the compiler knows: it then keeps the addresses apart
+    asm("" : "+s"(step));
+    for (int r0 = tile.row0; r0 < row1; r0 += step) pass(r0);
   }
 }
 
 // Y = H w_down for one expert's rows, kCols columns and one slice of the
 // k-blocks per block, shared by its W waves.  One slice: Y itself; more: fp32
 // partials [slice][R][D] for decode_reduce_kernel.
-template <typename T, int W, bool NT>
+template <typename T, int W, bool NT, bool MANY>
 __global__ __launch_bounds__(W * 64, 2) void decode_down_kernel(const T* __restrict__ h, const T* __restrict__ w_down,
-                                                                  const int32_t* __restrict__ offsets, int M, int D,
-                                                                  int64_t ldh, int64_t R, int kb_per, int slices,
+                                                                  const int32_t* __restrict__ offsets, int E, int M,
+                                                                  int D, int64_t ldh, int64_t R, int kb_per, int slices,
                                                                   T* __restrict__ y, float* __restrict__ ws) {
   constexpr int NC = kCols<T>, PART = kGroup * NC;
   __shared__ __attribute__((aligned(16))) float part[W * PART];
-  const int e = blockIdx.y;
-  const int row0 = offsets[e], row1 = offsets[e + 1];
-  if (row0 == row1) return;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int n0 = min((int)blockIdx.x * NC, D - NC);
-  const int nkb = (M + kKB - 1) / kKB, slice = (int)blockIdx.z % slices, kb0 = slice * kb_per, kb1 = min(kb0 + kb_per, nkb);
-  const T* w = w_down + (int64_t)e * M * D + n0;
-  const int chunk = (int)blockIdx.z / slices, chunks = (int)gridDim.z / slices;
-  for (int r0 = row0 + chunk * kRows; r0 < row1; r0 += chunks * kRows) {
+  RowTile tile;
+  bool more;
+  if (!block_tile(offsets, E, (D + NC - 1) / NC, lane, tile, more)) return;
+  const int row1 = tile.row1;
+  const int n0 = min(tile.col * NC, D - NC);
+  const int nkb = (M + kKB - 1) / kKB, slice = (int)blockIdx.z, kb0 = slice * kb_per, kb1 = min(kb0 + kb_per, nkb);
+  const T* w = w_down + (int64_t)tile.e * M * D + n0;
+  auto pass = [&](int r0) __attribute__((always_inline)) {
     dec_f32x4 acc[RG][kVec<T>] = {};
-    stream_rows<T, false, NT>(w, D, h + (int64_t)r0 * ldh, ldh, row1 - r0, M, kb0 + wave, kb1, W, lane, acc);
+    auto stream = [&](auto nt) __attribute__((always_inline)) {
+      stream_rows<T, false, decltype(nt)::value, MANY>(w, D, h + (int64_t)r0 * ldh, ldh, row1 - r0, M, kb0 + wave, kb1, W,
+                                                 lane, acc);
+    };
+    if (!(MANY && NT && more)) stream(std::bool_constant<NT>{});
+    else if constexpr (MANY && NT) stream(std::false_type{});
 #pragma unroll
     for (int r = 0; r < RG; ++r) {
       const int rg0 = r0 + r * kGroup;
@@ -273,61 +374,23 @@ __global__ __launch_bounds__(W * 64, 2) void decode_down_kernel(const T* __restr
         else *reinterpret_cast<float4*>(ws + ((int64_t)slice * R + row) * D + n0 + c) = t;
       }
     }
+  };
+  if constexpr (MANY) {
+    pass(tile.row0);
+  } else {
+    int step = kRows;
+    asm("" : "+s"(step));
+    for (int r0 = tile.row0; r0 < row1; r0 += step) pass(r0);
   }
 }
 
 // More rows per expert (bf16): blocks of up to 64 rows of one expert, so that
-// most experts' weights still stream once.  Block b's tile comes from the
-// offsets: (expert, columns, rows), the rows fastest, numbered over the
-// real ones only, an equal contiguous share to each XCD (block b runs on XCD b % 8),
-// so that the blocks that read the same weights run beside each other on one L2
-// (weights that are read nontemporal miss it: E 64 D 2048 M 1408, 682 tokens 346 -> 410 us).
+// most experts' weights still stream once, numbered as row_tile does (weights that
+// are read nontemporal miss the L2 there: E 64 D 2048 M 1408, 682 tokens 346 -> 410 us).
 // What bounds them is the weight stream as long as an expert's rows are one block's.
 // 64 rows: more would not fit the registers (128 of 256 hold the sums), fewer stream
 // the weights more often.
 constexpr int kMidRows = 64;
-
-struct MidTile {
-  int e, row0, row1, col;  // row1: the expert's end or row0 + kMidRows
-};
-
-// Every wave finds the tile by itself; false: this block has none.
-__device__ __forceinline__ bool mid_tile(const int32_t* __restrict__ offsets, int E, int cols, int lane, MidTile& t) {
-  auto chunks = [&](int e) { return e < E ? (offsets[e + 1] - offsets[e] + kMidRows - 1) / kMidRows : 0; };
-  int total = 0;
-  for (int e0 = 0; e0 < E; e0 += 64) {
-    int c = chunks(e0 + lane);
-#pragma unroll
-    for (int o = 32; o; o >>= 1) c += __shfl_xor(c, o, 64);
-    total += c;
-  }
-  const int per = (total * cols + 7) / 8, b = (int)blockIdx.x;
-  const int L = (b & 7) * per + (b >> 3);
-  if ((b >> 3) >= per || L >= total * cols) return false;
-  int before = 0;
-  for (int e0 = 0; e0 < E; e0 += 64) {
-    const int c = chunks(e0 + lane);
-    int end = c;  // inclusive scan over the lanes
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int u = __shfl_up(end, o, 64);
-      if (lane >= o) end += u;
-    }
-    const uint64_t past = __ballot((before + end) * cols > L);
-    if (past) {
-      const int l = __builtin_ctzll(past);
-      const int n = __builtin_amdgcn_readlane(c, l);
-      const int at = L - (before + __builtin_amdgcn_readlane(end, l) - n) * cols;
-      t.e = e0 + l;
-      t.col = at / n;
-      t.row0 = offsets[t.e] + at % n * kMidRows;
-      t.row1 = min(t.row0 + kMidRows, offsets[t.e + 1]);
-      return true;
-    }
-    before += __builtin_amdgcn_readlane(end, 63);
-  }
-  return false;
-}
 
 // acc[r][j] += step_mfma's product for G groups of 16 rows, each column transposed once.
 template <int G>
@@ -512,8 +575,8 @@ __global__ __launch_bounds__(256, 2) void mid_gateup_kernel(const uint16_t* __re
   constexpr int NC = kCols<uint16_t>;
   __shared__ __attribute__((aligned(16))) float part[4 * kGroup * NC];
   const int tid = threadIdx.x, cols = (M + NC - 1) / NC;
-  MidTile t;
-  if (!mid_tile(offsets, E, cols, tid & 63, t)) return;
+  RowTile t;
+  if (!row_tile<kMidRows, 0>(offsets, E, cols, (int)blockIdx.x, tid & 63, t)) return;
   const int half = __builtin_amdgcn_readfirstlane(tid >> 7), n0 = min(t.col * NC, M - NC);
   const uint16_t* w = (half ? w_up : w_gate) + (int64_t)t.e * D * M + n0;
   const bool pads = t.col == cols - 1;
@@ -531,8 +594,8 @@ __global__ __launch_bounds__(256, 2) void mid_down_kernel(const uint16_t* __rest
   constexpr int NC = kCols<uint16_t>;
   __shared__ __attribute__((aligned(16))) float part[4 * kGroup * NC];
   const int tid = threadIdx.x, slice = (int)blockIdx.y, slices = (int)gridDim.y;
-  MidTile t;
-  if (!mid_tile(offsets, E, (D + NC - 1) / NC, tid & 63, t)) return;
+  RowTile t;
+  if (!row_tile<kMidRows, 0>(offsets, E, (D + NC - 1) / NC, (int)blockIdx.x, tid & 63, t)) return;
   const int n0 = min(t.col * NC, D - NC);
   const int kb0 = slice * kb_per, kb1 = min(kb0 + kb_per, (M + kKB - 1) / kKB);
   const uint16_t* w = w_down + (int64_t)t.e * M * D + n0;
@@ -573,11 +636,11 @@ DownPlan plan_down(int64_t R, int64_t D, int64_t M, int64_t E, int cols) {
   return {(int)per, (int)((nkb + per - 1) / per)};
 }
 
-template <typename T, int W, bool UNALIGNED, bool NT>
+template <typename T, int W, bool UNALIGNED, bool NT, bool MANY>
 void launch_gateup(dim3 grid, hipStream_t s, const void* xp, const void* wg, const void* wu, const int32_t* offsets,
-                   int64_t D, int64_t M, int64_t ldh, void* h) {
-  hipLaunchKernelGGL((decode_gateup_kernel<T, W, UNALIGNED, NT>), grid, dim3(W * 64), 0, s, (const T*)xp, (const T*)wg,
-                     (const T*)wu, offsets, (int)D, (int)M, ldh, (T*)h);
+                   int64_t E, int64_t D, int64_t M, int64_t ldh, void* h) {
+  hipLaunchKernelGGL((decode_gateup_kernel<T, W, UNALIGNED, NT, MANY>), grid, dim3(W * 64), 0, s, (const T*)xp,
+                     (const T*)wg, (const T*)wu, offsets, (int)E, (int)D, (int)M, ldh, (T*)h);
 }
 
 template <typename T>
@@ -607,32 +670,26 @@ int launch_mid(const void* xp, const void* wg, const void* wu, const void* wd, c
   return launch_reduce<uint16_t>(ws, R * D, p.slices, y, s);
 }
 
-template <typename T, bool NT>
+template <typename T, bool NT, bool MANY>
 int launch(const void* xp, const void* wg, const void* wu, const void* wd, const int32_t* offsets, int64_t R, int64_t D,
            int64_t M, int64_t E, int64_t ldh, void* h, void* y, float* ws, hipStream_t s) {
   constexpr int NC = kCols<T>;
-  if (mid_rows(R, E, sizeof(T) == 2 ? kBF16 : kF32)) return launch_mid(xp, wg, wu, wd, offsets, R, D, M, E, ldh, h, y, ws, s);
-  // An expert's passes of 32 rows run beside each other, up to four: one expert
-  // may hold many of the rows (E 4 D 512 M 1024, 128 tokens top-1: 26 -> 19 us).
-  // They are the slowest grid dimension, so that the blocks without rows come
-  // last: between the others they left CUs idle (E 64, 64 tokens: 179 -> 484 us).
-  const unsigned chunks = (unsigned)std::min<int64_t>(4, (R + kRows - 1) / kRows);
-  const unsigned t1 = (unsigned)((M + NC - 1) / NC), t2 = (unsigned)((D + NC - 1) / NC);
+  const int64_t t1 = (M + NC - 1) / NC, t2 = (D + NC - 1) / NC, touched = std::min(E, R);
   const DownPlan p = plan_down(R, D, M, E, NC);
-  const int64_t touched = std::min(E, R);
-  const dim3 g1(t1, (unsigned)E, chunks), g2(t2, (unsigned)E, chunks * p.slices);
+  const dim3 g1((unsigned)t1, (unsigned)grid_rows(R, E, t1));
+  const dim3 g2((unsigned)t2, (unsigned)grid_rows(R, E, t2), (unsigned)p.slices);
   const bool ua = M % kVec<T> != 0;
   if (four_waves(t1 * touched))
-    (ua ? launch_gateup<T, 4, true, NT> : launch_gateup<T, 4, false, NT>)(g1, s, xp, wg, wu, offsets, D, M, ldh, h);
+    (ua ? launch_gateup<T, 4, true, NT, MANY> : launch_gateup<T, 4, false, NT, MANY>)(g1, s, xp, wg, wu, offsets, E, D, M, ldh, h);
   else
-    (ua ? launch_gateup<T, 8, true, NT> : launch_gateup<T, 8, false, NT>)(g1, s, xp, wg, wu, offsets, D, M, ldh, h);
+    (ua ? launch_gateup<T, 8, true, NT, MANY> : launch_gateup<T, 8, false, NT, MANY>)(g1, s, xp, wg, wu, offsets, E, D, M, ldh, h);
   ABACUS_CHECK_LAUNCH("experts_decode_fwd (gate/up)");
   if (four_waves(t2 * touched))
-    hipLaunchKernelGGL((decode_down_kernel<T, 4, NT>), g2, dim3(256), 0, s, (const T*)h, (const T*)wd, offsets, (int)M,
-                       (int)D, ldh, R, p.kb_per, p.slices, (T*)y, ws);
+    hipLaunchKernelGGL((decode_down_kernel<T, 4, NT, MANY>), g2, dim3(256), 0, s, (const T*)h, (const T*)wd, offsets,
+                       (int)E, (int)M, (int)D, ldh, R, p.kb_per, p.slices, (T*)y, ws);
   else
-    hipLaunchKernelGGL((decode_down_kernel<T, 8, NT>), g2, dim3(512), 0, s, (const T*)h, (const T*)wd, offsets, (int)M,
-                       (int)D, ldh, R, p.kb_per, p.slices, (T*)y, ws);
+    hipLaunchKernelGGL((decode_down_kernel<T, 8, NT, MANY>), g2, dim3(512), 0, s, (const T*)h, (const T*)wd, offsets,
+                       (int)E, (int)M, (int)D, ldh, R, p.kb_per, p.slices, (T*)y, ws);
   ABACUS_CHECK_LAUNCH("experts_decode_fwd (down)");
   return launch_reduce<T>(ws, R * D, p.slices, y, s);
 }
@@ -662,9 +719,12 @@ bool takes(int64_t R, int64_t D, int64_t M, int64_t E, int dtype) {
 template <typename T>
 int launch_for(const void* xp, const void* wg, const void* wu, const void* wd, const int32_t* offsets, int64_t R,
                int64_t D, int64_t M, int64_t E, int64_t ldh, void* h, void* y, float* ws, hipStream_t s) {
+  if (mid_rows(R, E, sizeof(T) == 2 ? kBF16 : kF32)) return launch_mid(xp, wg, wu, wd, offsets, R, D, M, E, ldh, h, y, ws, s);
   const int64_t bytes = 3 * std::min(E, R) * D * M * (int64_t)sizeof(T);
-  return bytes >= (128ll << 20) ? launch<T, true>(xp, wg, wu, wd, offsets, R, D, M, E, ldh, h, y, ws, s)
-                                : launch<T, false>(xp, wg, wu, wd, offsets, R, D, M, E, ldh, h, y, ws, s);
+  const bool nt = bytes >= (128ll << 20), many = R > 8 * E;  // (see block_tile)
+  const auto run = nt ? (many ? launch<T, true, true> : launch<T, true, false>)
+                      : (many ? launch<T, false, true> : launch<T, false, false>);
+  return run(xp, wg, wu, wd, offsets, R, D, M, E, ldh, h, y, ws, s);
 }
 
 }  // namespace

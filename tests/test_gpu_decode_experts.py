@@ -64,6 +64,19 @@ def test_decode_experts_match_fp64(dtype, counts, D, M):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["bf16", "fp32"])
+@pytest.mark.parametrize("counts,D,M", [
+    ([0, 300, 1, 0] + [0] * 66 + [700, 33, 32] + [0] * 55, 264, 263),  # row tiles past the first of four experts
+    ([0] * 127 + [2048], 128, 136),            # all rows on the last expert
+    ([1] * 70, 384, 1025),                     # odd hidden size, blocks of 4 waves
+    ([2] * 24, 1024, 1031),                    # ... weights past the caches (read nontemporal), 8 waves
+    ([2] * 60 + [40, 0, 0, 33], 512, 1031),    # ... 4 waves, and rows past the first tile
+], ids=["later_tiles", "one_expert", "odd_four_waves", "odd_streamed", "odd_streamed_four_waves"])
+def test_decode_experts_variants(dtype, counts, D, M):
+    """The forms of the kernels that a size or the routing selects, as test_decode_experts_match_fp64."""
+    test_decode_experts_match_fp64(dtype, counts, D, M)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["bf16", "fp32"])
 @pytest.mark.parametrize("T,D,M,E,K", [(1, 256, 301, 8, 2), (37, 132, 160, 16, 4)])
 def test_small_forward_matches_oracle(dtype, T, D, M, E, K):
     """The eval layer (decode kernels; D off the vector width pads first) against the oracle in fp64."""
