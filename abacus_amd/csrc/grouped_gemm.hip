@@ -2571,6 +2571,8 @@ int abacus_experts_down_bwd(const void* dy_RD, const void* w_down_EMD, const voi
   GemmArgs gd = args_down_dgrad(dy_RD, w_down_EMD, gate, up, offsets_E1, R, ld, D, E, dgate, dup);
   gd.b_estride = M * D;
   gd.b_rows = (int)M;
+  if (!dw_down_EMD)
+    return R == 0 ? 0 : dispatch_gemm<kDownDgrad>(kBF16, gd, (int)R, (hipStream_t)stream, "experts_down_bwd");
   GemmArgs gw = args_down_wgrad(h, dy_RD, offsets_E1, ld, D, E, dw_down_EMD);
   gw.c_estride = M * D;
   gw.c_rows = (int)M;
@@ -2601,6 +2603,7 @@ int abacus_experts_gateup_bwd(const void* dgate, const void* dup, const void* w_
   if (dtype == kF32 ? check_gemm_shape(R, D, M, E, dtype) : check_hidden(R, D, M, ld, E)) return 1;
   ABACUS_CHECK_ARG(dtype != kF32 || ld == M, "fp32: ld %lld must be hidden_dim %lld", (long long)ld, (long long)M);
   ABACUS_CHECK_ARG(tile_ctr != nullptr, "tile_ctr workspace is NULL");
+  ABACUS_CHECK_ARG(!dw_gate_EDM == !dw_up_EDM, "dw_gate and dw_up come together");
   const hipStream_t s = (hipStream_t)stream;
   GemmArgs gd = args_gateup_dgrad(dgate, dup, w_gate, w_up, offsets_E1, R, D, ld, E, dx_perm_RD);
   GemmArgs gw = args_gateup_wgrad(x_perm_RD, dgate, dup, offsets_E1, D, ld, E, dw_gate_EDM, dw_up_EDM);
@@ -2609,18 +2612,22 @@ int abacus_experts_gateup_bwd(const void* dgate, const void* dup, const void* w_
   gw.c_cols = ld == M ? 0 : (int)M;
   gw.tile_ctr = tile_ctr;
   const char* name = "experts_gateup_bwd";
+  if (!dx_perm_RD) return dw_gate_EDM ? dispatch_gemm<kGateUpWgrad>(dtype, gw, (int)R, s, name) : 0;
   const int slices = gateup_bwd_slices(dtype, gd, R, D, ld, E);
   if (slices > 1 && ws != nullptr && ws_bytes >= slices_ws_bytes(slices, R, D)) {
     gd.ksplit = slices;
     gd.ksplit_ws = (float*)ws;
     if (dtype == kBF16) {
-      if (launch_rows<uint16_t, kGateUpDgrad, kGateUpWgrad>(gd, (int)R, &gw, -1, true, s, name)) return 1;
+      if (dw_gate_EDM ? launch_rows<uint16_t, kGateUpDgrad, kGateUpWgrad>(gd, (int)R, &gw, -1, true, s, name)
+                      : launch_rows<uint16_t, kGateUpDgrad, -1>(gd, (int)R, nullptr, -1, true, s, name))
+        return 1;
       return launch_rows_reduce<uint16_t>(gd.ksplit_ws, R, D, slices, dx_perm_RD, s, name);
     }
     if (launch_rows<float, kGateUpDgrad, -1>(gd, (int)R, nullptr, -1, true, s, name)) return 1;
     if (launch_rows_reduce<float>(gd.ksplit_ws, R, D, slices, dx_perm_RD, s, name)) return 1;
-    return dispatch_gemm<kGateUpWgrad>(dtype, gw, (int)R, s, name);
+    return dw_gate_EDM ? dispatch_gemm<kGateUpWgrad>(dtype, gw, (int)R, s, name) : 0;
   }
+  if (!dw_gate_EDM) return R == 0 ? 0 : dispatch_gemm<kGateUpDgrad>(dtype, gd, (int)R, s, name);
   return dispatch_pair<kGateUpDgrad, kGateUpWgrad>(dtype, gd, gw, (int)R, s, name, name, name);
 }
 

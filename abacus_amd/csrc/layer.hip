@@ -101,8 +101,11 @@ extern "C" int abacus_layer_bwd(const int64_t* plan, const void* x, const void* 
   } else {
     RUN(abacus_moe_down_bwd_dgrad(dy, w_down, gate, up, offsets, R, p.M, p.D, p.E, dt, dgate, dup, s));
   }
-  const bool want_x = dx != nullptr || pitched, want_w = dw_gate != nullptr;
-  if (want_x && want_w && (pitched || p.bws_bytes > 0)) {
+  const bool want_x = dx != nullptr, want_w = dw_gate != nullptr;
+  if ((want_x || want_w) && pitched) {
+    RUN(abacus_experts_gateup_bwd(dgate, dup, w_gate, w_up, xp, offsets, R, p.D, p.M, p.ld, p.E, dt, want_x ? dxp : nullptr,
+                                  dw_gate, dw_up, ctr, at(scratch, p.bws), p.bws_bytes, s));
+  } else if (want_x && want_w && p.bws_bytes > 0) {
     RUN(abacus_experts_gateup_bwd(dgate, dup, w_gate, w_up, xp, offsets, R, p.D, p.M, p.ld, p.E, dt, dxp, dw_gate, dw_up,
                                   ctr, at(scratch, p.bws), p.bws_bytes, s));
   } else if (want_x && want_w) {

@@ -181,20 +181,19 @@ def _layer_backward(ctx, dout):
     x_TD, w_DE, w_gate, w_up, w_down, route, keep = ctx.saved_tensors
     plan, needs, dev = ctx.plan, ctx.needs_input_grad, x_TD.device
     dout = _contig(dout.to(x_TD.dtype))
-    pitched = plan.at["ld"] != plan.at["M"]
     scratch = torch.empty(plan.bwd_bytes, dtype=torch.uint8, device=dev)
     dx = torch.empty_like(x_TD) if needs[0] else None
     dw_DE = torch.empty_like(w_DE) if needs[1] else None
     dw_gate = dw_up = None
-    if needs[2] or needs[3] or pitched:
+    if needs[2] or needs[3]:
         dw_gate, dw_up = torch.empty_like(w_gate), torch.empty_like(w_up)
-    dw_down = torch.empty_like(w_down) if needs[4] or pitched else None
+    dw_down = torch.empty_like(w_down) if needs[4] else None
     call(
         "abacus_layer_bwd", plan.fields, ptr(x_TD), ptr(w_DE), ptr(w_gate), ptr(w_up), ptr(w_down), ctx.route_scale,
         route.data_ptr(), keep.data_ptr(), ptr(dout), scratch.data_ptr(), ptr(dx), ptr(dw_DE), ptr(dw_gate), ptr(dw_up),
         ptr(dw_down), _lib.stream_of(dev),
     )
-    return (dx, dw_DE, dw_gate if needs[2] else None, dw_up if needs[3] else None, dw_down if needs[4] else None,
+    return (dx, dw_DE, dw_gate if needs[2] else None, dw_up if needs[3] else None, dw_down,
             None, None, None, None, None, None)
 
 
@@ -408,15 +407,13 @@ class _MoEFunction(torch.autograd.Function):
         ld = gate.shape[1]
         dgate = torch.empty(R, ld, dtype=x_TD.dtype, device=dev)
         dup = torch.empty(R, ld, dtype=x_TD.dtype, device=dev)
-        dw_down = None
+        dw_down = torch.empty_like(w_down) if needs[4] else None
         if ld != M:
-            dw_down = torch.empty_like(w_down)
             call(
                 "abacus_experts_down_bwd", ptr(dy), ptr(w_down), ptr(gate), ptr(up), ptr(h), ptr(offsets), R, M, ld, D, E,
                 ptr(dgate), ptr(dup), ptr(dw_down), ptr(_lib.tile_ctr(dev)), s,
             )
         elif needs[4]:
-            dw_down = torch.empty_like(w_down)
             call(
                 "abacus_moe_down_bwd", ptr(dy), ptr(w_down), ptr(gate), ptr(up), ptr(h), ptr(offsets), R, M, D, E,
                 dt, ptr(dgate), ptr(dup), ptr(dw_down), ptr(_lib.tile_ctr(dev)), s,
@@ -426,13 +423,14 @@ class _MoEFunction(torch.autograd.Function):
                 "abacus_moe_down_bwd_dgrad", ptr(dy), ptr(w_down), ptr(gate), ptr(up), ptr(offsets), R, M, D, E, dt,
                 ptr(dgate), ptr(dup), s,
             )
-        dxp = torch.empty(R, D, dtype=x_TD.dtype, device=dev) if needs[0] or ld != M else None
+        dxp = torch.empty(R, D, dtype=x_TD.dtype, device=dev) if needs[0] else None
         dw_gate = dw_up = None
-        if needs[2] or needs[3] or ld != M:
+        if needs[2] or needs[3]:
             dw_gate, dw_up = (torch.empty(E, D, M, dtype=x_TD.dtype, device=dev) for _ in range(2))
-        both = dxp is not None and dw_gate is not None
-        ws_bytes = query("abacus_experts_gateup_bwd_ws_bytes", R, D, ld, E, dt) if both and x_TD.is_cuda else 0
-        if ws_bytes > 0 or ld != M:  # (ld != M: w_gate and w_up are the forward's padded copies)
+        both, pitched = dxp is not None and dw_gate is not None, ld != M
+        ws_bytes = query("abacus_experts_gateup_bwd_ws_bytes", R, D, ld, E, dt) if (both or pitched) and x_TD.is_cuda else 0
+        if (both and ws_bytes > 0) or (pitched and (dxp is not None or dw_gate is not None)):
+            # (pitched: w_gate and w_up are the forward's padded copies)
             ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes > 0 else None
             call(
                 "abacus_experts_gateup_bwd", ptr(dgate), ptr(dup), ptr(w_gate), ptr(w_up), ptr(xp), ptr(offsets), R, D, M,
@@ -454,7 +452,7 @@ class _MoEFunction(torch.autograd.Function):
                 ptr(dw_gate), ptr(dw_up), ptr(_lib.tile_ctr(dev)), s,
             )
         dx, dw_DE = _router_dgrad_wgrad(needs[0], needs[1], x_TD, w_DE, dlogit, idx32, pos, dxp, wt)
-        return (dx, dw_DE, dw_gate if needs[2] else None, dw_up if needs[3] else None, dw_down if needs[4] else None,
+        return (dx, dw_DE, dw_gate if needs[2] else None, dw_up if needs[3] else None, dw_down,
                 None, None, None, None, None, None)
 
 

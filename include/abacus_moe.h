@@ -148,7 +148,7 @@ int abacus_experts_decode_fwd(const void* x_perm_RD, const void* w_gate_EDM, con
  * w_up (E*D rows of M) into rows of ld, which abacus_moe_gateup_fwd takes as a
  * hidden size of ld; w_down, and every weight gradient, keep rows and columns of
  * M.  Otherwise as abacus_moe_down_fwd (workspace of abacus_moe_down_fwd_ws_bytes
- * for ld) and abacus_moe_down_bwd. */
+ * for ld) and abacus_moe_down_bwd, where a NULL dw_down is not computed. */
 int abacus_experts_pad_columns(const void* src, int64_t rows, int64_t M, int64_t ld, void* dst, void* stream);
 int abacus_experts_down_fwd(const void* h, const void* w_down_EMD, const int32_t* offsets_E1, int64_t R, int64_t M,
                             int64_t ld, int64_t D, int64_t E, void* y_RD, void* ws, int64_t ws_bytes, void* stream);
@@ -159,7 +159,8 @@ int abacus_experts_down_bwd(const void* dy_RD, const void* w_down_EMD, const voi
 /* abacus_moe_gateup_bwd for any hidden size (bf16; w_gate and w_up with rows of
  * ld; fp32: ld = M), with a workspace of abacus_experts_gateup_bwd_ws_bytes bytes
  * (for a hidden size of ld; 0: no use for one) that lets the data gradient run as
- * slices of its reduction where its tiles are too few for the GPU. */
+ * slices of its reduction where its tiles are too few for the GPU.  A NULL dx_perm
+ * is not computed, nor are NULL dw_gate and dw_up (both or neither). */
 int64_t abacus_experts_gateup_bwd_ws_bytes(int64_t R, int64_t D, int64_t M, int64_t E, int dtype);
 int abacus_experts_gateup_bwd(const void* dgate, const void* dup, const void* w_gate, const void* w_up,
                               const void* x_perm_RD, const int32_t* offsets_E1, int64_t R, int64_t D, int64_t M,
