@@ -49,7 +49,12 @@ class Routing:
 
 
 class _PlanRouting(Routing):
-    """A Routing whose tensors are views of the layer's route buffer, made when they are asked for."""
+    """A Routing whose tensors are views of the layer's route buffer, made when they are asked for.
+
+    The buffer is saved for the backward, so a change of what the backward reads (weights, offsets,
+    pos) is noticed there; the rest is viewed apart from that watch and may be changed."""
+
+    _READ_BY_BACKWARD = ("weights", "offsets", "pos")
 
     def __init__(self, route: torch.Tensor, plan: "_LayerPlan", dtype: torch.dtype):
         self._route, self._at, self._sizes, self._dtype = route, plan.at, plan.sizes, dtype
@@ -58,7 +63,8 @@ class _PlanRouting(Routing):
         n, a = dtype.itemsize, self._at[name]
         for d in shape:
             n *= d
-        return self._route[a:a + n].view(dtype).view(shape)
+        route = self._route if name in self._READ_BY_BACKWARD else self._route.data
+        return route[a:a + n].view(dtype).view(shape)
 
     @functools.cached_property
     def logits_TE(self):

@@ -89,3 +89,22 @@ def test_frozen_experts_hand_the_backward_no_weight_gradients(monkeypatch):
     _run(layer, x, dy)
     (args,) = [a for n, a in made if n == "abacus_layer_bwd"]
     assert args[-4:-1] == (None, None, None)  # dw_gate, dw_up, dw_down
+
+
+def test_routing_record_may_be_changed():
+    """The layer's routing record belongs to the caller: what the backward does not read may change before it."""
+    layer, x, dy = _layer(*SHAPES[0])
+    want = _run(layer, x, dy)
+    layer.zero_grad(set_to_none=True)
+    layer.router.expert_bias_E.zero_()
+    xi = x.clone().requires_grad_()
+    out = layer(xi)
+    r = layer.router.last_routing
+    for t in (r.logits_TE, r.indices_TK, r.counts_E, r.perm_R):
+        t.zero_()
+    out.backward(dy)
+    assert torch.equal(xi.grad, want["x"]) and torch.equal(layer.w_up_EDM.grad, want["w_up_EDM"])
+    out = layer(xi)
+    layer.router.last_routing.weights_TK.zero_()  # the backward reads these
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        out.backward(dy)
