@@ -10,8 +10,8 @@ routes the same way).  Forward-only workloads (the small skewed batches) run the
 forward under no_grad.
 
 Prints one JSON line with the throughput, the roofline position of the dominant
-kernel (device time from HIP events recorded on the launch stream around every
-entry point during the timed steps), per-kernel figures, and the CPU baseline: the
+kernel and per-kernel figures (device time from HIP events recorded on the launch
+stream around every entry point, in further steps after the timed ones), and the CPU baseline: the
 oracle's restatement of the reference algorithm timed on the host cores on a bounded
 token sample of the same layer.
 """
@@ -45,7 +45,24 @@ GEMM_FLOPS = {  # multiples of R*D*M per entry point
     "abacus_moe_gateup_bwd_dgrad": 4,
     "abacus_moe_gateup_bwd_wgrad": 4,
     "abacus_moe_gateup_bwd": 8,          # dgrad + wgrad in one launch
+    "abacus_experts_gateup_bwd": 8,      # the same with a workspace, or for a padded hidden pitch
+    "abacus_experts_down_fwd": 2,        # a padded hidden pitch
+    "abacus_experts_down_bwd": 4,
 }
+NOT_GEMM = {"abacus_experts_pad_columns"}
+
+
+def is_moe(name):
+    """Whether an entry point is the MoE layer's."""
+    return name.startswith(("abacus_moe_", "abacus_experts_"))
+
+
+def check_known(names):
+    """Every expert entry point that ran is in the product table or known not to be a product."""
+    unknown = [n for n in names if n.startswith(("abacus_experts_", "abacus_moe_gateup", "abacus_moe_down"))
+               and n not in GEMM_FLOPS and n not in NOT_GEMM]
+    if unknown:
+        raise RuntimeError(f"no operation count for {unknown}")
 
 
 def parse_args():
@@ -235,6 +252,9 @@ def bench_decoder(args, dtype):
     ms_per_step = 1000.0 * elapsed / args.steps
     # After the timed region: as many steps again with HIP events around every entry point (each
     # event record delays the next kernel by a few microseconds, so none are in the timed steps).
+    with _lib.KernelTimer():
+        train_step(model, opt, tokens)  # the first of that route
+        torch.cuda.synchronize()
     timer = _lib.KernelTimer()
     t1 = time.perf_counter()
     with timer:
@@ -243,7 +263,8 @@ def bench_decoder(args, dtype):
         torch.cuda.synchronize()
     full_elapsed = time.perf_counter() - t1
     totals = timer.totals_ms()
-    moe_ms = sum(ms for name, (ms, _) in totals.items() if name.startswith("abacus_moe_")) / args.steps
+    check_known(totals)
+    moe_ms = sum(ms for name, (ms, _) in totals.items() if is_moe(name)) / args.steps
     lib_ms = sum(ms for ms, _ in totals.values()) / args.steps  # every entry point: MoE, norms, AdamW
     kernels = {name: {"avg_us": round(ms / n * 1000.0, 2), "calls": n,
                       "share": round(ms / (full_elapsed * 1000.0), 4)}
@@ -496,31 +517,25 @@ def main():
             loss.backward()
         xi.grad = None
 
-    # Warmup; its last step (or one more step when there is no warmup) runs under a timer on every
-    # entry point, which names the dominant kernel.
-    for _ in range(max(0, args.warmup - 1)):
+    for _ in range(max(1, args.warmup)):
         step()
-    probe = _lib.KernelTimer()
-    with probe:
-        step()
-    dominant = max(probe.totals_ms().items(), key=lambda kv: kv[1][0])[0]
     torch.cuda.synchronize()
 
-    # The timed region: HIP events only around the dominant kernel (every event record is a packet
-    # between two kernels and delays the next by a few microseconds).
-    timer = _lib.KernelTimer(only={dominant})
+    # The timed region, without a timer: the layer then makes one call per direction, as in a
+    # program that uses it (with a KernelTimer active it calls its entry points one by one).
     t0 = time.perf_counter()
-    with timer:
-        for _ in range(args.steps):
-            step()
-        torch.cuda.synchronize()
+    for _ in range(args.steps):
+        step()
+    torch.cuda.synchronize()
     elapsed = time.perf_counter() - t0
     ms_per_step = 1000.0 * elapsed / args.steps
     tokens_per_s = wl.tokens / (ms_per_step / 1000.0)
-    d_ms, d_n = timer.totals_ms()[dominant]
 
     # After the timed region: the same steps again with events around every entry point, for the
     # per-kernel table (times there include the events' own delays between kernels only).
+    with _lib.KernelTimer():
+        step()  # the first of that route
+        torch.cuda.synchronize()
     full = _lib.KernelTimer()
     t1 = time.perf_counter()
     with full:
@@ -528,6 +543,18 @@ def main():
             step()
         torch.cuda.synchronize()
     full_elapsed = time.perf_counter() - t1
+    totals = full.totals_ms()
+    check_known(totals)
+    dominant = max(totals.items(), key=lambda kv: kv[1][0])[0]
+
+    # And with events around the dominant kernel only (every event record is a packet between two
+    # kernels and delays the next by a few microseconds), for the roofline.
+    timer = _lib.KernelTimer(only={dominant})
+    with timer:
+        for _ in range(args.steps):
+            step()
+        torch.cuda.synchronize()
+    d_ms, d_n = timer.totals_ms()[dominant]
 
     # Forward-only workloads: the same eval-mode forward replayed from a HIP graph (one graph
     # launch per step instead of the forward's kernel launches and Python calls), timed over
@@ -555,7 +582,6 @@ def main():
         torch.cuda.synchronize()
         del src, dst
 
-    totals = full.totals_ms()
     R, D, M = wl.rows, wl.dim, wl.hidden
     peak_mfma = PEAK_BF16_TFLOPS if wl.dtype == torch.bfloat16 else PEAK_FP32_TFLOPS
     kernels = {}
@@ -625,8 +651,9 @@ def main():
         "grouped_gemm": {"tflops": round(gemm_tf, 1), "mfma_frac": round(gemm_tf / peak_mfma, 4),
                          "ms_per_step": round(gemm_ms, 4)},
         "kernels": kernels,
-        "timing": {"value": "the timed steps carry HIP events only around the dominant kernel (roofline)",
-                   "kernels": "HIP events around every entry point over as many further steps",
+        "timing": {"value": "the timed steps carry no events",
+                   "kernels": "HIP events around every entry point, called one by one, over as many further steps",
+                   "roofline": "HIP events around the dominant kernel only, over as many further steps",
                    "kernels_pass_ms_per_step": round(1000.0 * full_elapsed / args.steps, 4)},
     }
     if graph is not None:

@@ -14,3 +14,14 @@ def test_more_than_one_gpu_is_refused():
     assert r.returncode == 2
     assert "measures one GPU" in r.stderr and "--gpus 2" in r.stderr
     assert r.stdout == ""  # no JSON line
+
+
+def test_every_expert_product_is_counted():
+    """The FLOP table and the MoE layer's share know every expert entry point of the library."""
+    sys.path.insert(0, ROOT)
+    import bench
+    from abacus_amd import _lib
+
+    experts = [n for n in _lib.SIGNATURES if "_experts_" in n and not n.endswith("_bytes")]
+    assert len(experts) >= 5 and all(bench.is_moe(n) for n in experts)
+    bench.check_known(n for n in _lib.SIGNATURES if not n.endswith("_bytes"))
