@@ -161,27 +161,30 @@ template <typename T>
 __global__ __launch_bounds__(1024) void ce_mean_kernel(const float* __restrict__ loss, const int64_t* __restrict__ tgt,
                                                        int64_t N, int64_t ignore_index, T* __restrict__ out,
                                                        float* __restrict__ count) {
-  __shared__ float sum_s[16], cnt_s[16];
+  __shared__ float sum_s[16];
+  __shared__ int cnt_s[16];
   float s = 0.f;
-  int64_t n = 0;
+  int n = 0;  // (a wave's rows, at most 2^29)
 #pragma unroll 4
   for (int64_t i = threadIdx.x; i < N; i += 1024) {
     s += loss[i];
     n += tgt[i] != ignore_index ? 1 : 0;
   }
-  float c = (float)n;  // (a thread's rows, at most 2^23: exact)
   s = wave_sum(s);
-  c = wave_sum(c);
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) n += __shfl_xor(n, off, 64);
   if ((threadIdx.x & 63) == 0) {
     sum_s[threadIdx.x >> 6] = s;
-    cnt_s[threadIdx.x >> 6] = c;
+    cnt_s[threadIdx.x >> 6] = n;
   }
   __syncthreads();
   if (threadIdx.x == 0) {
+    int64_t total = n;
     for (int w = 1; w < 16; ++w) {
       s += sum_s[w];
-      c += cnt_s[w];
+      total += cnt_s[w];
     }
+    const float c = (float)total;
     *out = from_f32<T>(s / c);
     *count = c;
   }

@@ -5,6 +5,7 @@ import pytest
 import torch
 import torch.nn.functional as F
 
+from abacus_amd import _lib
 from abacus_amd.train import cross_entropy
 
 pytestmark = pytest.mark.gpu
@@ -40,3 +41,17 @@ def test_no_rows_left_is_nan():
     assert torch.count_nonzero(x.grad) == 0
     assert torch.isnan(cross_entropy(torch.randn(0, 16, device="cuda"), torch.zeros(0, dtype=torch.int64, device="cuda")))
 
+
+
+def test_count_of_many_rows_is_rounded_once():
+    """More rows than fp32 counts exactly: the count is the exact one, rounded once."""
+    N, V = 3 << 24, 8
+    x = torch.zeros(N, V, device="cuda", dtype=torch.bfloat16)
+    t = torch.zeros(N, device="cuda", dtype=torch.int64)
+    for wave in range(9, 16):  # odd sums of the waves past the first 2^24 rows
+        t[wave * 64:wave * 64 + 3] = -100
+    rows = torch.empty(2, N, device="cuda")
+    loss, count = torch.empty((), device="cuda", dtype=torch.bfloat16), torch.empty((), device="cuda")
+    _lib.call("abacus_cross_entropy_mean_fwd", _lib.ptr(x), _lib.ptr(t), N, V, -100, _lib.BF16, rows.data_ptr(),
+              rows[1].data_ptr(), _lib.ptr(loss), _lib.ptr(count), _lib.stream_of(x.device))
+    assert float(count) == float((t != -100).sum().float())
