@@ -161,18 +161,20 @@ template <typename T>
 __global__ __launch_bounds__(1024) void ce_mean_kernel(const float* __restrict__ loss, const int64_t* __restrict__ tgt,
                                                        int64_t N, int64_t ignore_index, T* __restrict__ out,
                                                        float* __restrict__ count) {
-  __shared__ float sum_s[16];
+  __shared__ double sum_s[16];
   __shared__ int cnt_s[16];
-  float s = 0.f;
+  double s = 0.0;  // (a thread adds every 1024th row one by one: 16384 in a batch of 2^24)
   int n = 0;  // (a wave's rows, at most 2^29)
 #pragma unroll 4
   for (int64_t i = threadIdx.x; i < N; i += 1024) {
-    s += loss[i];
+    s += (double)loss[i];
     n += tgt[i] != ignore_index ? 1 : 0;
   }
-  s = wave_sum(s);
 #pragma unroll
-  for (int off = 32; off > 0; off >>= 1) n += __shfl_xor(n, off, 64);
+  for (int off = 32; off > 0; off >>= 1) {
+    s += __shfl_xor(s, off, 64);
+    n += __shfl_xor(n, off, 64);
+  }
   if ((threadIdx.x & 63) == 0) {
     sum_s[threadIdx.x >> 6] = s;
     cnt_s[threadIdx.x >> 6] = n;
@@ -185,7 +187,7 @@ __global__ __launch_bounds__(1024) void ce_mean_kernel(const float* __restrict__
       total += cnt_s[w];
     }
     const float c = (float)total;
-    *out = from_f32<T>(s / c);
+    *out = from_f32<T>((float)(s / total));
     *count = c;
   }
 }

@@ -1,6 +1,8 @@
 """cross_entropy's mean on the device: row sums and counts of one and several passes of the mean kernel, vocabularies
 off the vector (rows at any alignment), an ignore index of its own, no rows left, against fp64."""
 
+import math
+
 import pytest
 import torch
 import torch.nn.functional as F
@@ -55,3 +57,11 @@ def test_count_of_many_rows_is_rounded_once():
     _lib.call("abacus_cross_entropy_mean_fwd", _lib.ptr(x), _lib.ptr(t), N, V, -100, _lib.BF16, rows.data_ptr(),
               rows[1].data_ptr(), _lib.ptr(loss), _lib.ptr(count), _lib.stream_of(x.device))
     assert float(count) == float((t != -100).sum().float())
+
+
+def test_sum_of_many_rows_keeps_its_digits():
+    """The row losses of a large batch are added without the error of a long fp32 chain (row losses: 1e-6)."""
+    N = 1 << 24
+    x = torch.zeros(N, 4, device="cuda")
+    loss = cross_entropy(x, torch.zeros(N, device="cuda", dtype=torch.int64))
+    assert abs(float(loss) - math.log(4.0)) <= 2e-6 * math.log(4.0)
