@@ -2210,6 +2210,7 @@ int dispatch_gemm(int dtype, const GemmArgs& g, int R, hipStream_t s, const char
     if (dtype == kBF16) return launch_pipe<uint16_t, KIND>(g, R, s, name);
     if constexpr (!KindTraits<KIND>::WGRAD && KIND != kDownDgrad) return launch_pipe<float, KIND>(g, R, s, name);
   }
+  ABACUS_CHECK_ARG(dtype == kF32, "%s: no kernel for dtype code %d with these dimensions", name, dtype);
   return launch_gemm<float, KIND>(g, R, s, name);
 }
 
