@@ -14,12 +14,13 @@
 //   DOWN_WGRAD    dWd[e] (M x D)        H^T           mc   dY          nc     reduction
 //   GATEUP_WGRAD  dWg,dWu[e] (D x M)    xp^T          mc   dG,dU       nc     reduction
 //
-// (kc = k-contiguous in memory, mc/nc = row/column-contiguous.)  Every
-// operand is staged through LDS as [row][k] with k contiguous; mn-contiguous
-// operands are loaded as 16-byte rows of VEC x VEC micro-blocks and
-// transposed in registers on the way into LDS, so every MFMA fragment read is
-// a single ds_read_b128.  bf16 uses v_mfma_f32_16x16x32_bf16, fp32 uses
-// v_mfma_f32_16x16x4_f32; accumulation is always fp32.
+// (kc = k-contiguous in memory, mc/nc = row/column-contiguous.)  bf16 uses
+// v_mfma_f32_32x32x16_bf16, fp32 v_mfma_f32_32x32x2_f32; accumulation is always
+// fp32.  All of bf16 and the larger fp32 launches run on the pipelined kernel
+// (namespace pipe); the generic kernel, which the other fp32 launches take, stages
+// every operand through LDS as [row][k] with k contiguous: mn-contiguous operands
+// are loaded as 16-byte rows of VEC x VEC micro-blocks and transposed in registers on
+// the way, so every MFMA fragment read is a single ds_read_b128.
 #include <algorithm>
 #include <atomic>
 #include <cmath>
@@ -84,7 +85,8 @@ struct GemmArgs {
   // (0: Ndim); c_rows / c_cols: rows / columns of C that are stored (0: all),
   // c_cols with rows of C at any alignment.
   int b_rows, c_rows, c_cols;
-  int tiles_m, tiles_n;      // padded logical tile space of the pipelined kernel
+  int tiles_m, tiles_n;      // logical tile space of the pipelined kernel (whole GM x GN groups; tiles_n of
+                             // row-grouped kinds: real tiles)
   // Split tail (pipelined kernel, row-grouped kinds without a fused
   // epilogue): of the `total` real tiles, the largest multiple of split_cus
   // run whole in blocks [0, split_from); the rest (fewer than split_cus) run
@@ -142,19 +144,6 @@ template <> struct MfmaOp<float, 32> {
 // In-register transpose of a VEC x VEC micro-block: in[r] holds VEC
 // consecutive columns of row r; out[c] gets VEC consecutive rows of column c.
 template <typename T> struct Transpose;
-template <> struct Transpose<uint16_t> {
-  __device__ static inline void run(const Vec16* in, Vec16* out) {
-#pragma unroll
-    for (int c = 0; c < 8; ++c) {
-      const int w = c >> 1;
-#pragma unroll
-      for (int p = 0; p < 4; ++p) {
-        const uint32_t lo = in[2 * p].w[w], hi = in[2 * p + 1].w[w];
-        out[c].w[p] = (c & 1) ? ((lo >> 16) | (hi & 0xffff0000u)) : ((lo & 0xffffu) | (hi << 16));
-      }
-    }
-  }
-};
 template <> struct Transpose<float> {
   __device__ static inline void run(const Vec16* in, Vec16* out) {
 #pragma unroll

@@ -1,5 +1,5 @@
 """abacus_attention_any_fwd / _bwd: lengths off the 128-query blocks and 64-key tiles, and head dim 128, against fp64
-(the bounds of test_gpu_attention.py: torch's fused kernel's error, or 4e-3)."""
+(the bound is derived where it is applied)."""
 
 import math
 
