@@ -117,7 +117,8 @@ def cross_entropy(input: torch.Tensor, target: torch.Tensor, weight: torch.Tenso
     if _use_liger and input.device.type != "cuda":
         raise RuntimeError("Liger cross entropy needs a CUDA tensor")
     fused = (input.is_cuda and input.dim() == 2 and input.dtype in (torch.float32, torch.bfloat16)
-             and target.dim() == 1 and target.shape[0] == input.shape[0] and weight is None
+             and target.dim() == 1 and target.shape[0] == input.shape[0] and target.device == input.device
+             and weight is None
              and size_average is None and reduce is None and reduction == "mean" and label_smoothing == 0.0)
     if not fused:
         return F.cross_entropy(input, target, weight=weight, size_average=size_average, ignore_index=ignore_index,
@@ -149,7 +150,8 @@ def next_token_loss(logits_BLV: torch.Tensor, tokens_BL: torch.Tensor) -> torch.
         raise IndexError(f"Target {int(targets[bad][0])} is out of bounds.")
     targets_BL = F.pad(targets, (0, 1), value=-100)
     logits_NV = logits_BLV.reshape(-1, V)
-    if logits_NV.is_cuda and logits_NV.dtype in (torch.float32, torch.bfloat16):
+    if logits_NV.is_cuda and logits_NV.dtype in (torch.float32, torch.bfloat16) and (
+            tokens_BL.device == logits_BLV.device):
         # HIP kernels; the loss in the logits' dtype, as torch's cross_entropy returns it
         loss = _CrossEntropyFunction.apply(logits_NV.contiguous(), targets_BL.reshape(-1).to(torch.int64).contiguous(),
                                            count, -100)

@@ -8,7 +8,7 @@ import torch
 import torch.nn.functional as F
 
 from abacus_amd import _lib
-from abacus_amd.train import cross_entropy
+from abacus_amd.train import cross_entropy, next_token_loss
 
 pytestmark = pytest.mark.gpu
 
@@ -65,3 +65,11 @@ def test_sum_of_many_rows_keeps_its_digits():
     x = torch.zeros(N, 4, device="cuda")
     loss = cross_entropy(x, torch.zeros(N, device="cuda", dtype=torch.int64))
     assert abs(float(loss) - math.log(4.0)) <= 2e-6 * math.log(4.0)
+
+
+def test_targets_on_the_cpu_raise():
+    x, t = torch.randn(1, 5, 16, device="cuda"), torch.zeros(1, 5, dtype=torch.int64)
+    with pytest.raises(RuntimeError):
+        cross_entropy(x[0], t[0])
+    with pytest.raises(RuntimeError):
+        next_token_loss(x, t)

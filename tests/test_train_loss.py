@@ -42,3 +42,20 @@ def test_out_of_range_target_raises():
     tokens = torch.tensor([[1, 2, 7, 3]])
     with pytest.raises(IndexError, match="out of bounds"):
         next_token_loss(torch.zeros(1, 4, 5), tokens)
+
+
+def test_targets_on_another_device_reach_no_kernel(monkeypatch):
+    """GPU logits with CPU targets end in torch's device error; the kernel would read a host address."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+
+    from abacus_amd import train
+
+    made = []
+    monkeypatch.setattr(train._lib, "call", lambda name, *args: made.append(name))
+    monkeypatch.setattr(train._lib, "ptr", lambda t: 0)
+    monkeypatch.setattr(train._lib, "stream_of", lambda device: 0)
+    with FakeTensorMode():
+        logits, targets = torch.empty(3, 8, device="cuda"), torch.empty(3, dtype=torch.int64)
+        with pytest.raises(Exception, match="device"):
+            train.cross_entropy(logits, targets)
+    assert made == []
