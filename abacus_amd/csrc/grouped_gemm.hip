@@ -2114,8 +2114,8 @@ bool pipe_ok(int dtype, const GemmArgs& g, int R) {
 // Slices of a row-grouped launch (the down projection's forward, the gate/up data
 // gradient).  Their output is D wide and their reduction M or 2M long, so a narrow
 // layer with a long hidden size has few tiles, each a long serial chain, and most
-// CUs idle.  The slice count minimises an estimate of the launch for evenly filled
-// experts: the longest CU's tiles, or the launch's whole work (with `extra_us` of
+// CUs idle.  The slice count minimises an estimate of the launch, for evenly filled
+// experts and in fp32 also for all rows on few of them: the longest CU's tiles, or the launch's whole work (with `extra_us` of
 // work that other blocks of it do) shared by all CUs if that is more, plus the
 // pass over the fp32 partials.  Measured per k-tile 1.7 us (bf16; 1.1 thin) and 7
 // us (fp32; 1.9 thin), per block 8 us, partials at 4 TB/s; fp32 on the generic
@@ -2124,6 +2124,10 @@ bool pipe_ok(int dtype, const GemmArgs& g, int R) {
 // tokens top-8, down forward 269 -> 115, gate/up backward 787 -> 611; E 8 D 448 M
 // 13632, 1027 tokens top-2, 114 -> 57 and 640 -> 223; fp32 E 4 D 1472 M 2496, 273
 // tokens top-2, 189 -> 97 and 543 -> 331.
+// The second layout is there because a full fp32 tile takes 3.7 times a thin one per
+// k-tile: sliced for thin tiles alone, one expert of more than 128 rows was the launch.
+// Layer forward + backward, E 16 D 1024 M 2816 top-2 (unsliced; for even rows; now): 512 tokens
+// Zipf-skewed 1635, 2016, 1386, on two experts 1234, 1614, 925; 1024 tokens evenly routed 1838, 2212, 1720.
 template <typename T, int KIND>
 int row_slices(const GemmArgs& g, int64_t R, double extra_us) {
   static_assert(KIND == kDownFwd || KIND == kGateUpDgrad, "plain-store row kinds");
@@ -2132,24 +2136,40 @@ int row_slices(const GemmArgs& g, int64_t R, double extra_us) {
   const int64_t E = std::min<int64_t>(g.E, R), r = (R + E - 1) / E;
   const int64_t nt = (g.Ndim + pipe::BN - 1) / pipe::BN, nt_thin = (g.Ndim + pipe::kThinN<T> - 1) / pipe::kThinN<T>;
   // an expert of r rows: rounded full tiles, and in half of the cases a thin one beside them
-  const double full = r <= pipe::THIN ? 0.0 : (double)(E * std::max<int64_t>(1, (r + 128) / 256) * nt);
-  const double thin = (double)(E * nt_thin) * (r <= pipe::THIN ? 1.0 : 0.5);
+  struct Layout { double full, thin, unsliced_us; } layouts[2];
+  layouts[0].full = r <= pipe::THIN ? 0.0 : (double)(E * std::max<int64_t>(1, (r + 128) / 256) * nt);
+  layouts[0].thin = (double)(E * nt_thin) * (r <= pipe::THIN ? 1.0 : 0.5);
+  int n_layouts = 1;
+  if (kF) {
+    if (4 * r > 3 * pipe::THIN && 4 * r <= 5 * pipe::THIN) {  // some experts above the thin tiles' rows, some below
+      layouts[0].full = 0.5 * (double)(E * nt);
+      layouts[0].thin = 0.5 * (double)(E * nt_thin);
+    }
+    layouts[n_layouts++] = {R > pipe::THIN ? (double)((R + 255) / 256 * nt) : 0.0, (double)nt_thin, 0.0};
+  }
   const int64_t kt = (KindTraits<KIND>::DUAL_K ? 2 : 1) * (((int64_t)g.Kdim + pipe::kBKT<T> - 1) / pipe::kBKT<T>);
   const auto rounds = [&](double blocks) { return std::max(1.0, std::ceil(blocks / cus)); };
+  const bool generic = kF && !pipe_ok<KIND>(kF32, g, (int)R);
   int best = 1;
-  double best_us = 0.0;
+  double best_cost = 1.0;
   for (int s = 1; s <= 16 && (s == 1 || kt / s >= 4); ++s) {
     const double k = (double)((kt + s - 1) / s), b_full = k * per_k + per_block, b_thin = k * per_k_thin + per_block;
-    const double chain = full > 0.0 ? rounds(full * s) * b_full : rounds(thin * s) * b_thin;
-    const double share = (full * s * b_full + thin * s * b_thin + extra_us) / cus;
-    double us = std::max(chain, share) + (s > 1 ? 6.0 + (double)s * (double)R * g.Ndim * 8.0 / 4e6 : 0.0);
-    if (kF && s == 1 && !pipe_ok<KIND>(kF32, g, (int)R)) {
-      const double tiles = (double)((E + R / 128) * ((g.Ndim + 127) / 128));
-      us = (double)kt * (tiles <= cus ? 2.4 : 4.2 * std::max(1.0, tiles / (2.0 * cus)));
+    double cost = 0.0;  // against the unsliced launch, in the layout that gains least
+    for (int l = 0; l < n_layouts; ++l) {
+      Layout& t = layouts[l];
+      const double chain = t.full > 0.0 ? rounds(t.full * s) * b_full : rounds(t.thin * s) * b_thin;
+      const double share = (t.full * s * b_full + t.thin * s * b_thin + extra_us) / cus;
+      double us = std::max(chain, share) + (s > 1 ? 6.0 + (double)s * (double)R * g.Ndim * 8.0 / 4e6 : 0.0);
+      if (generic && s == 1) {
+        const double tiles = (double)((E + R / 128) * ((g.Ndim + 127) / 128));
+        us = (double)kt * (tiles <= cus ? 2.4 : 4.2 * std::max(1.0, tiles / (2.0 * cus)));
+      }
+      if (s == 1) t.unsliced_us = us;
+      cost = std::max(cost, us / t.unsliced_us);
     }
-    if (s == 1 || us < (best == 1 ? 0.93 : 0.97) * best_us) {
+    if (s > 1 && cost < (best == 1 ? 0.93 : 0.97) * best_cost) {
       best = s;
-      best_us = us;
+      best_cost = cost;
     }
   }
   return best;

@@ -73,3 +73,21 @@ def test_sliced_products_match_fp64(dtype, counts, D, M):
         ):
             err = float((got.double() - want).norm() / want.norm())
             assert err < tol, f"{name} expert {e}: {err:.3g}"
+
+
+@pytest.mark.parametrize("dtype,counts,D,M", [
+    (torch.float32, [104, 145, 0, 128, 129, 3, 260], 256, 2816),  # experts on both sides of the thin tiles' rows
+    (torch.float32, [0] * 7 + [500], 512, 2048),                 # all rows on one expert
+], ids=["fp32_mixed", "fp32_one_expert"])
+def test_uneven_sliced_products_match_fp64(dtype, counts, D, M):
+    test_sliced_products_match_fp64(dtype, counts, D, M)
+
+
+@pytest.mark.parametrize("R,D,M,E", [(1024, 1024, 2816, 16), (2048, 1024, 2816, 16), (800, 1024, 2816, 16),
+                                     (600, 512, 2048, 8), (512, 128, 2376, 64), (256, 2048, 1408, 32)])
+def test_fp32_slices_bound_a_full_tile(R, D, M, E):
+    """However the rows are spread, no full 256-row tile's slice (7 us per 32 of the reduction) takes longer than the
+    whole launch does unsliced (2.4 us), which an expert with most of the rows would show."""
+    n = _lib.query("abacus_moe_down_fwd_ws_bytes", R, M, D, E, _lib.F32)
+    slices, k_tiles = max(1, n // (R * D * 4)), -(-M // 32)
+    assert slices == 1 or 7.0 * -(-k_tiles // slices) + 8.0 < 2.4 * k_tiles, slices
