@@ -56,6 +56,9 @@ class _PlanRouting(Routing):
 
     _READ_BY_BACKWARD = ("weights", "offsets", "pos")
 
+    def __new__(cls, *args, **fields):  # dataclasses.replace calls with the fields: a record of those tensors
+        return Routing(**fields) if fields else super().__new__(cls)
+
     def __init__(self, route: torch.Tensor, plan: "_LayerPlan", dtype: torch.dtype):
         self._route, self._at, self._sizes, self._dtype = route, plan.at, plan.sizes, dtype
 
