@@ -19,9 +19,9 @@ call, ptr = _lib.call, _lib.ptr
 @pytest.mark.parametrize("counts,D,M", [
     ([1, 0, 1], 1024, 4096),                   # one row each: sliced down projection
     ([0, 3, 16, 17, 32, 33, 70, 0, 0, 0, 0], 136, 136),  # every row-group remainder, one tile and an overlapping one
-    ([58, 1, 0, 5], 264, 263),                 # odd hidden size; an expert of three passes
+    ([58, 1, 0, 5], 264, 263),                 # odd hidden size; an expert of two row tiles
     ([1, 0, 2] * 60, 384, 384),                # enough tiles for blocks of 4 waves
-    ([150] + [0] * 127 + [3] * 40, 1032, 520),  # ... with more passes than run beside each other
+    ([150] + [0] * 127 + [3] * 40, 1032, 520),  # ... and numbered row tiles past the first
     ([6, 9], 128, 2731),                       # odd, several slices with a tail block
     ([2, 1, 0, 4], 320, 130),
 ], ids=["single_rows", "row_groups", "odd", "four_waves", "one_heavy", "odd_sliced", "two_mod_vector"])
