@@ -2119,8 +2119,8 @@ bool pipe_ok(int dtype, const GemmArgs& g, int R) {
 // work that other blocks of it do) shared by all CUs if that is more, plus the
 // pass over the fp32 partials.  Measured per k-tile 1.7 us (bf16; 1.1 thin) and 7
 // us (fp32; 1.9 thin), per block 8 us, partials at 4 TB/s; fp32 on the generic
-// kernel 2.4 us per k-tile up to a 128 x 128 tile per CU, 4.2 up to two.  1:
-// unsliced.  Measured (us, unsliced -> sliced): bf16 E 64 D 256 M 11200, 366
+// kernel 4 us and 2.4 per k-tile up to a 128 x 128 tile per CU, 4.2 per k-tile up to
+// two.  1: unsliced.  Measured (us, unsliced -> sliced): bf16 E 64 D 256 M 11200, 366
 // tokens top-8, down forward 269 -> 115, gate/up backward 787 -> 611; E 8 D 448 M
 // 13632, 1027 tokens top-2, 114 -> 57 and 640 -> 223; fp32 E 4 D 1472 M 2496, 273
 // tokens top-2, 189 -> 97 and 543 -> 331.
@@ -2128,6 +2128,10 @@ bool pipe_ok(int dtype, const GemmArgs& g, int R) {
 // k-tile: sliced for thin tiles alone, one expert of more than 128 rows was the launch.
 // Layer forward + backward, E 16 D 1024 M 2816 top-2 (unsliced; for even rows; now): 512 tokens
 // Zipf-skewed 1635, 2016, 1386, on two experts 1234, 1614, 925; 1024 tokens evenly routed 1838, 2212, 1720.
+// Where no count gains in both, the one that gains most on even rows and loses nothing on few experts:
+// the gate/up data gradient of E 8 D 128 M 256, 512 rows, 41.7 -> 16.4 in even rows, 41.5 -> 41.2 all on one
+// expert.  That holds while the unsliced tiles are at most one per CU: past that the estimate of them is
+// too rough (E 128 D 792 M 2196, 752 rows on two experts 425 -> 522).
 template <typename T, int KIND>
 int row_slices(const GemmArgs& g, int64_t R, double extra_us) {
   static_assert(KIND == kDownFwd || KIND == kGateUpDgrad, "plain-store row kinds");
@@ -2150,29 +2154,35 @@ int row_slices(const GemmArgs& g, int64_t R, double extra_us) {
   const int64_t kt = (KindTraits<KIND>::DUAL_K ? 2 : 1) * (((int64_t)g.Kdim + pipe::kBKT<T> - 1) / pipe::kBKT<T>);
   const auto rounds = [&](double blocks) { return std::max(1.0, std::ceil(blocks / cus)); };
   const bool generic = kF && !pipe_ok<KIND>(kF32, g, (int)R);
-  int best = 1;
-  double best_cost = 1.0;
+  const double tiles = (double)((E + R / 128) * ((g.Ndim + 127) / 128));  // of the generic kernel
+  int best = 1, best_even = 1;
+  double best_cost = 1.0, best_even_cost = 0.85;
   for (int s = 1; s <= 16 && (s == 1 || kt / s >= 4); ++s) {
     const double k = (double)((kt + s - 1) / s), b_full = k * per_k + per_block, b_thin = k * per_k_thin + per_block;
-    double cost = 0.0;  // against the unsliced launch, in the layout that gains least
+    double cost = 0.0, even = 0.0;  // against the unsliced launch: in the layout that gains least, in the even one
     for (int l = 0; l < n_layouts; ++l) {
       Layout& t = layouts[l];
       const double chain = t.full > 0.0 ? rounds(t.full * s) * b_full : rounds(t.thin * s) * b_thin;
       const double share = (t.full * s * b_full + t.thin * s * b_thin + extra_us) / cus;
       double us = std::max(chain, share) + (s > 1 ? 6.0 + (double)s * (double)R * g.Ndim * 8.0 / 4e6 : 0.0);
       if (generic && s == 1) {
-        const double tiles = (double)((E + R / 128) * ((g.Ndim + 127) / 128));
-        us = (double)kt * (tiles <= cus ? 2.4 : 4.2 * std::max(1.0, tiles / (2.0 * cus)));
+        us = tiles <= cus ? 4.0 + 2.4 * (double)kt : 4.2 * (double)kt * std::max(1.0, tiles / (2.0 * cus));
       }
       if (s == 1) t.unsliced_us = us;
-      cost = std::max(cost, us / t.unsliced_us);
+      const double rel = us / t.unsliced_us;
+      if (l == 0) even = rel;
+      cost = std::max(cost, rel);
     }
     if (s > 1 && cost < (best == 1 ? 0.93 : 0.97) * best_cost) {
       best = s;
       best_cost = cost;
     }
+    if (generic && tiles <= cus && cost < 1.01 && even < best_even_cost) {
+      best_even = s;
+      best_even_cost = even;
+    }
   }
-  return best;
+  return best > 1 ? best : best_even;
 }
 
 inline int64_t slices_ws_bytes(int slices, int64_t R, int64_t N) { return slices > 1 ? slices * R * N * 4 : 0; }

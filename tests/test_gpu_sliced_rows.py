@@ -78,7 +78,9 @@ def test_sliced_products_match_fp64(dtype, counts, D, M):
 @pytest.mark.parametrize("dtype,counts,D,M", [
     (torch.float32, [104, 145, 0, 128, 129, 3, 260], 256, 2816),  # experts on both sides of the thin tiles' rows
     (torch.float32, [0] * 7 + [500], 512, 2048),                 # all rows on one expert
-], ids=["fp32_mixed", "fp32_one_expert"])
+    (torch.float32, [1085] * 4 + [1084] * 4, 184, 876),          # the down product sliced for what even rows gain
+    (torch.float32, [0] * 7 + [8676], 184, 876),                 # ... on one expert
+], ids=["fp32_mixed", "fp32_one_expert", "fp32_for_even_rows", "fp32_for_even_rows_one_expert"])
 def test_uneven_sliced_products_match_fp64(dtype, counts, D, M):
     test_sliced_products_match_fp64(dtype, counts, D, M)
 
@@ -91,3 +93,26 @@ def test_fp32_slices_bound_a_full_tile(R, D, M, E):
     n = _lib.query("abacus_moe_down_fwd_ws_bytes", R, M, D, E, _lib.F32)
     slices, k_tiles = max(1, n // (R * D * 4)), -(-M // 32)
     assert slices == 1 or 7.0 * -(-k_tiles // slices) + 8.0 < 2.4 * k_tiles, slices
+
+
+@pytest.mark.parametrize("counts", [[64] * 8, [0] * 7 + [512]], ids=["even", "one_expert"])
+def test_small_fp32_data_gradient(counts):
+    """A gate/up data gradient that is sliced although its down product is not, against fp64."""
+    R, D, M, E = sum(counts), 128, 256, len(counts)
+    dev = torch.device("cuda")
+    gen = torch.Generator(device=dev).manual_seed(52)
+    rn = lambda *shape: torch.randn(*shape, device=dev, generator=gen)
+    n = _lib.query("abacus_experts_gateup_bwd_ws_bytes", R, D, M, E, _lib.F32)
+    assert n >= 2 * R * D * 4 and _lib.query("abacus_moe_down_fwd_ws_bytes", R, M, D, E, _lib.F32) == 0
+    dg, du, x, wg, wu = rn(R, M), rn(R, M), rn(R, D), rn(E, D, M) * 0.05, rn(E, D, M) * 0.05
+    offs = [0] + list(itertools.accumulate(counts))
+    offsets = torch.tensor(offs, dtype=torch.int32, device=dev)
+    dx, ws = torch.full((R, D), float("nan"), device=dev), torch.full((n // 4,), float("nan"), device=dev)
+    ctr = torch.zeros(_lib.TILE_CTR_INTS, dtype=torch.int32, device=dev)
+    call("abacus_experts_gateup_bwd", ptr(dg), ptr(du), ptr(wg), ptr(wu), ptr(x), ptr(offsets), R, D, M, M, E, _lib.F32,
+         ptr(dx), None, None, ptr(ctr), ptr(ws), n, _lib.stream_of(dev))
+    for e in range(E):
+        a, b = offs[e], offs[e + 1]
+        want = dg[a:b].double() @ wg[e].double().t() + du[a:b].double() @ wu[e].double().t()
+        # sums of 512 products in fp32, in four parts: at most 128 roundings of 2^-24 each in one of them
+        assert a == b or float((dx[a:b].double() - want).norm() / want.norm()) < 128 * 2 ** -24
