@@ -25,3 +25,15 @@ def test_every_expert_product_is_counted():
     experts = [n for n in _lib.SIGNATURES if "_experts_" in n and not n.endswith("_bytes")]
     assert len(experts) >= 5 and all(bench.is_moe(n) for n in experts)
     bench.check_known(n for n in _lib.SIGNATURES if not n.endswith("_bytes"))
+
+
+def test_settle_takes_the_set_up_out_of_the_collector():
+    import gc
+
+    import bench
+
+    try:
+        bench.settle()
+        assert gc.get_freeze_count() > 0 and gc.isenabled()
+    finally:
+        gc.unfreeze()
