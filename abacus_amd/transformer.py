@@ -138,6 +138,15 @@ def _recorded(op, grads, d_out, *inputs):
     return _KernelGradient.apply(op, grads, d_out, *inputs) if torch.is_grad_enabled() else grads
 
 
+def _by_kernel(op, gradients, d_out, *inputs):
+    """gradients(), a kernel backward of `op`, as _recorded gives it."""
+    if not torch.is_grad_enabled():
+        return gradients()
+    with torch.no_grad():
+        grads = gradients()
+    return _recorded(op, grads, d_out, *inputs)
+
+
 def _norm_op(x, gamma, eps):
     return gamma * x * torch.rsqrt(x.square().mean(dim=-1, keepdim=True) + eps)
 
@@ -196,9 +205,8 @@ class _RMSNormFunction(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dy):
         x, gamma, rstd = ctx.saved_tensors
-        with torch.no_grad():
-            grads = _RMSNormFunction.gradients(dy, x.contiguous(), gamma, rstd)
-        return (*_recorded(lambda x, g: _norm_op(x, g, ctx.eps), grads, dy, x, gamma), None)
+        return (*_by_kernel(lambda x, g: _norm_op(x, g, ctx.eps),
+                           lambda: _RMSNormFunction.gradients(dy, x.contiguous(), gamma, rstd), dy, x, gamma), None)
 
     @staticmethod
     def gradients(dy, xc, gamma, rstd):
@@ -246,10 +254,9 @@ class _RMSNormRopeFunction(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dy):
         x, gamma, rstd, cos_c, sin_c = ctx.saved_tensors
-        with torch.no_grad():
-            grads = _RMSNormRopeFunction.gradients(dy, x.contiguous(), gamma, rstd, cos_c, sin_c)
+        gradients = lambda: _RMSNormRopeFunction.gradients(dy, x.contiguous(), gamma, rstd, cos_c, sin_c)
         op = lambda x, g: _norm_rope_op(x, g, cos_c, sin_c, ctx.eps)
-        return (*_recorded(op, grads, dy, x, gamma), None, None, None)
+        return (*_by_kernel(op, gradients, dy, x, gamma), None, None, None)
 
     @staticmethod
     def gradients(dy, xc, gamma, rstd, cos_c, sin_c):
@@ -392,9 +399,7 @@ class _FlashAttentionFunction(torch.autograd.Function):
     @staticmethod
     def backward(ctx, d_o):
         saved = ctx.saved_tensors
-        with torch.no_grad():
-            grads = _FlashAttentionFunction.gradients(d_o, *saved)
-        return _recorded(_causal_op, grads, d_o, *saved[:3])
+        return _by_kernel(_causal_op, lambda: _FlashAttentionFunction.gradients(d_o, *saved), d_o, *saved[:3])
 
     @staticmethod
     def gradients(d_o, q, k, v, o, lse):
@@ -529,16 +534,15 @@ class _AttentionFunction(torch.autograd.Function):
     @staticmethod
     def backward(ctx, d_o):
         saved = ctx.saved_tensors
-        *inputs, cos_c, sin_c = saved[:8]
-        with torch.no_grad():
-            grads = _AttentionFunction.gradients(ctx.needs_input_grad, d_o, *saved)
+        cos_c, sin_c = saved[6:8]
 
         def op(x, w_q, w_k, w_v, gamma_q, gamma_k):
             q, k, v = ((x @ w.flatten(1)).unflatten(2, w.shape[1:]) for w in (w_q, w_k, w_v))
             return _causal_op(_norm_rope_op(q, gamma_q, cos_c, sin_c, ctx.eps),
                               _norm_rope_op(k, gamma_k, cos_c, sin_c, ctx.eps), v)
 
-        return (*_recorded(op, grads, d_o, *inputs), None, None, None)
+        gradients = lambda: _AttentionFunction.gradients(ctx.needs_input_grad, d_o, *saved)
+        return (*_by_kernel(op, gradients, d_o, *saved[:6]), None, None, None)
 
     @staticmethod
     def gradients(needs, d_o, x_BLD, w_q, w_k, w_v, gamma_q, gamma_k, cos_c, sin_c, q, k, v, qn, kn, o, rstd, lse):
